@@ -204,8 +204,8 @@ int sph_hip_download_particles(sph_ctx *ctx, sph_particle_v1 *out,
  * on, without changing the state or the results of later steps.  Per
  * particle id: count[i] = neighbours with multiplicity (the terms the
  * reference sums, src/sph.cpp:40-66); walk[i] (may be NULL) = bit 0: its
- * wave task walks the union of its lanes' stencils, bit 1: the task is
- * split into parts, bit 2: a neighbour list was recorded; list_count[i]
+ * wave task walks the union of its lanes' stencils together (one candidate
+ * at a time, or staged on chip), bit 1: the task is split into parts, bit 2: a neighbour list was recorded; list_count[i]
  * (may be NULL) = list entries or 0xFFFFFFFF; list (may be NULL): 64
  * entries per id, the listed neighbours' ids (each once) in walk order. */
 int sph_hip_walk_dump(sph_ctx *ctx, uint32_t *count, uint32_t *walk,

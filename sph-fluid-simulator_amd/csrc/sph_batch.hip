@@ -834,7 +834,7 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
     launch_scatter(stream, a, c, S);
     launch_sort_big_cells(stream, a, c);
     launch_reorder(stream, a, c, S);
-    launch_plan_parts(stream, a, c, S, pp);
+    launch_plan_parts(stream, a, c, S, pp, nl, (uint32_t *)tcount.ptr);
     NeighborDump d{(uint32_t *)tcount.ptr, nullptr, nullptr, true};
     launch_density(stream, a, c, S, &d, &pp, kStencilBlock, &nl);
 
@@ -874,7 +874,7 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
             return fail(SPH_E_HIP, "walk_dump: slot %u holds id %u of %u", q, id, n);
         count[id] = cnt[q];
         if (walk)
-            walk[id] = (wk[2 * t + 1].w ? 1u : 0u) | (off[t + 1] != off[t] ? 2u : 0u) | (lc[q] != kNoList ? 4u : 0u);
+            walk[id] = (wk[2 * t + 1].w & (int)kWalkUnion ? 1u : 0u) | (off[t + 1] != off[t] ? 2u : 0u) | (lc[q] != kNoList ? 4u : 0u);
         if (list_count)
             list_count[id] = lc[q];
         if (list && lc[q] != kNoList)

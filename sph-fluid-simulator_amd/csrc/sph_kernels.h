@@ -77,7 +77,12 @@ struct SceneSet {
     const StepParams *params;  // one per scene
     const WaveTask *tasks;     // one per 64-slot wave
     uint32_t nwaves;
+    bool staged;               // some scene's walks may be staged (stageable)
 };
+
+// Whether short walks of a scene are staged in LDS (k_plan_list): cells of
+// h or larger, and the per-lane walk not forced.
+SPH_HD inline bool stageable(const StepParams &P) { return P.reach == 1 && P.lane_walk == 0u; }
 
 // Spare part tasks of a scene of `waves` wave tasks (beyond one per task):
 // the scene's part size is its total walk over this room, so a scene
@@ -101,6 +106,11 @@ SPH_HD inline uint64_t part_room(uint64_t waves)
 // finish adds the partial sums in part order, so results are
 // deterministic.  An unsplit task sums in candidate order (and its two
 // walks agree bit for bit); a split one differs from it by rounding only.
+// The long walks of a scene add their lengths to kTotalSlots sums (one
+// address takes an atomic every few nanoseconds: thousands of them would
+// outlast the pass).
+constexpr uint32_t kTotalSlots = 8;
+
 struct PartPlan {
     uint32_t *nparts;    // per wave task: parts of a split task, 0 for an unsplit one; padded
                          // to a kScanChunk multiple (zero outside use)
@@ -108,7 +118,7 @@ struct PartPlan {
     uint32_t *scan_partials;
     uint32_t padded;     // padded length of nparts
     uint32_t *measure;   // walk length per wave task
-    unsigned long long *total;  // sum of the walk lengths per scene (zero between steps)
+    unsigned long long *total;  // sums of the long walks' lengths, kTotalSlots per scene (zero between steps)
     uint32_t nscenes;
     uint32_t cap;        // part-task capacity: sum over scenes of waves + part_room(waves)
     uint32_t *tasks;     // (wave task << kPartBits) | part, cap entries
@@ -116,14 +126,23 @@ struct PartPlan {
     float4 *buf;         // partial sums: (part task) * 64 + lane, cap * 64 entries
     uint32_t *done;      // parts finished per wave task (zero between passes)
     int4 *walk;          // per wave task, two entries: union box (x0, x1, y0, y1), (z0, z1, union
-                         // count, 1 = union walk / 0 = per-lane walk)
+                         // count, kWalk* bits)
     uint32_t *own;       // per slot of a per-lane-walk wave task: length of its own stencil
 };
 
+// How a wave task walks its candidates (0: each lane its own, from memory).
+constexpr uint32_t kWalkUnion = 1u;   // the wave shares one set of candidates
+constexpr uint32_t kWalkBox = 2u;     // ... that of the union box
+constexpr uint32_t kWalkSummed = 4u;  // ... staged in LDS; its density pass is done
+
+struct NeighborLists;
+
 // Plans the parts of every wave task of S from the B-order cells and
-// cell ranges, and clears the task queues.
+// cell ranges, and clears the task queues.  Tasks of short walks get their
+// densities and neighbour lists here (k_plan_list); `count` (may be null)
+// receives their neighbour counts with multiplicity.
 void launch_plan_parts(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
-                       const PartPlan &pp);
+                       const PartPlan &pp, const NeighborLists &nl, uint32_t *count = nullptr);
 
 // Debug outputs of the density pass: per-particle neighbour count (with
 // multiplicity) and, when out != nullptr, the neighbour ids of row s at

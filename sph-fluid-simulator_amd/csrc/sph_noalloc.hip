@@ -111,7 +111,7 @@ Layout make_layout(uint32_t n, uint64_t ncells)
     L.off = c.take(4ull * (L.waves_padded + 1));
     L.ppartials = c.take(4ull * (L.waves_padded / kScanChunk));
     L.measure = c.take(4ull * L.nwaves);
-    L.total = c.take(8);
+    L.total = c.take(8 * kTotalSlots);
     L.ptasks = c.take(4ull * L.cap);
     L.queue = c.take(16);
     L.buf = c.take(sizeof(float4) * 64ull * L.cap);
@@ -254,6 +254,7 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     set.params = dparams;
     set.tasks = dtasks;
     set.nwaves = L.nwaves;
+    set.staged = stageable(P);
 
     PartPlan pp;
     pp.nparts = (uint32_t *)at(L.nparts);
@@ -276,16 +277,16 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     launch_fill_u32(st, c.counts, 0u, c.ncells_padded);
     launch_fill_u32(st, pp.nparts, 0u, L.waves_padded);
     launch_fill_u32(st, pp.done, 0u, L.nwaves);
-    launch_fill_u32(st, (uint32_t *)pp.total, 0u, 2);
+    launch_fill_u32(st, (uint32_t *)pp.total, 0u, 2 * kTotalSlots);
 
     launch_init_keys(st, a, c, set);
     launch_scan(st, c, false);
     launch_scatter(st, a, c, set);
     launch_sort_big_cells(st, a, c);
     launch_reorder(st, a, c, set);
-    launch_plan_parts(st, a, c, set, pp);
     float4 *force = (float4 *)at(L.force);
     const NeighborLists nl{(uint32_t *)at(L.nlist), (uint32_t *)at(L.ncount), n};
+    launch_plan_parts(st, a, c, set, pp, nl);
     launch_density(st, a, c, set, nullptr, &pp, kStencilBlock, &nl);
     launch_force_integrate(st, a, c, set, force, /*next_keys=*/false, &pp, kStencilBlock, &nl);
 

@@ -304,10 +304,10 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
     if (cap > 0xFFFFFFFFull)
         return fail(SPH_E_LIMIT, "part plan: %zu part tasks", cap);
     const bool fresh_counters = padded > parts_padded || pdone.bytes < 4 * nw ||
-                                ptotal.bytes < 8 * std::max<size_t>(scenes.size(), 1);
+                                ptotal.bytes < 8 * kTotalSlots * std::max<size_t>(scenes.size(), 1);
     if ((rc = pnparts.reserve(4ull * padded)) || (rc = poff.reserve(4ull * (padded + 1))) ||
         (rc = ppartials.reserve(4ull * (padded / kScanChunk))) || (rc = pmeasure.reserve(4ull * nw)) ||
-        (rc = ptotal.reserve(8ull * std::max<size_t>(scenes.size(), 1))) || (rc = ptasks.reserve(4ull * cap)) ||
+        (rc = ptotal.reserve(8ull * kTotalSlots * std::max<size_t>(scenes.size(), 1))) || (rc = ptasks.reserve(4ull * cap)) ||
         (rc = pqueue.reserve(16)) ||
         (rc = pbuf.reserve(sizeof(float4) * 64ull * cap)) || (rc = pdone.reserve(4ull * nw)) ||
         (rc = pwalk.reserve(2ull * sizeof(int4) * nw)) || (rc = pown.reserve(4ull * std::max<size_t>(nslots, 1))))
@@ -328,6 +328,9 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
         e = hipStreamSynchronize(st);  // the host vectors go out of scope
     if (e != hipSuccess)
         return hip_fail(e, "scene table upload");
+    staged = false;
+    for (const StepParams &sp : scenes)
+        staged = staged || stageable(sp);
     nwaves = (uint32_t)t.size();
     nscenes = (uint32_t)scenes.size();
     part_cap = (uint32_t)cap;
@@ -370,6 +373,7 @@ SceneSet Workspace::scene_set() const
     S.params = (const StepParams *)params.ptr;
     S.tasks = (const WaveTask *)tasks.ptr;
     S.nwaves = nwaves;
+    S.staged = staged;
     return S;
 }
 
@@ -436,10 +440,10 @@ void enqueue_step(hipStream_t st, Workspace &w, float4 *force_out, bool next_key
         timer->mark(st, "scatter");
     launch_reorder(st, a, c, S);
     const PartPlan pp = w.part_plan();
-    launch_plan_parts(st, a, c, S, pp);
     if (timer)
         timer->mark(st, "reorder");
     const NeighborLists nl = w.lists();
+    launch_plan_parts(st, a, c, S, pp, nl);
     launch_density(st, a, c, S, nullptr, &pp, w.stencil_block, &nl);
     if (timer)
         timer->mark(st, "density");
@@ -598,8 +602,8 @@ int update_particles(sph_particle_v1 *particles, float *transforms, size_t n_,
     CellArrays c = w.cells();
     const SceneSet set = w.scene_set();
     const PartPlan pp = w.part_plan();
-    launch_plan_parts(st, a, c, set, pp);
     const NeighborLists nl = w.lists();
+    launch_plan_parts(st, a, c, set, pp, nl);
     launch_density(st, a, c, set, nullptr, &pp, kStencilBlock, &nl);
     launch_force_integrate(st, a, c, set, (float4 *)w.force.ptr, /*next_keys=*/false, &pp, kStencilBlock, &nl);
     CellArrays c16 = cells16(S);
