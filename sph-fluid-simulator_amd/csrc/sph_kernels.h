@@ -42,11 +42,16 @@ constexpr int kBigSortBlock = 1024;        // threads of the big-cell sort
 constexpr int kBigSortBlocks = 256;        // blocks walking the big-cell list
 constexpr uint32_t kPartBits = 8;          // part index bits of a part task
 constexpr uint32_t kMaxParts = 1u << kPartBits;  // parts of one split wave task, at most
-constexpr uint32_t kPartCandidates = 2048; // candidates per part, at least
+constexpr uint32_t kPartCandidates = 1024; // candidates per part, at least: half as many as before parts
+                                           // were combined without fences (late states: 51 thousand
+                                           // particles, force 0.28 -> 0.22 ms; 240 thousand, density
+                                           // 0.53 -> 0.45; a million the same)
 constexpr uint32_t kPartRoomPerWave = 3;   // spare part tasks per wave task of a scene, at least
 constexpr uint32_t kPartRoomMin = 49152;   // ... raised to this many per scene (~10 rounds of the
                                            // resident waves, so tasks stay short in mid-size scenes)
 constexpr uint32_t kPartRoomMaxPerWave = 16;  // ... but at most this many per wave task
+constexpr uint32_t kShortWalk = 409;       // own candidates of a lane whose wave may be staged, or left
+                                           // unsplit in spite of slow lanes, to record neighbour lists
 constexpr uint32_t kLaneWalkWeight = 5;    // per-lane walk candidates count this many times
 constexpr uint32_t kSlowWalkWeight = 8;    // ... in a wave with slow lanes (m_ij counted per neighbour)
 
@@ -123,7 +128,7 @@ struct PartPlan {
     uint32_t cap;        // part-task capacity: sum over scenes of waves + part_room(waves)
     uint32_t *tasks;     // (wave task << kPartBits) | part, cap entries
     uint32_t *queue;     // pulled-task counters: [0] density, [1] force
-    float4 *buf;         // partial sums: (part task) * 64 + lane, cap * 64 entries
+    float4 *buf;         // partial sums: four arrays of 64 lanes per part task (cap * 64 entries)
     uint32_t *done;      // parts finished per wave task (zero between passes)
     int4 *walk;          // per wave task, two entries: union box (x0, x1, y0, y1), (z0, z1, union
                          // count, kWalk* bits)
@@ -134,6 +139,7 @@ struct PartPlan {
 constexpr uint32_t kWalkUnion = 1u;   // the wave shares one set of candidates
 constexpr uint32_t kWalkBox = 2u;     // ... that of the union box
 constexpr uint32_t kWalkSummed = 4u;  // ... staged in LDS; its density pass is done
+constexpr uint32_t kWalkSegments = 8u;  // with kWalkBox: its segments' stencils instead of one box
 
 struct NeighborLists;
 

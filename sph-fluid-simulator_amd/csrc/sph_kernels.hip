@@ -588,21 +588,37 @@ __device__ inline float dist2_ref(float4 pi, float4 q, float &dx, float &dy, flo
     return dx * dx + dy * dy + dz * dz;
 }
 
-// Correctly rounded sqrt for d2 >= 2^-96 (any d2 a neighbour pair can have
-// short of coincident points; d2 = 0 also comes out exact): v_sqrt_f32 is
-// within 1 ulp, and the neighbouring candidate whose residual
-// d2 - s * s' changes sign is the correctly rounded root (the tiny-input
-// rescaling of the library sequence is not needed in this range).
-__device__ inline float sqrt_rn(float x)
+// r = sqrt(x) correctly rounded and y = 1 / sqrt(x) within an ulp, for
+// x >= 2^-96 (any d2 a neighbour pair can have short of coincident points,
+// where both come out NaN / inf as the reference's division by r = 0 does):
+// one Newton step on v_rsq_f32, whose result equals the rounded root for
+// every mantissa at every exponent from -62 to 23 (all 2^23 of each tried
+// against the double root).  One transcendental and four multiplies or fmas
+// in place of v_sqrt, v_rcp and two compare-and-select corrections: 18 against
+// 41 issue cycles a wave, and 1 / r is nearer (1.6 against 2.0 half-ulps).
+__device__ inline float root(float x, float &y)
 {
-    float s = __builtin_amdgcn_sqrtf(x);
-    float down = __uint_as_float(__float_as_uint(s) - 1u);
-    float up = __uint_as_float(__float_as_uint(s) + 1u);
-    float r_down = fmaf(-down, s, x);
-    float r_up = fmaf(-up, s, x);
-    s = (r_down <= 0.0f) ? down : s;
-    s = (r_up > 0.0f) ? up : s;
-    return s;
+    y = __builtin_amdgcn_rsqf(x);
+    const float r0 = x * y;
+    return fmaf(fmaf(-r0, r0, x), 0.5f * y, r0);
+}
+
+// max(x, 0).  UNIT: x is at most 1, so a clamp to [0, 1] will do, which comes
+// free with the operation that made x (v_max is an instruction of its own, at
+// half the rate of an add).  NaN gives 0 either way.
+template <bool UNIT>
+__device__ inline float positive(float x)
+{
+    return UNIT ? __builtin_amdgcn_fmed3f(x, 0.0f, 1.0f) : fmaxf(x, 0.0f);
+}
+
+// x in a vector register: an instruction with a scalar-register operand
+// issues at half the rate of one without (measured: 4.4 against 2.3 cycles a
+// wave for add and multiply).
+__device__ inline float in_vgpr(float x)
+{
+    asm("" : "+v"(x));
+    return x;
 }
 
 struct RefCell {
@@ -781,10 +797,13 @@ __device__ inline int wave_max_i(int x)
 // (span + 2R)^2 rows fit the 64 lanes that stage them (R = 1: 4, 2: 4, 3: 2).
 __device__ inline int union_span(int R) { return min(4, 8 - 2 * R); }
 
-// A box of grid cells [x0, x1] x [y0, y1] x [z0, z1] (inside the grid)
-// whose rows a wave walks with one candidate index for all of its lanes.
+// What a wave walks together: a box of grid cells [x0, x1] x [y0, y1] x
+// [z0, z1] (inside the grid), or the stencils of the wave's segments (runs
+// of lanes in one x-row of cells), one after the other, each for its own
+// lanes.
 struct UnionRows {
     int x0, x1, y0, y1, z0, z1;
+    bool segments;
 };
 
 __device__ inline uint32_t row_base(const StepParams &P, int y, int z)
@@ -792,21 +811,6 @@ __device__ inline uint32_t row_base(const StepParams &P, int y, int z)
     return P.cell_base + (uint32_t)P.nx * ((uint32_t)y + (uint32_t)P.ny * (uint32_t)z);
 }
 
-// Chooses between the two ways a wave walks its candidates:
-//  * per lane: each lane walks its own (2R + 1)^3 stencil (gathers);
-//  * union: all lanes walk the union of their stencils together, so the
-//    candidate index is wave-uniform and its record is a scalar load
-//    broadcast to every lane.
-// Union is taken when all lanes sit in one cell (the dense regime: one
-// cell holds many waves), or when their cells span at most 16 cells in x
-// and union_span(R) in y and z (so the union has at most 64 rows) and the
-// union holds at most 3x the largest own stencil (a per-lane walk costs
-// about three times as much per candidate).  A candidate the union adds
-// to a lane's own stencil lies in a cell R + 1 or more cells away, beyond
-// R whole cells of edge >= h (1 + 2^-10) / R along some axis, so its
-// float squared distance is above h^2 and it never passes: both walks
-// visit a lane's passing candidates in the same order (rows z-major, then
-// y, slots ascending) and give bit-identical sums.
 // Length of the lane's own (2R + 1)^3 stencil, the sum of its rows'
 // lengths as for_each_row visits them; the bounds of one z-layer's rows are
 // loaded together (all in flight at once) instead of a row ahead.
@@ -835,13 +839,70 @@ __device__ inline uint32_t stencil_length(const uint32_t *__restrict__ cstart, u
     return own;
 }
 
+// The segments of a wave: the lanes are in cell order, so those of one (y, z)
+// row of cells are consecutive and ascend in x.
+__device__ inline uint64_t segment_heads(uint32_t cc, bool active)
+{
+    const uint32_t yz = cc & ~kSlowBit & ~2047u;
+    const uint32_t before = (uint32_t)__shfl_up((int)yz, 1, 64);
+    return __ballot(active && ((threadIdx.x & 63u) == 0u || yz != before));
+}
+
+// Row `lane` of the wave's segments' stencils ((2R + 1)^2 rows each, z-major
+// then y): its first slot and length (0 where there is no such row).
+__device__ inline void segment_row(const uint32_t *__restrict__ cstart, uint32_t cc, bool active, uint64_t heads,
+                                   const StepParams &P, uint32_t &b, uint32_t &len)
+{
+    const int R = P.reach;
+    const uint32_t W = 2u * (uint32_t)R + 1u, lane = threadIdx.x & 63u;
+    const uint32_t nact = (uint32_t)__builtin_popcountll(__ballot(active));
+    uint32_t first = 0, last = 0;  // cells of the ends of the lane's segment
+    uint32_t k = 0;
+    for (uint64_t h = heads; h != 0ull; ++k) {
+        const uint32_t a = (uint32_t)__builtin_ctzll(h);
+        h &= h - 1ull;
+        const uint32_t e = h != 0ull ? (uint32_t)__builtin_ctzll(h) - 1u : nact - 1u;
+        if (lane / (W * W) == k) {
+            first = (uint32_t)__builtin_amdgcn_readlane((int)cc, (int)a);
+            last = (uint32_t)__builtin_amdgcn_readlane((int)cc, (int)e);
+        }
+    }
+    b = len = 0u;
+    const int r = (int)(lane % (W * W));
+    const int y = cell_y(first) + r % (int)W - R, z = cell_z(first) + r / (int)W - R;
+    if (lane < k * W * W && y >= 0 && y < P.ny && z >= 0 && z < P.nz) {
+        const uint32_t r0 = row_base(P, y, z);
+        b = cstart[r0 + (uint32_t)max(cell_x(first) - R, 0)];
+        len = cstart[r0 + (uint32_t)min(cell_x(last) + R, P.nx - 1) + 1u] - b;
+    }
+}
+
 // own: the lane's own candidate count when this computed it (the
 // comparison needs it unless all lanes share one cell), else kNoOwn.
 constexpr uint32_t kNoOwn = 0xFFFFFFFFu;
 
-__device__ inline bool plan_union(const uint32_t *__restrict__ cstart, uint32_t cc, const StepParams &P,
+// Chooses between the two ways a wave walks its candidates:
+//  * per lane: each lane walks its own (2R + 1)^3 stencil (gathers);
+//  * union: all lanes walk the union of their stencils together, read from
+//    LDS with one broadcast for the wave.
+// Union is taken when all lanes sit in one cell (the dense regime: one cell
+// holds many waves), or when their cells span at most union_span(R) in y and
+// z (so the union has at most 64 rows) and the union holds at most 3x the
+// largest own stencil (a per-lane walk costs three times as much per
+// candidate and more).  A wave whose cells lie further apart (the end of one
+// clump and the start of the next) walks its segments' stencils, under the
+// same limits: per lane such waves took 1.0 of the 1.9 ms of a density pass
+// over a late state of a million particles, a tenth of its tasks.
+// A candidate the union adds to a lane's own stencil lies in a cell R + 1 or
+// more cells away, beyond R whole cells of edge >= h (1 + 2^-10) / R along
+// some axis, so its float squared distance is above h^2 and it never passes
+// (and a segment's candidates are met by its own lanes only): both walks
+// visit a lane's passing candidates in the same order (rows z-major, then y,
+// slots ascending) and give bit-identical sums.
+__device__ inline bool plan_union(const uint32_t *__restrict__ cstart, uint32_t cc, bool active, const StepParams &P,
                                   UnionRows &U, uint32_t &count, uint32_t &own)
 {
+    U = UnionRows{0, 0, 0, 0, 0, 0, false};
     if (P.lane_walk)
         return false;
     const uint32_t cell = cc & ~kSlowBit;
@@ -860,51 +921,55 @@ __device__ inline bool plan_union(const uint32_t *__restrict__ cstart, uint32_t 
         y1 = wave_max_i(gy);
         z0 = wave_min_i(gz);
         z1 = wave_max_i(gz);
-        const int span = union_span(P.reach);
-        if (x1 - x0 > 15 || y1 - y0 >= span || z1 - z0 >= span)
-            return false;
     }
-    const int R = P.reach;
-    U.x0 = max(x0 - R, 0);
-    U.x1 = min(x1 + R, P.nx - 1);
-    U.y0 = max(y0 - R, 0);
-    U.y1 = min(y1 + R, P.ny - 1);
-    U.z0 = max(z0 - R, 0);
-    U.z1 = min(z1 + R, P.nz - 1);
-    uint32_t un = 0;
-    for (int z = U.z0; z <= U.z1; ++z)
-        for (int y = U.y0; y <= U.y1; ++y) {
-            const uint32_t r0 = row_base(P, y, z);
-            un += cstart[r0 + (uint32_t)U.x1 + 1u] - cstart[r0 + (uint32_t)U.x0];
-        }
-    count = __builtin_amdgcn_readfirstlane(un);
-    if (one)
-        return true;
-    own = stencil_length(cstart, cc, P);
-    const uint32_t own_max = (uint32_t)wave_max_i((int)own);
+    uint32_t own_max = 0;
+    if (!one) {
+        own = stencil_length(cstart, cc, P);
+        own_max = (uint32_t)wave_max_i((int)own);
+    }
+    const int R = P.reach, span = union_span(R);
+    if (y1 - y0 < span && z1 - z0 < span) {
+        U.x0 = max(x0 - R, 0);
+        U.x1 = min(x1 + R, P.nx - 1);
+        U.y0 = max(y0 - R, 0);
+        U.y1 = min(y1 + R, P.ny - 1);
+        U.z0 = max(z0 - R, 0);
+        U.z1 = min(z1 + R, P.nz - 1);
+        uint32_t un = 0;
+        for (int z = U.z0; z <= U.z1; ++z)
+            for (int y = U.y0; y <= U.y1; ++y) {
+                const uint32_t r0 = row_base(P, y, z);
+                un += cstart[r0 + (uint32_t)U.x1 + 1u] - cstart[r0 + (uint32_t)U.x0];
+            }
+        count = __builtin_amdgcn_readfirstlane(un);
+        if (one || count <= 3ull * own_max)
+            return true;
+    }
+    const uint64_t heads = segment_heads(cc, active);
+    const uint32_t W = 2u * (uint32_t)R + 1u;
+    if ((uint32_t)__builtin_popcountll(heads) * W * W > 64u)
+        return false;
+    uint32_t b, len;
+    segment_row(cstart, cc, active, heads, P, b, len);
+    count = (uint32_t)__builtin_amdgcn_readlane((int)wave_inclusive_scan(len), 63);
+    U.segments = true;
     return count <= 3ull * own_max;
 }
 
-// The walk a wave task takes and, for the union walk, its box and count:
-// from the step's part plan when there is one (decided once per wave task
-// by k_plan_parts), else decided here.  Waves with a slow lane take the
-// per-lane walk.
-__device__ inline bool walk_of(const PartPlan &pp, uint32_t wt, const uint32_t *__restrict__ cstart, uint32_t cc,
-                               const StepParams &P, bool slow, UnionRows &U, uint32_t &count)
+// Whether a wave task takes the union walk, and then its box, from the
+// step's part plan.
+__device__ inline bool walk_of(const PartPlan &pp, uint32_t wt, UnionRows &U)
 {
-    if (pp.walk) {
-        const int4 a = pp.walk[2u * wt], b = pp.walk[2u * wt + 1u];
-        U.x0 = __builtin_amdgcn_readfirstlane(a.x);
-        U.x1 = __builtin_amdgcn_readfirstlane(a.y);
-        U.y0 = __builtin_amdgcn_readfirstlane(a.z);
-        U.y1 = __builtin_amdgcn_readfirstlane(a.w);
-        U.z0 = __builtin_amdgcn_readfirstlane(b.x);
-        U.z1 = __builtin_amdgcn_readfirstlane(b.y);
-        count = (uint32_t)__builtin_amdgcn_readfirstlane(b.z);
-        return (__builtin_amdgcn_readfirstlane(b.w) & kWalkBox) != 0;
-    }
-    uint32_t own = kNoOwn;
-    return plan_union(cstart, cc, P, U, count, own) && !__any(slow);
+    const int4 a = pp.walk[2u * wt], b = pp.walk[2u * wt + 1u];
+    U.x0 = __builtin_amdgcn_readfirstlane(a.x);
+    U.x1 = __builtin_amdgcn_readfirstlane(a.y);
+    U.y0 = __builtin_amdgcn_readfirstlane(a.z);
+    U.y1 = __builtin_amdgcn_readfirstlane(a.w);
+    U.z0 = __builtin_amdgcn_readfirstlane(b.x);
+    U.z1 = __builtin_amdgcn_readfirstlane(b.y);
+    const int w = __builtin_amdgcn_readfirstlane(b.w);
+    U.segments = (w & (int)kWalkSegments) != 0;
+    return (w & (int)kWalkBox) != 0;
 }
 
 // Length of the lane's own candidate sequence (its (2R + 1)^3 stencil).
@@ -916,122 +981,163 @@ __device__ inline uint32_t own_length(const PartPlan &pp, uint32_t s, const uint
     return stencil_length(cstart, cc, P);
 }
 
-// Scalar union walk: the positions [lo, hi) of the union's flattened
-// candidate sequence as wave-uniform runs (slots ascending), each split at
-// the wave's own slots [first, first + 64) so only that run carries the
-// self test.  run(j0, j1, self) walks slots [j0, j1); the candidate
-// records are then scalar loads broadcast to the lanes through SGPRs.
-template <class Run, class Layer>
-__device__ inline void scalar_union_walk(const uint32_t *__restrict__ cstart, const UnionRows &U,
-                                         const StepParams &P, uint32_t lo, uint32_t hi, uint32_t first, Run run,
-                                         Layer layer)
+__device__ inline void wave_lds_sync()
 {
-    uint32_t off = 0;
-    for (int z = U.z0; z <= U.z1; ++z) {
-        for (int y = U.y0; y <= U.y1; ++y) {
-            const uint32_t r0 = row_base(P, y, z);
-            const uint32_t b = __builtin_amdgcn_readfirstlane(cstart[r0 + (uint32_t)U.x0]);
-            const uint32_t e = __builtin_amdgcn_readfirstlane(cstart[r0 + (uint32_t)U.x1 + 1u]);
-            const uint32_t s0 = max(lo, off), s1 = min(hi, off + (e - b));
-            if (s0 < s1) {
-                const uint32_t j0 = b + (s0 - off), j1 = b + (s1 - off);
-                const uint32_t m0 = min(max(j0, first), j1), m1 = min(max(j0, first + 64u), j1);
-                if (j0 < m0)
-                    run(j0, m0, std::false_type{});
-                if (m0 < m1)
-                    run(m0, m1, std::true_type{});
-                if (m1 < j1)
-                    run(m1, j1, std::false_type{});
-            }
-            off += e - b;
-        }
-        layer();
-    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Union walk staged through LDS.  The wave's union candidates, flattened
-// in row order (rows as for_each_row visits them, slots ascending), are
-// fetched 64 at a time -- one coalesced load per lane and record array, a
-// chunk ahead of their use -- into a per-wave LDS double buffer, then read
-// back by all lanes with one broadcast LDS read per record, so the
-// candidate loop never waits on a global load and never pays per-row
-// overhead.  Lanes past the end stage a sentinel (position +inf, slot ~0)
-// that fails every test, so chunks run in groups of four unchecked.
+// Union walk.  The wave's union candidates, flattened in row order (rows as
+// for_each_row visits them, slots ascending, the rows of each z-layer
+// starting at a multiple of 64), are fetched 64 at a time -- one coalesced
+// load per lane and record array, a chunk ahead of their use -- into a
+// per-wave LDS double buffer, then read back by all lanes together, so the
+// candidate loop never waits on a global load, never pays per-row overhead,
+// and its operands are vector registers (fed from scalar registers the same
+// loop issues its three subtractions at half rate).  Places that hold no
+// candidate stage a record far away, with slot ~0, that fails every test, so
+// chunks run in groups of four unchecked.
+constexpr float kFarAway = 1.0e18f;  // its square is finite
+constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
+
+// One record array (positions, w unused) is kept as three coordinate arrays:
+// four candidates are three 16-byte reads instead of four (a read that all
+// lanes share still returns 1 KB: 8 cycles of the LDS that four SIMDs share).
 template <int NV>
-struct StageBuf {
-    float4 rec[2][NV][64];
-    uint32_t slot[2][64];
+struct ChunkRecords {
+    float4 rec[NV][64];
+};
+template <>
+struct ChunkRecords<1> {
+    alignas(16) float x[64], y[64], z[64];
 };
 
-// Walks the positions [lo, hi) of the flattened sequence.
-template <int NV, class Visit>
-__device__ inline void staged_union_walk(const uint32_t *__restrict__ cstart, const UnionRows &U,
-                                         const StepParams &P, uint32_t lo, uint32_t hi,
-                                         const float4 *const (&src)[NV], StageBuf<NV> &sb, Visit visit)
+template <int NV>
+struct UnionStage {
+    ChunkRecords<NV> chunk[2];
+    uint32_t slot[2][64];
+    // rows: first flattened position, end, and slot less position
+    uint32_t start[65], end[65], shift[65];
+    uint32_t ny;           // rows of a z-layer
+    uint32_t segment[64];  // of each lane, when segments are walked
+};
+
+// The row table of U in T; returns the length of the flattened sequence
+// (layers padded).  Every lane of the wave calls it.
+template <int NV>
+__device__ inline uint32_t union_rows(const uint32_t *__restrict__ cstart, const UnionRows &U, uint32_t cc, bool active,
+                                      const StepParams &P, UnionStage<NV> &T)
 {
     const uint32_t lane = threadIdx.x & 63u;
-    const int ny = U.y1 - U.y0 + 1;
-    const int nrows = ny * (U.z1 - U.z0 + 1);  // at most (union_span + 2R)^2 <= 64 lanes
-    uint32_t b = 0, len = 0;
-    if ((int)lane < nrows) {
-        const uint32_t r0 = row_base(P, U.y0 + (int)lane % ny, U.z0 + (int)lane / ny);
-        b = cstart[r0 + (uint32_t)U.x0];
-        len = cstart[r0 + (uint32_t)U.x1 + 1u] - b;
+    const uint32_t W = 2u * (uint32_t)P.reach + 1u;
+    uint32_t ny, nrows, b = 0, len = 0;
+    if (U.segments) {
+        const uint64_t heads = segment_heads(cc, active);
+        ny = W;
+        nrows = W * W * (uint32_t)__builtin_popcountll(heads);
+        segment_row(cstart, cc, active, heads, P, b, len);
+        const uint64_t upto = (2ull << lane) - 1ull;  // lanes 0 .. lane
+        T.segment[lane] = active ? (uint32_t)__builtin_popcountll(heads & upto) - 1u : 0u;
+    } else {
+        ny = (uint32_t)(U.y1 - U.y0 + 1);
+        nrows = ny * (uint32_t)(U.z1 - U.z0 + 1);  // at most (union_span + 2R)^2 <= 64 lanes
+        if (lane < nrows) {
+            const uint32_t r0 = row_base(P, U.y0 + (int)(lane % ny), U.z0 + (int)(lane / ny));
+            b = cstart[r0 + (uint32_t)U.x0];
+            len = cstart[r0 + (uint32_t)U.x1 + 1u] - b;
+        }
     }
-    const uint32_t end = wave_inclusive_scan(len);  // flattened end of the lane's row
-    const uint32_t total = min(__builtin_amdgcn_readlane(end, 63), hi);
-    const uint32_t shift = b - (end - len);         // slot = flattened position + shift
+    const uint32_t sum = wave_inclusive_scan(len);
+    const uint32_t before = (uint32_t)__shfl((int)sum, (int)(lane - ny) & 63, 64);
+    uint32_t pad = 0;  // behind the last row of a layer
+    if (lane < nrows && lane % ny == ny - 1u)
+        pad = (0u - (sum - (lane >= ny ? before : 0u))) & 63u;
+    const uint32_t end = wave_inclusive_scan(len + pad);
+    const uint32_t start = end - len - pad;
+    T.start[lane] = lane < nrows ? start : 0xFFFFFFFFu;
+    T.end[lane] = start + len;
+    T.shift[lane] = b - start;
+    if (lane == 0u) {
+        T.start[64] = 0xFFFFFFFFu;
+        T.end[64] = 0u;
+        T.shift[64] = 0u;
+        T.ny = ny;
+    }
+    wave_lds_sync();
+    return (uint32_t)__builtin_amdgcn_readlane((int)end, 63);
+}
+
+// Part `part` of `nparts` equal slices (whole chunks) of a flattened sequence.
+__device__ inline void part_slice(uint32_t total, uint32_t part, uint32_t nparts, uint32_t &lo, uint32_t &hi)
+{
+    const uint64_t chunks = (total + 63u) >> 6;
+    lo = (uint32_t)(chunks * part / nparts) << 6;
+    hi = (uint32_t)(chunks * (part + 1u) / nparts) << 6;
+}
+
+// Walks the positions [lo, hi) (multiples of 64) of the table's sequence:
+// chunk(records, slots, n, odd, layer) for each 64 of them, n candidates (a
+// multiple of four with the ones far away), all of z-layer `layer` (2R + 1 to
+// a segment).  odd: the
+// chunk holds some of the wave's own slots [first, first + 64) or, with
+// FINITE, a record that is not finite.
+template <int NV, bool FINITE, class Chunk>
+__device__ inline void union_walk(uint32_t lo, uint32_t hi, uint32_t first, const float4 *const (&src)[NV],
+                                  UnionStage<NV> &T, Chunk chunk)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t ny = __builtin_amdgcn_readfirstlane(T.ny);
+    uint32_t row = 0, next = T.start[1];
     auto fetch = [&](uint32_t f0, float4(&r)[NV], uint32_t &slot) {
         const uint32_t f = f0 + lane;
-        uint32_t row = 0;
-        for (int k = 0; k < nrows; ++k)
-            row += f >= (uint32_t)__builtin_amdgcn_readlane(end, k) ? 1u : 0u;
-        const uint32_t sh = (uint32_t)__shfl((int)shift, (int)min(row, 63u), 64);
-        if (f < total) {
-            slot = f + sh;
+        while (f >= next) {  // ends at the last row: the starts behind it are ~0
+            ++row;
+            next = T.start[row + 1u];
+        }
+        if (f < T.end[row]) {
+            slot = f + T.shift[row];
 #pragma unroll
             for (int v = 0; v < NV; ++v)
                 r[v] = src[v][slot];
         } else {
-            slot = 0xFFFFFFFFu;
-            r[0] = make_float4(__builtin_inff(), __builtin_inff(), __builtin_inff(), 0.0f);
+            slot = kNoSlot;
+            r[0] = make_float4(kFarAway, kFarAway, kFarAway, 0.0f);
 #pragma unroll
             for (int v = 1; v < NV; ++v)
                 r[v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
     };
-    const uint32_t nch = total > lo ? (total - lo + 63u) >> 6 : 0u;
     float4 nr[NV];
-    uint32_t ns = 0;
-    if (nch)
+    uint32_t ns = kNoSlot;
+    if (lo < hi)
         fetch(lo, nr, ns);
-    for (uint32_t c = 0; c < nch; ++c) {
-        const uint32_t bs = c & 1u;
+    for (uint32_t f0 = lo, bs = 0; f0 < hi; f0 += 64u, bs ^= 1u) {
+        const uint32_t layer = (uint32_t)__builtin_amdgcn_readfirstlane((int)row) / ny;
+        bool odd = ns - first < 64u;
+        if (FINITE) {
+            float size = 0.0f;
 #pragma unroll
-        for (int v = 0; v < NV; ++v)
-            sb.rec[bs][v][lane] = nr[v];
-        sb.slot[bs][lane] = ns;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (c + 1u < nch)
-            fetch(lo + ((c + 1u) << 6), nr, ns);
-        const uint32_t cnt = min(64u, total - lo - (c << 6));
-        const uint32_t cnt4 = (cnt + 3u) & ~3u;
-        for (uint32_t k = 0; k < cnt4; k += 4u) {
-            // all four records and slots in registers before the first use
-            float4 q[4][NV];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int v = 0; v < NV; ++v)
-                    q[i][v] = sb.rec[bs][v][k + i];
-            const uint4 j4 = *reinterpret_cast<const uint4 *>(&sb.slot[bs][k]);
-            visit(j4.x, q[0]);
-            visit(j4.y, q[1]);
-            visit(j4.z, q[2]);
-            visit(j4.w, q[3]);
+            for (int v = 0; v < NV; ++v)
+                size += fabsf(nr[v].x) + fabsf(nr[v].y) + fabsf(nr[v].z) + fabsf(nr[v].w);
+            odd = odd || !(size <= 8.0f * kFarAway);
         }
+        const bool any_odd = __any(odd);
+        const uint32_t n = (uint32_t)__builtin_popcountll(__ballot(ns != kNoSlot));
+        if constexpr (NV == 1) {
+            T.chunk[bs].x[lane] = nr[0].x;
+            T.chunk[bs].y[lane] = nr[0].y;
+            T.chunk[bs].z[lane] = nr[0].z;
+        } else {
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                T.chunk[bs].rec[v][lane] = nr[v];
+        }
+        T.slot[bs][lane] = ns;
+        wave_lds_sync();
+        if (f0 + 64u < hi)
+            fetch(f0 + 64u, nr, ns);
+        chunk(T.chunk[bs], T.slot[bs], (n + 3u) & ~3u, any_odd, layer);
     }
 }
 
@@ -1059,28 +1165,12 @@ struct Stage {
     StagedLayer layer[3];
 };
 
-__device__ inline void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // *src of each lane into dst + lane (dst wave-uniform), without registers
 // in between; the caller waits for vmcnt.
 __device__ inline void load_to_lds(const float *src, float *dst)
 {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
                                      (__attribute__((address_space(3))) void *)dst, 4, 0, 0);
-}
-
-// x in a vector register: an instruction with a scalar-register operand
-// issues at half the rate of one without (measured: 4.4 against 2.3 cycles a
-// wave for add and multiply).
-__device__ inline float in_vgpr(float x)
-{
-    asm("" : "+v"(x));
-    return x;
 }
 
 struct __attribute__((packed, aligned(4))) Bounds4 {
@@ -1091,8 +1181,8 @@ struct __attribute__((packed, aligned(4))) Bounds4 {
 // are short, runs its density pass at once: one block of three waves per
 // task, a wave for each z-layer of the stencil.
 //
-// Short walks (the largest own stencil at most kPartCandidates /
-// kLaneWalkWeight candidates, cells of h or larger) are staged: each wave
+// Short walks (the largest own stencil at most kShortWalk candidates, cells
+// of h or larger) are staged: each wave
 // copies the three rows of its layer, for every segment of the task's lanes,
 // to LDS with asynchronous loads, all in flight together, and its lanes walk
 // their own cut stencil (for_each_cut_row's cells, in its order) from there.
@@ -1150,12 +1240,9 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
             if (y >= 0 && y < P.ny && z >= 0 && z < P.nz)
                 v[r] = *reinterpret_cast<const Bounds4 *>(cstart + row_base(P, y, z) + (uint32_t)xs);
         }
-        // segments: lanes are in cell order, so those of one (y, z) row of
-        // cells are consecutive and ascend in x
         const uint32_t yz = cc & ~kSlowBit & ~2047u;
-        const uint32_t before = (uint32_t)__shfl_up((int)yz, 1, 64);
-        const bool head = active && (lane == 0u || yz != before);
-        const uint64_t heads = __ballot(head);
+        const uint64_t heads = segment_heads(cc, active);
+        const bool head = (heads >> lane & 1ull) != 0ull;
         const uint32_t nact = (uint32_t)__builtin_popcountll(__ballot(active));
         const uint32_t nseg = (uint32_t)__builtin_popcountll(heads);
         const uint64_t upto = (2ull << lane) - 1ull;  // lanes 0 .. lane
@@ -1250,7 +1337,7 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
         own = layers[0].own[lane] + layers[1].own[lane] + layers[2].own[lane];
         const uint32_t longest = (uint32_t)wave_max_i((int)own);
         if (__builtin_amdgcn_readfirstlane(layers[0].fits & layers[1].fits & layers[2].fits) != 0u &&
-            longest * kLaneWalkWeight <= kPartCandidates) {
+            longest <= kShortWalk) {
             const float h2 = in_vgpr(P.h2);
             float acc = 0.0f;
             uint32_t mask[3][kStageWords];
@@ -1287,10 +1374,7 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
                                 z = *reinterpret_cast<const float4 *>(&stage.z[from + k + 4u]);
 #pragma unroll
                                 for (int i = 0; i < 4; ++i) {
-                                    // max(u, 0); as a clamp to [0, 1] it
-                                    // comes with the subtraction
-                                    float t = decltype(unit_tag)::value ? __builtin_amdgcn_fmed3f(u[i], 0.0f, 1.0f)
-                                                                        : fmaxf(u[i], 0.0f);
+                                    float t = positive<decltype(unit_tag)::value>(u[i]);
                                     if (decltype(own_row)::value)
                                         t = (k + (uint32_t)i != self) ? t : 0.0f;
                                     acc = fmaf(t * t, t, acc);
@@ -1363,10 +1447,10 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
             }
             if (lz != 0)
                 return;
-            UnionRows U{0, 0, 0, 0, 0, 0};
+            UnionRows U{0, 0, 0, 0, 0, 0, false};
             uint32_t ucount = 0, unused = kNoOwn, w = kWalkUnion | kWalkSummed;
-            if (!listing && plan_union(cstart, cc, P, U, ucount, unused) && !any_slow)
-                w |= kWalkBox;  // for the force pass
+            if (!listing && plan_union(cstart, cc, active, P, U, ucount, unused) && !any_slow)
+                w |= kWalkBox | (U.segments ? kWalkSegments : 0u);  // for the force pass
             if (active) {
                 const float4 vs = vel[s];
                 const float sum = (acc + layers[1].sum[lane]) + layers[2].sum[lane];
@@ -1389,30 +1473,32 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
     }
     if (lz != 0)
         return;
-    UnionRows U{0, 0, 0, 0, 0, 0};
+    UnionRows U;
     uint32_t ucount = 0, len, fresh = kNoOwn;
-    const bool use_union = plan_union(cstart, cc, P, U, ucount, fresh) && !any_slow;
-    if (use_union) {
+    const bool use_union = plan_union(cstart, cc, active, P, U, ucount, fresh) && !any_slow;
+    if (__builtin_amdgcn_readfirstlane(own) == kNoOwn)  // wave-uniform
+        own = fresh;
+    if (!use_union && __builtin_amdgcn_readfirstlane(own) == kNoOwn)
+        own = stencil_length(cstart, cc, P);
+    const uint32_t longest = (uint32_t)wave_max_i((int)own);  // kNoOwn (-1): all lanes in one cell
+    if (longest <= kShortWalk) {
+        len = 0;  // left whole: it records neighbour lists, which the force pass then visits
+    } else if (use_union) {
         len = ucount;
     } else {
-        // Per-lane walks cost about three times as much per candidate
-        // as the wave-uniform walk (divergent gathers, no shared loads),
-        // so they count three times toward the part size; with slow
-        // lanes (m_ij counted from the 27 buckets per neighbour, the
-        // wave waiting on them) more again, unless the walk is short
-        // enough to be left whole and record neighbour lists, which the
-        // force pass then visits.
-        if (__builtin_amdgcn_readfirstlane(own) == kNoOwn)  // wave-uniform
-            own = __builtin_amdgcn_readfirstlane(fresh) == kNoOwn ? stencil_length(cstart, cc, P) : fresh;
-        const uint32_t longest = (uint32_t)wave_max_i((int)own);
-        const bool whole = longest * kLaneWalkWeight <= kPartCandidates;
-        len = longest * (!whole && any_slow ? kSlowWalkWeight : kLaneWalkWeight);
-        if (active)
-            pp.own[s] = own;
+        // Per-lane walks cost several times as much per candidate as the
+        // union walk (divergent gathers, no shared loads), so they count
+        // several times toward the part size; with slow lanes (m_ij counted
+        // from the 27 buckets per neighbour, the wave waiting on them) more
+        // again.
+        len = longest * (any_slow ? kSlowWalkWeight : kLaneWalkWeight);
     }
+    if (!use_union && active)
+        pp.own[s] = own;
     if (lane == 0u) {
         pp.walk[2u * task] = make_int4(U.x0, U.x1, U.y0, U.y1);
-        pp.walk[2u * task + 1u] = make_int4(U.z0, U.z1, (int)ucount, use_union ? (int)(kWalkUnion | kWalkBox) : 0);
+        pp.walk[2u * task + 1u] = make_int4(
+            U.z0, U.z1, (int)ucount, use_union ? (int)(kWalkUnion | kWalkBox | (U.segments ? kWalkSegments : 0u)) : 0);
         pp.measure[task] = len;
         // only walks that may be split count toward the scene's part size
         if (len > kPartCandidates)
@@ -1527,39 +1613,51 @@ __device__ inline void for_each_part(const SceneSet &S, const PartPlan &pp, uint
     }
 }
 
-__device__ inline float load_agent(const float *p)
-{
-    return __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t *>(p), __ATOMIC_RELAXED,
-                                             __HIP_MEMORY_SCOPE_AGENT));
-}
-
 // Part `part` of wave task w stores its N partial sums; the last part to
 // finish gets every part's sums added in part order in v and returns true
 // (the others return false).  Every lane of the wave calls it.
+//
+// The parts of a task run on different XCDs, whose L2s do not see each
+// other's lines.  The sums are stored and loaded at agent scope (past the
+// L2), and each wave waits for its own stores before it counts itself
+// finished, so the last one finds every sum in memory.  A device-wide fence
+// would do the same by writing back the whole L2, once per part: with some
+// 42,000 parts a step those fences took a quarter of a density pass.
 template <int N>
 __device__ inline bool combine_parts(const PartPlan &pp, uint32_t w, uint32_t part, uint32_t nparts, float (&v)[N])
 {
+    static_assert(N <= 4, "a part task has room for four sums per lane");
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t base = __builtin_amdgcn_readfirstlane(pp.off[w]);
-    float *mine = reinterpret_cast<float *>(pp.buf + ((size_t)base + part) * 64u + lane);
+    auto at = [&](uint32_t q, int k) {  // sum k of part q: the lanes side by side
+        return reinterpret_cast<uint32_t *>(pp.buf) + (((size_t)base + q) * 4u + (uint32_t)k) * 64u + lane;
+    };
 #pragma unroll
     for (int k = 0; k < N; ++k)
-        mine[k] = v[k];
-    __threadfence();
+        __hip_atomic_store(at(part, k), __float_as_uint(v[k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // keeps the order in the program ...
+    __builtin_amdgcn_s_waitcnt(0x0F70);                     // ... and vmcnt 0: the stores are done
     uint32_t prev = 0;
     if (lane == 0u)
-        prev = atomicAdd(&pp.done[w], 1u);
+        prev = __hip_atomic_fetch_add(&pp.done[w], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     prev = __builtin_amdgcn_readfirstlane(prev);
     if (prev + 1u != nparts)
         return false;
-    __threadfence();
-    for (uint32_t q = 0; q < nparts; ++q) {
-        const float *src = reinterpret_cast<const float *>(pp.buf + ((size_t)base + q) * 64u + lane);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    for (uint32_t q0 = 0; q0 < nparts; q0 += 4u) {  // four parts' loads in flight
+        float x[4][N];
 #pragma unroll
-        for (int k = 0; k < N; ++k) {
-            const float x = load_agent(src + k);
-            v[k] = q == 0u ? x : v[k] + x;
-        }
+        for (uint32_t i = 0; i < 4u; ++i)
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+                x[i][k] = __uint_as_float(__hip_atomic_load(at(min(q0 + i, nparts - 1u), k), __ATOMIC_RELAXED,
+                                                            __HIP_MEMORY_SCOPE_AGENT));
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+            if (q0 + i < nparts)
+#pragma unroll
+                for (int k = 0; k < N; ++k)
+                    v[k] = q0 + i == 0u ? x[i][k] : v[k] + x[i][k];
     }
     if (lane == 0u)
         pp.done[w] = 0u;  // ready for the next pass
@@ -1580,6 +1678,7 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
     NeighborDump dump, PartPlan pp, NeighborLists nl)
 {
     constexpr bool kCount = MODE >= 1;
+    __shared__ UnionStage<1> stage[MODE == 0 || MODE == 3 ? BLOCK / 64 : 1];
     for_each_part<BLOCK, true>(S, pp, pp.queue, [&](uint32_t wt, uint32_t part, uint32_t nparts) {
         Lane L;
         bool active;
@@ -1633,77 +1732,78 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
         // take the per-lane walk, so the union walk needs no m_ij.  A split
         // task walks its slice [part, part + 1) / nparts of the sequence.
         UnionRows U;
-        uint32_t ucount = 0;
-        if ((MODE == 0 || MODE == 3) && walk_of(pp, wt, cstart, cc, P, slow, U, ucount)) {
-            // Wave-uniform candidate j: scalar loads, four records at a time
-            // (density is too short per candidate to feed from LDS).
-            const uint32_t lo = (uint32_t)((uint64_t)ucount * part / nparts);
-            const uint32_t hi = (uint32_t)((uint64_t)ucount * (part + 1u) / nparts);
-            auto cand = [&](uint32_t j, float4 q, auto self_tag) {
-                float dx, dy, dz;
-                const float d2 = dist2_ref(pi, q, dx, dy, dz);
-                // Branch-free: h2 - d2 > 0 exactly when d2 < h2 (the float
-                // difference of unequal values is nonzero), so clamping it
-                // at 0 turns a failing candidate into a +0 term, which
-                // leaves acc unchanged bit for bit.
-                float t = fmaxf(h2 - d2, 0.0f);
-                if (decltype(self_tag)::value)
-                    t = (j != s) ? t : 0.0f;
-                acc = fmaf(t * t, t, acc);
-                if (kCount)
-                    cnt += t > 0.0f ? 1u : 0u;
-            };
+        if ((MODE == 0 || MODE == 3) && walk_of(pp, wt, U)) {
+            UnionStage<1> &T = stage[threadIdx.x >> 6];
+            uint32_t lo, hi;
+            part_slice(union_rows(cstart, U, cc, active, P, T), part, nparts, lo, hi);
+            const float4 *const src[1] = {pos};
+            const float h2v = in_vgpr(h2);
             // An unsplit task records its lanes' neighbours here too (in
             // walk order, as the per-lane walk below), until one of them
             // has more than a list holds: the force pass then visits 30-odd
             // listed slots instead of the union's hundreds of candidates
             // (64 scenes of 1.06 million particles: 415 -> 169 us).
             bool listing = nl.list && nparts == 1u;
-            uint32_t nn = 0;
+            uint32_t nn = 0, at_layer = kNoSlot;
             uint32_t *lp = nl.list + s;
-            auto record = [&](uint32_t j, float4 q, auto self_tag) {
-                float dx, dy, dz;
-                const float d2 = dist2_ref(pi, q, dx, dy, dz);
-                float t = fmaxf(h2 - d2, 0.0f);
-                if (decltype(self_tag)::value)
-                    t = (j != s) ? t : 0.0f;
-                acc = fmaf(t * t, t, acc);
-                if (t > 0.0f) {
-                    if (kCount)
-                        ++cnt;
-                    if (nn < kListMax) {
-                        *lp = j;
-                        lp += nl.stride;
+            const uint32_t W = 2u * (uint32_t)P.reach + 1u;
+            float4 me = pi;  // far away from the candidates of other lanes' segments
+            auto walk = [&](auto unit_tag) {
+                union_walk<1, false>(lo, hi, L.first, src, T, [&](const ChunkRecords<1> &c, const uint32_t *slots,
+                                                                      uint32_t n, bool odd, uint32_t lz) {
+                    if (lz != at_layer) {
+                        layer();
+                        at_layer = lz;
+                        if (U.segments)
+                            me.x = T.segment[threadIdx.x & 63u] == lz / W ? pi.x : kFarAway;
                     }
-                    ++nn;
-                }
+                    // Branch-free: h2 - d2 > 0 exactly when d2 < h2 (the float
+                    // difference of unequal values is nonzero), so clamping it
+                    // at 0 turns a failing candidate into a +0 term, which
+                    // leaves acc unchanged bit for bit.
+                    auto term = [&](float x, float y, float z) {
+                        float dx, dy, dz;
+                        return positive<decltype(unit_tag)::value>(
+                            h2v - dist2_ref(me, make_float4(x, y, z, 0.0f), dx, dy, dz));
+                    };
+                    if (listing || odd) {
+                        for (uint32_t k = 0; k < n; ++k) {
+                            const uint32_t j = slots[k];
+                            const float t = j != s ? term(c.x[k], c.y[k], c.z[k]) : 0.0f;
+                            acc = fmaf(t * t, t, acc);
+                            if (t > 0.0f) {
+                                if (kCount)
+                                    ++cnt;
+                                if (listing && nn < kListMax) {
+                                    *lp = j;
+                                    lp += nl.stride;
+                                }
+                                ++nn;
+                            }
+                        }
+                        listing = listing && !__any(nn > kListMax);
+                        return;
+                    }
+                    for (uint32_t k = 0; k < n; k += 4u) {
+                        const float4 x = *reinterpret_cast<const float4 *>(&c.x[k]);
+                        const float4 y = *reinterpret_cast<const float4 *>(&c.y[k]);
+                        const float4 z = *reinterpret_cast<const float4 *>(&c.z[k]);
+                        const float t[4] = {term(x.x, y.x, z.x), term(x.y, y.y, z.y), term(x.z, y.z, z.z),
+                                            term(x.w, y.w, z.w)};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            acc = fmaf(t[i] * t[i], t[i], acc);
+                            if (kCount)
+                                cnt += t[i] > 0.0f ? 1u : 0u;
+                        }
+                    }
+                });
             };
-            scalar_union_walk(cstart, U, P, lo, hi, L.first, [&](uint32_t j0, uint32_t j1, auto self_tag) {
-                const float4 *p = pos + j0;
-                uint32_t j = j0;
-                if (listing) {
-                    for (; j + 4u <= j1; j += 4u, p += 4) {
-                        const float4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
-                        record(j, q0, self_tag);
-                        record(j + 1u, q1, self_tag);
-                        record(j + 2u, q2, self_tag);
-                        record(j + 3u, q3, self_tag);
-                    }
-                    for (; j < j1; ++j, ++p)
-                        record(j, p[0], self_tag);
-                    listing = !__any(nn > kListMax);
-                    return;
-                }
-                for (; j + 4u <= j1; j += 4u, p += 4) {
-                    const float4 q0 = p[0], q1 = p[1], q2 = p[2], q3 = p[3];
-                    cand(j, q0, self_tag);
-                    cand(j + 1u, q1, self_tag);
-                    cand(j + 2u, q2, self_tag);
-                    cand(j + 3u, q3, self_tag);
-                }
-                for (; j < j1; ++j, ++p)
-                    cand(j, p[0], self_tag);
-            }, layer);
+            if (P.h2 <= 1.0f)
+                walk(std::true_type{});
+            else
+                walk(std::false_type{});
+            layer();
             if (listing)
                 listed = nn;
         } else if ((MODE == 0 || MODE == 3) && nl.list && nparts == 1u) {
@@ -1830,16 +1930,16 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
             }
             for_each_row_span(cstart, cc, P, lo, hi, [&](uint32_t b, uint32_t e) {
                 uint32_t j = b;
-                for (; j + 1u < e; j += 2u) {  // two candidates in flight
-                    const float4 q0 = pos[j];
-                    const float4 q1 = pos[j + 1u];
-                    if (j != s)
-                        body(j, q0);
-                    if (j + 1u != s)
-                        body(j + 1u, q1);
+                for (; j + 3u < e; j += 4u) {  // four candidates in flight
+                    const float4 q[4] = {pos[j], pos[j + 1u], pos[j + 2u], pos[j + 3u]};
+#pragma unroll
+                    for (uint32_t i = 0; i < 4u; ++i)
+                        if (j + i != s)
+                            body(j + i, q[i]);
                 }
-                if (j < e && j != s)
-                    body(j, pos[j]);
+                for (; j < e; ++j)
+                    if (j != s)
+                        body(j, pos[j]);
             }, layer);
         }
         acc = sum;
@@ -1978,23 +2078,26 @@ __device__ inline void integrate_and_walls(float4 &x, float4 &v, float fx, float
     }
 }
 
-// The force of one passing neighbour, accumulated into (fx, fy, fz):
+// The force of one candidate, accumulated into (fx, fy, fz):
 //   cp = -m spikyGrad (p_i + p_j) m_ij (0.5 / rho_j) (h - r)^2 / r
 //   cv = 2 mu m spikyLap (h - r) m_ij (0.5 / rho_j)
 //   F += cp d + cv (v_j - v_i)
 // q = (x_j, 0.5 / rho_j), w = (v_j, p_j), d = x_j - x_i, am = m_ij (0.5 / rho_j).
+// r and h - r are the reference's values bit for bit (near the support edge
+// h - r cancels, and an error in r would be amplified).  A candidate that is
+// no neighbour has d2 >= fl(h h), so r >= h (the root of the rounded square
+// is h itself) and h - r clamps to 0: it adds zeros, without a test.
+template <bool UNIT>
 __device__ inline void force_pair(float d2, float dx, float dy, float dz, float am, float4 w, float4 vi,
                                   float p_i, float h, float neg_m_spg, float mu2_m_lap, float &fx,
                                   float &fy, float &fz)
 {
-    // r = sqrt(d2) correctly rounded and hr = h - r exactly as the
-    // reference forms them: near the support edge h - r cancels and any
-    // error in r would be amplified.
-    const float r = sqrt_rn(d2);
-    const float rinv = __builtin_amdgcn_rcpf(r);
-    const float hr = h - r;
-    const float cp = neg_m_spg * (p_i + w.w) * am * (hr * hr) * rinv;
-    const float cv = mu2_m_lap * hr * am;
+    float rinv;
+    const float r = root(d2, rinv);
+    const float hr = positive<UNIT>(h - r);
+    const float u = hr * am;
+    const float cp = ((p_i + w.w) * neg_m_spg) * u * (hr * rinv);
+    const float cv = u * mu2_m_lap;
     fx = fmaf(cp, dx, fx);
     fy = fmaf(cp, dy, fy);
     fz = fmaf(cp, dz, fz);
@@ -2018,7 +2121,7 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
     uint32_t *__restrict__ cellcA, uint32_t *__restrict__ counts,
     float4 *__restrict__ force_out, SceneSet S, PartPlan pp, NeighborLists nl)
 {
-    __shared__ StageBuf<2> stage[BLOCK / 64];
+    __shared__ UnionStage<2> stage[BLOCK / 64];
     for_each_part<BLOCK, false>(S, pp, pp.queue ? pp.queue + 1 : nullptr, [&](uint32_t wt, uint32_t part,
                                                                       uint32_t nparts) {
         Lane L;
@@ -2036,8 +2139,8 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
         if (slow)
             ci = ref_cell(pi, P);
         const float p_i = vr.w;
-        const float h = P.h, h2 = P.h2, neg_m_spg = P.neg_m_spg;
-        const float mu2_m_lap = 2.0f * P.mu_m_lap;
+        const float h = in_vgpr(P.h), h2 = P.h2, neg_m_spg = in_vgpr(P.neg_m_spg);
+        const float mu2_m_lap = in_vgpr(2.0f * P.mu_m_lap);
         float fx = 0.0f, fy = 0.0f, fz = 0.0f;
 
         // The term of neighbour j in the order the walks visit it.
@@ -2050,7 +2153,7 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                 asm volatile("" : "+v"(cx), "+v"(cy), "+v"(cz));
                 am = q.w * (float)bucket_multiplicity(cx, cy, cz, __float_as_uint(posB[j].w) & 0xFFFFu);
             }
-            force_pair(d2, dx, dy, dz, am, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+            force_pair<false>(d2, dx, dy, dz, am, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
         };
         // Every lane holds its neighbour list (the density pass walked this
         // task per lane, unsplit): visit the listed slots four at a time,
@@ -2059,7 +2162,6 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
         const uint32_t listed = (nl.count && nparts == 1u) ? nl.count[s] : kNoList;
         const bool use_list = nl.count && nparts == 1u && __all(listed != kNoList);
         UnionRows U;
-        uint32_t ucount = 0;
         if (use_list) {
             const uint32_t groups = ((uint32_t)wave_max_i((int)listed) + 3u) >> 2;
             const uint32_t *ent = nl.list + s;
@@ -2089,18 +2191,52 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                 if (k + 3u < listed)
                     pair(j3, q3, w3);
             }
-        } else if (walk_of(pp, wt, cstart, cc, P, slow, U, ucount)) {  // as in k_density
+        } else if (walk_of(pp, wt, U)) {  // as in k_density
+            UnionStage<2> &T = stage[threadIdx.x >> 6];
+            uint32_t lo, hi;
+            part_slice(union_rows(cstart, U, cc, active, P, T), part, nparts, lo, hi);
             const float4 *const src[2] = {posR, velR};
-            const uint32_t lo = (uint32_t)((uint64_t)ucount * part / nparts);
-            const uint32_t hi = (uint32_t)((uint64_t)ucount * (part + 1u) / nparts);
-            staged_union_walk<2>(cstart, U, P, lo, hi, src, stage[threadIdx.x >> 6],
-                                 [&](uint32_t j, const float4(&r)[2]) {
-                const float4 q = r[0], w = r[1];  // (x_j, 0.5 / rho_j), (v_j, p_j)
-                float dx, dy, dz;
-                const float d2 = dist2_ref(pi, q, dx, dy, dz);
-                if (d2 < h2 && j != s)
-                    force_pair(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);  // am = q.w * 1
-            });
+            // Values that are not finite (or far beyond any scene's) would
+            // reach a lane through a candidate that is no neighbour (0 x inf):
+            // a chunk that holds some, and every chunk of a wave that does, is
+            // walked with a test per candidate, as are the wave's own slots.
+            const bool plain = __all(fabsf(pi.x) + fabsf(pi.y) + fabsf(pi.z) + fabsf(vi.x) + fabsf(vi.y) +
+                                         fabsf(vi.z) + fabsf(p_i) <= kFarAway);
+            const uint32_t W = 2u * (uint32_t)P.reach + 1u;
+            uint32_t at_layer = kNoSlot;
+            float4 me = pi;  // far away from the candidates of other lanes' segments
+            auto walk = [&](auto unit_tag) {
+                constexpr bool unit = decltype(unit_tag)::value;
+                union_walk<2, true>(lo, hi, L.first, src, T, [&](const ChunkRecords<2> &c, const uint32_t *slots,
+                                                                     uint32_t n, bool odd, uint32_t lz) {
+                    const float4(&rec)[2][64] = c.rec;
+                    float dx, dy, dz;
+                    if (U.segments && lz != at_layer) {
+                        at_layer = lz;
+                        me.x = T.segment[threadIdx.x & 63u] == lz / W ? pi.x : kFarAway;
+                    }
+                    if (odd || !plain) {
+                        for (uint32_t k = 0; k < n; ++k) {
+                            const float4 q = rec[0][k], w = rec[1][k];  // (x_j, 0.5 / rho_j), (v_j, p_j)
+                            const float d2 = dist2_ref(me, q, dx, dy, dz);
+                            if (d2 < h2 && slots[k] != s)
+                                force_pair<unit>(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                        }
+                        return;
+                    }
+                    for (uint32_t k = 0; k < n; k += 2u) {
+                        const float4 q0 = rec[0][k], w0 = rec[1][k], q1 = rec[0][k + 1u], w1 = rec[1][k + 1u];
+                        float d2 = dist2_ref(me, q0, dx, dy, dz);
+                        force_pair<unit>(d2, dx, dy, dz, q0.w, w0, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                        d2 = dist2_ref(me, q1, dx, dy, dz);
+                        force_pair<unit>(d2, dx, dy, dz, q1.w, w1, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                    }
+                });
+            };
+            if (P.h <= 1.0f)
+                walk(std::true_type{});
+            else
+                walk(std::false_type{});
         } else {
             uint32_t lo = 0, hi = 0xFFFFFFFFu;
             if (nparts > 1u) {
