@@ -3,6 +3,7 @@
 // serving loop.
 #pragma once
 
+#include <array>
 #include <vector>
 
 #include "sph_runtime.h"
@@ -43,6 +44,7 @@ struct BatchScene {
     StepParams P;  // constants, grid, slot range
     double lo[3] = {0.0, 0.0, 0.0}, hi[3] = {0.0, 0.0, 0.0};  // bounds the grid covers
     bool uploaded = false;
+    bool bounds_pending = false;  // lo, hi and the grid wait for the bounds the device found
     uint64_t steps = 0;  // steps since the upload
     double scale = 0.0;  // cell scale of the current grid (0: desc.cell_scale)
     double last_ratio = 0.0;  // candidates per neighbour at the last evaluation
@@ -53,6 +55,8 @@ int validate_desc(const sph_scene_desc_v1 &d);
 // Bounds of b's grid from its box and particles, then its grid (scene_regrid
 // with the scene's own cell scale).
 void scene_grid(BatchScene &b, const float *pos, uint32_t n);
+// The same from the bounds of the finite positions (min > max: none).
+void scene_grid(BatchScene &b, double pmin[3], double pmax[3]);
 // b's grid over its bounds with cell scale `scale` (0: desc.cell_scale).
 int scene_regrid(BatchScene &b, double scale);
 // A scene entry for desc (validated): constants, flags; no slot range yet.
@@ -68,7 +72,12 @@ struct Batch {
     uint64_t max_capacity = 0;  // particle capacity relayout may grow to (0: unbounded)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    DevBuf aos, xf;  // download staging
+    using GraphKey = std::array<uint64_t, 42>;
+    GraphKey captured{};     // what the launches of `exec` were given
+    bool complete = false;  // every scene has been uploaded since the scene list last changed
+    DevBuf aos, xf;  // download_particles staging
+    DevBuf bounds;   // bounds of every scene's last upload
+    HostStage stage;
     DevBuf gstat;    // grid statistic: candidates, neighbours per scene
     bool stat_ok = false;    // B order and cell ranges are those of the last step
     bool hold_grid = false;  // steps neither count nor re-grid (autotune trials)
@@ -100,8 +109,12 @@ struct Batch {
     int step(int nsteps);
     // nsteps steps on the current layout (no grid decisions)
     int step_plain(int nsteps);
-    // Captures the step into the graph when there is none (use_graph).
+    // Captures the step into the graph when there is none for the present
+    // buffers and sizes (use_graph).
     int capture();
+    GraphKey graph_key() const;
+    // Gives freshly uploaded scenes their grids (waits for the device).
+    int resolve_bounds();
     // Sampled candidates per neighbour of every scene (ratio[s]): fresh =
     // from the cell order of the current state (sorted here), else from
     // the last step's (0 if there is none).

@@ -48,7 +48,6 @@ int validate_desc(const sph_scene_desc_v1 &d)
 // least 16 h).  Depends on nothing but the scene.
 void scene_grid(BatchScene &b, const float *pos, uint32_t n)
 {
-    const sph_scene_desc_v1 &d = b.desc;
     double pmin[3] = {INFINITY, INFINITY, INFINITY}, pmax[3] = {-INFINITY, -INFINITY, -INFINITY};
     for (uint32_t i = 0; i < n; ++i)
         for (int k = 0; k < 3; ++k) {
@@ -58,6 +57,12 @@ void scene_grid(BatchScene &b, const float *pos, uint32_t n)
                 pmax[k] = std::max(pmax[k], v);
             }
         }
+    scene_grid(b, pmin, pmax);
+}
+
+void scene_grid(BatchScene &b, double pmin[3], double pmax[3])
+{
+    const sph_scene_desc_v1 &d = b.desc;
     double *lo = b.lo, *hi = b.hi;
     const double h = b.P.h;
     for (int k = 0; k < 3; ++k) {
@@ -184,6 +189,15 @@ int Batch::relayout(std::vector<BatchScene> next, const std::vector<int> &from)
     hipError_t e = hipStreamSynchronize(stream);
     if (e != hipSuccess)
         return hip_fail(e, "relayout");
+    if ((rc = resolve_bounds()))  // the bounds are kept by scene index
+        return rc;
+    for (size_t k = 0; k < next.size(); ++k)
+        if (from[k] >= 0 && next[k].bounds_pending) {  // taken from the list before its grid was known
+            const StepParams P = next[k].P;
+            next[k] = scenes[from[k]];
+            next[k].P.p_begin = P.p_begin;
+            next[k].P.p_end = P.p_end;
+        }
     drop_graph();
     // Destination of the moved state: the B arrays (scratch between steps)
     // when they are large enough, else fresh buffers with head room.
@@ -242,6 +256,7 @@ int Batch::relayout(std::vector<BatchScene> next, const std::vector<int> &from)
     }
     scenes = std::move(next);
     total_n = (uint32_t)total;
+    complete = false;
     layout_dirty = true;
     keys_dirty = true;
     stat_ok = false;
@@ -258,37 +273,38 @@ int Batch::upload(uint32_t s, const float *pos, const float *vel)
     }
     BatchScene &b = scenes[s];
     const uint32_t n = b.desc.n, p0 = b.P.p_begin;
-    scene_grid(b, pos, n);
-    std::vector<float4> p4(n), v4(n);
-    for (uint32_t i = 0; i < n; ++i) {
-        p4[i] = make_float4(pos[3 * (size_t)i], pos[3 * (size_t)i + 1], pos[3 * (size_t)i + 2], 0.0f);
-        float vx = vel ? vel[3 * (size_t)i] : 0.0f, vy = vel ? vel[3 * (size_t)i + 1] : 0.0f;
-        float vz = vel ? vel[3 * (size_t)i + 2] : 0.0f;
-        uint32_t id = i;
-        float idf;
-        std::memcpy(&idf, &id, 4);
-        v4[i] = make_float4(vx, vy, vz, idf);
-    }
+    int rc;
+    if ((rc = bounds.reserve(24ull * scenes.size())))
+        return rc;
+    // The caller's arrays go to the device as they are, into the neighbour
+    // lists (scratch between steps, at least ten times their size), and are
+    // spread into the particle arrays there, which also finds the bounds the
+    // grid needs.
     (void)hipStreamSynchronize(stream);
-    drop_graph();
-    ParticleArrays a = w.particles();
-    hipError_t e = hipMemcpyAsync(a.posA + p0, p4.data(), sizeof(float4) * (size_t)n, hipMemcpyHostToDevice, stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(a.velA + p0, v4.data(), sizeof(float4) * (size_t)n, hipMemcpyHostToDevice, stream);
+    const size_t bytes = 12ull * n;
+    float *raw = (float *)w.nlist.ptr, *raw_vel = raw + 3 * (size_t)n;
+    hipError_t e;
+    if (unsigned char *pinned = stage.small(2 * bytes)) {
+        std::memcpy(pinned, pos, bytes);
+        if (vel)
+            std::memcpy(pinned + bytes, vel, bytes);
+        e = hipMemcpyAsync(raw, pinned, vel ? 2 * bytes : bytes, hipMemcpyHostToDevice, stream);
+    } else {
+        e = hipMemcpyAsync(raw, pos, bytes, hipMemcpyHostToDevice, stream);
+        if (e == hipSuccess && vel)
+            e = hipMemcpyAsync(raw_vel, vel, bytes, hipMemcpyHostToDevice, stream);
+    }
     if (e != hipSuccess)
         return hip_fail(e, "upload");
-    launch_fill_u32(stream, (uint32_t *)(a.rhoB + p0), 0u, n);
-    launch_fill_u32(stream, (uint32_t *)(a.posR + p0), 0u, 4ull * n);
-    launch_fill_u32(stream, (uint32_t *)(a.velR + p0), 0u, 4ull * n);
-    launch_fill_u32(stream, (uint32_t *)(a.posB + p0), 0u, 4ull * n);
-    if (keep_force)
-        launch_fill_u32(stream, (uint32_t *)w.force.ptr + 4ull * p0, 0u, 4ull * n);
+    launch_load_state(stream, raw, vel ? raw_vel : nullptr, w.particles(),
+                      keep_force ? (float4 *)w.force.ptr : nullptr, p0, n, (int32_t *)bounds.ptr + 6 * s);
     e = hipStreamSynchronize(stream);
     if (e == hipSuccess)
         e = hipGetLastError();
     if (e != hipSuccess)
         return hip_fail(e, "upload");
     b.uploaded = true;
+    b.bounds_pending = true;
     b.steps = 0;
     b.scale = 0.0;
     b.last_ratio = 0.0;
@@ -297,21 +313,55 @@ int Batch::upload(uint32_t s, const float *pos, const float *vel)
     keys_dirty = true;
     stat_ok = false;
     // Once every scene holds particles, the first step's set-up (cells,
-    // scene table, keys, the automatic grid's first choice) runs here
-    // rather than inside the first step.
+    // scene table, keys, the automatic grid's first choice, the step's graph)
+    // runs here rather than inside the first step.  When a scene of several
+    // is replaced later, the others may follow: then the next step does it,
+    // once (64 scenes, each preparing all of them again: 13 ms).
     for (const BatchScene &o : scenes)
         if (!o.uploaded)
             return SPH_OK;
-    int rc;
+    if (complete && scenes.size() > 1)
+        return SPH_OK;
+    complete = true;
     if (!hold_grid && (rc = auto_grid()))
         return rc;
     if ((rc = prepare()))
         return rc;
-    if (use_graph && (rc = capture()))  // the step's graph too, outside the first step
+    if (use_graph && (rc = capture()))
         return rc;
     e = hipStreamSynchronize(stream);
     if (e != hipSuccess)
         return hip_fail(e, "upload");
+    return SPH_OK;
+}
+
+int Batch::resolve_bounds()
+{
+    bool any = false;
+    for (const BatchScene &b : scenes)
+        any = any || b.bounds_pending;
+    if (!any)
+        return SPH_OK;
+    std::vector<int32_t> bb(6 * scenes.size());
+    hipError_t e = hipMemcpyAsync(bb.data(), bounds.ptr, 24ull * scenes.size(), hipMemcpyDeviceToHost, stream);
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(stream);
+    if (e != hipSuccess)
+        return hip_fail(e, "bounds readback");
+    for (size_t s = 0; s < scenes.size(); ++s) {
+        BatchScene &b = scenes[s];
+        if (!b.bounds_pending)
+            continue;
+        double pmin[3], pmax[3];
+        for (int k = 0; k < 3; ++k) {
+            const int32_t lo = bb[6 * s + k], hi = bb[6 * s + 3 + k];
+            const bool none = lo == INT32_MAX;  // no finite coordinate on this axis
+            pmin[k] = none ? INFINITY : from_ordered(lo);
+            pmax[k] = none ? -INFINITY : from_ordered(hi);
+        }
+        scene_grid(b, pmin, pmax);
+        b.bounds_pending = false;
+    }
     return SPH_OK;
 }
 
@@ -321,6 +371,8 @@ int Batch::prepare()
     for (const BatchScene &b : scenes)
         if (!b.uploaded)
             return fail(SPH_E_STATE, "batch: every scene needs an upload before stepping");
+    if ((rc = resolve_bounds()))
+        return rc;
     if (layout_dirty) {
         uint64_t base = 0;
         std::vector<StepParams> table;
@@ -331,7 +383,6 @@ int Batch::prepare()
                 return fail(SPH_E_LIMIT, "batch: %llu grid cells exceed the 2^31 limit", (unsigned long long)base);
             table.push_back(b.P);
         }
-        drop_graph();
         stat_ok = false;
         if ((rc = w.reserve_cells(base)) || (rc = w.set_scenes(table, stream)))
             return rc;
@@ -503,10 +554,33 @@ int Batch::auto_grid()
     return SPH_OK;
 }
 
+// Every argument and grid size of a step's launches: a graph made with the
+// same ones is the step's graph, whatever the scenes hold (their constants are
+// read from device memory).  Capturing and instantiating one takes 0.3 ms.
+Batch::GraphKey Batch::graph_key() const
+{
+    const ParticleArrays a = w.particles();
+    const CellArrays c = w.cells();
+    const SceneSet S = w.scene_set();
+    const PartPlan p = w.part_plan();
+    const NeighborLists l = w.lists();
+    auto at = [](const void *q) { return (uint64_t)(uintptr_t)q; };
+    return GraphKey{at(a.posA),    at(a.velA),   at(a.posB),      at(a.velB),      at(a.cellcA),   at(a.rankA),
+                    at(a.cellcB),  at(a.perm),   at(a.rhoB),      at(a.posR),      at(a.velR),     at(c.counts),
+                    at(c.cstart),  at(c.partials), at(c.big),     at(c.unordered), at(S.params),   at(S.tasks),
+                    at(p.nparts),  at(p.off),    at(p.scan_partials), at(p.measure), at(p.total),  at(p.tasks),
+                    at(p.queue),   at(p.buf),    at(p.done),      at(p.walk),      at(p.own),      at(l.list),
+                    at(l.count),   at(w.force.ptr), c.big_cap,    c.ncells_padded, S.nwaves,       S.staged,
+                    p.padded,      p.nscenes,    p.cap,           l.stride,        (uint64_t)w.stencil_block,
+                    keep_force};
+}
+
 int Batch::capture()
 {
-    if (exec)
+    const GraphKey key = graph_key();
+    if (exec && key == captured)
         return SPH_OK;
+    drop_graph();
     hipError_t e = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess)
         return hip_fail(e, "hipStreamBeginCapture");
@@ -518,6 +592,7 @@ int Batch::capture()
         drop_graph();
         return hip_fail(e, "graph capture");
     }
+    captured = key;
     return SPH_OK;
 }
 
@@ -686,49 +761,26 @@ int Batch::download(uint32_t s, float *pos, float *vel, float *rho, float *press
     if (!scenes[s].uploaded)
         return fail(SPH_E_STATE, "download: scene not uploaded");
     const uint32_t n = scenes[s].desc.n, p0 = scenes[s].P.p_begin;
-    ParticleArrays a = w.particles();
-    std::vector<float4> p4, v4, r4;
-    std::vector<float> r;
-    hipError_t e = hipSuccess;
-    if (pos) {
-        p4.resize(n);
-        e = hipMemcpyAsync(p4.data(), a.posA + p0, sizeof(float4) * (size_t)n, hipMemcpyDeviceToHost, stream);
-    }
-    if (e == hipSuccess && (vel || ids)) {
-        v4.resize(n);
-        e = hipMemcpyAsync(v4.data(), a.velA + p0, sizeof(float4) * (size_t)n, hipMemcpyDeviceToHost, stream);
-    }
-    if (e == hipSuccess && rho) {
-        r.resize(n);
-        e = hipMemcpyAsync(r.data(), a.rhoB + p0, 4ull * n, hipMemcpyDeviceToHost, stream);
-    }
-    if (e == hipSuccess && pressure) {
-        r4.resize(n);
-        e = hipMemcpyAsync(r4.data(), a.velR + p0, sizeof(float4) * (size_t)n, hipMemcpyDeviceToHost, stream);
-    }
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(stream);
+    // laid out as the caller's arrays in the neighbour lists (scratch
+    // between steps), and copied from there
+    float *raw = (float *)w.nlist.ptr;
+    HostSpan out[5];
+    int k = 0;
+    auto span = [&](void *dst, size_t per) -> float * {
+        if (!dst)
+            return nullptr;
+        float *at = raw;
+        raw += per * n;
+        out[k++] = HostSpan{dst, at, 4 * per * n};
+        return at;
+    };
+    float *d_pos = span(pos, 3), *d_vel = span(vel, 3), *d_rho = span(rho, 1), *d_prs = span(pressure, 1);
+    uint32_t *d_ids = (uint32_t *)span(ids, 1);
+    launch_store_state(stream, w.particles(), p0, n, d_pos, d_vel, d_rho, d_prs, d_ids);
+    hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return hip_fail(e, "download");
-    for (uint32_t i = 0; i < n; ++i) {
-        if (pos) {
-            pos[3 * (size_t)i] = p4[i].x;
-            pos[3 * (size_t)i + 1] = p4[i].y;
-            pos[3 * (size_t)i + 2] = p4[i].z;
-        }
-        if (vel) {
-            vel[3 * (size_t)i] = v4[i].x;
-            vel[3 * (size_t)i + 1] = v4[i].y;
-            vel[3 * (size_t)i + 2] = v4[i].z;
-        }
-        if (ids)
-            std::memcpy(&ids[i], &v4[i].w, 4);
-        if (rho)
-            rho[i] = r[i];
-        if (pressure)
-            pressure[i] = r4[i].w;
-    }
-    return SPH_OK;
+    return copy_to_host(stream, out, k, stage);
 }
 
 int Batch::download_particles(uint32_t s, sph_particle_v1 *out, float *transforms)
@@ -743,14 +795,8 @@ int Batch::download_particles(uint32_t s, sph_particle_v1 *out, float *transform
         return rc;
     launch_pack_state(stream, w.particles(), keep_force ? (const float4 *)w.force.ptr : nullptr, p0, n,
                       scenes[s].P.xf_scale, aos.ptr, transforms ? (float *)xf.ptr : nullptr);
-    hipError_t e = hipMemcpyAsync(out, aos.ptr, sizeof(sph_particle_v1) * (size_t)n, hipMemcpyDeviceToHost, stream);
-    if (e == hipSuccess && transforms)
-        e = hipMemcpyAsync(transforms, xf.ptr, 64ull * n, hipMemcpyDeviceToHost, stream);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(stream);
-    if (e != hipSuccess)
-        return hip_fail(e, "download_particles");
-    return SPH_OK;
+    const HostSpan spans[2] = {{out, aos.ptr, sizeof(sph_particle_v1) * (size_t)n}, {transforms, xf.ptr, 64ull * n}};
+    return copy_to_host(stream, spans, transforms ? 2 : 1, stage);
 }
 
 int Batch::profile(int nsteps, double *ms, int max_k, int *nk, char *names_buf, size_t names_cap)

@@ -189,7 +189,15 @@ inline uint32_t blocks_for(uint32_t n, int block = kBlock) { return (n + block -
 
 void launch_fill_u32(hipStream_t st, uint32_t *p, uint32_t value, size_t n);
 void launch_unpack_aos(hipStream_t st, const void *aos, uint32_t n, float4 *posA, float4 *velA);
+// Bounds of the finite positions as order-preserving ints (x, y, z minima,
+// then maxima; INT32_MAX / INT32_MIN where there is none).
 void launch_bbox(hipStream_t st, const float4 *pos, uint32_t n, int32_t *bbox6);
+// Upload and download of a scene's slots [first, first + n) from and to
+// device arrays laid out as the caller's (see the kernels).
+void launch_load_state(hipStream_t st, const float *pos3, const float *vel3, const ParticleArrays &a, float4 *force,
+                       uint32_t first, uint32_t n, int32_t *bbox6);
+void launch_store_state(hipStream_t st, const ParticleArrays &a, uint32_t first, uint32_t n, float *pos3, float *vel3,
+                        float *rho, float *pressure, uint32_t *ids);
 void launch_init_keys(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S);
 // Scan of the cell counts; also lists the cells above kSmallCell in c.big.
 // clear_counts: zero the counts (else the scatter counts them back down).

@@ -157,25 +157,23 @@ __device__ inline int32_t ordered_int(float f)
     return i >= 0 ? i : (int32_t)(i ^ 0x7FFFFFFF);
 }
 
-// Bounding box of finite positions: bbox6 = {min x,y,z, max x,y,z} as
-// ordered ints (pre-filled with INT_MAX / INT_MIN).
-__global__ void k_bbox(const float4 *__restrict__ pos, uint32_t n, int32_t *__restrict__ bbox6)
+__device__ inline void widen(int32_t (&v)[6], float x, float y, float z)
 {
-    __shared__ int32_t red[6][kBlock / 64];
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    int32_t v[6] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN, INT32_MIN};
-    if (i < n) {
-        float4 p = pos[i];
-        float c[3] = {p.x, p.y, p.z};
+    const float c[3] = {x, y, z};
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            if (c[k] - c[k] == 0.0f) {  // finite
-                int32_t o = ordered_int(c[k]);
-                v[k] = o;
-                v[k + 3] = o;
-            }
+    for (int k = 0; k < 3; ++k) {
+        if (c[k] - c[k] == 0.0f) {  // finite
+            const int32_t o = ordered_int(c[k]);
+            v[k] = min(v[k], o);
+            v[k + 3] = max(v[k + 3], o);
         }
     }
+}
+
+// Joins every thread's bounds into bbox6: six atomics a block.
+__device__ inline void join_bounds(const int32_t (&v)[6], int32_t *__restrict__ bbox6)
+{
+    __shared__ int32_t red[6][kBlock / 64];
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
         int32_t x = v[k];
@@ -199,9 +197,107 @@ __global__ void k_bbox(const float4 *__restrict__ pos, uint32_t n, int32_t *__re
     }
 }
 
+// Bounding box of finite positions: bbox6 = {min x,y,z, max x,y,z} as
+// ordered ints.  kBoundsBlocks blocks at most: what the pass costs is its
+// atomics on six addresses (one block per 256 particles took 26 us at 262
+// thousand of them).
+constexpr uint32_t kBoundsBlocks = 128;
+
+__global__ void k_bbox_init(int32_t *__restrict__ bbox6)
+{
+    if (threadIdx.x < 6u)
+        bbox6[threadIdx.x] = threadIdx.x < 3u ? INT32_MAX : INT32_MIN;
+}
+
+__global__ __launch_bounds__(kBlock) void k_bbox(const float4 *__restrict__ pos, uint32_t n,
+                                                int32_t *__restrict__ bbox6)
+{
+    int32_t v[6] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN, INT32_MIN};
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const float4 p = pos[i];
+        widen(v, p.x, p.y, p.z);
+    }
+    join_bounds(v, bbox6);
+}
+
 void launch_bbox(hipStream_t st, const float4 *pos, uint32_t n, int32_t *bbox6)
 {
-    hipLaunchKernelGGL(k_bbox, dim3(blocks_for(n)), dim3(kBlock), 0, st, pos, n, bbox6);
+    hipLaunchKernelGGL(k_bbox_init, dim3(1), dim3(64), 0, st, bbox6);
+    hipLaunchKernelGGL(k_bbox, dim3(std::min(blocks_for(n), kBoundsBlocks)), dim3(kBlock), 0, st, pos, n, bbox6);
+}
+
+// A scene's state from the caller's arrays (three floats a particle; vel may
+// be null) into slots [first, first + n): ids in order, everything a step
+// has not yet computed cleared, and the bounds of the finite positions.
+__global__ __launch_bounds__(kBlock) void k_load_state(const float *__restrict__ pos3, const float *__restrict__ vel3,
+                                                      ParticleArrays a, float4 *__restrict__ force, uint32_t first,
+                                                      uint32_t n, int32_t *__restrict__ bbox6)
+{
+    int32_t v[6] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN, INT32_MIN};
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const size_t k = 3 * (size_t)i, s = (size_t)first + i;
+        const float x = pos3[k], y = pos3[k + 1], z = pos3[k + 2];
+        widen(v, x, y, z);
+        a.posA[s] = make_float4(x, y, z, 0.0f);
+        a.velA[s] = vel3 ? make_float4(vel3[k], vel3[k + 1], vel3[k + 2], __uint_as_float(i))
+                         : make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(i));
+        a.rhoB[s] = 0.0f;
+        a.posB[s] = zero;
+        a.posR[s] = zero;
+        a.velR[s] = zero;
+        if (force)
+            force[s] = zero;
+    }
+    join_bounds(v, bbox6);
+}
+
+void launch_load_state(hipStream_t st, const float *pos3, const float *vel3, const ParticleArrays &a, float4 *force,
+                       uint32_t first, uint32_t n, int32_t *bbox6)
+{
+    hipLaunchKernelGGL(k_bbox_init, dim3(1), dim3(64), 0, st, bbox6);
+    hipLaunchKernelGGL(k_load_state, dim3(std::min(blocks_for(n), 4u * kBoundsBlocks)), dim3(kBlock), 0, st, pos3,
+                       vel3, a, force, first, n, bbox6);
+}
+
+// The downloaded quantities of slots [first, first + n), each an array of its
+// own (null: not wanted): positions, velocities, densities, pressures, ids.
+__global__ __launch_bounds__(kBlock) void k_store_state(ParticleArrays a, uint32_t first, uint32_t n,
+                                                       float *__restrict__ pos3, float *__restrict__ vel3,
+                                                       float *__restrict__ rho, float *__restrict__ pressure,
+                                                       uint32_t *__restrict__ ids)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n)
+        return;
+    const size_t k = 3 * (size_t)i, s = (size_t)first + i;
+    if (pos3) {
+        const float4 x = a.posA[s];
+        pos3[k] = x.x;
+        pos3[k + 1] = x.y;
+        pos3[k + 2] = x.z;
+    }
+    if (vel3 || ids) {
+        const float4 v = a.velA[s];
+        if (vel3) {
+            vel3[k] = v.x;
+            vel3[k + 1] = v.y;
+            vel3[k + 2] = v.z;
+        }
+        if (ids)
+            ids[i] = __float_as_uint(v.w);
+    }
+    if (rho)
+        rho[i] = a.rhoB[s];
+    if (pressure)
+        pressure[i] = a.velR[s].w;
+}
+
+void launch_store_state(hipStream_t st, const ParticleArrays &a, uint32_t first, uint32_t n, float *pos3, float *vel3,
+                        float *rho, float *pressure, uint32_t *ids)
+{
+    hipLaunchKernelGGL(k_store_state, dim3(blocks_for(n)), dim3(kBlock), 0, st, a, first, n, pos3, vel3, rho, pressure,
+                       ids);
 }
 
 // Cell key and bucket of the positions in posA, counted into their cells

@@ -132,8 +132,6 @@ __global__ void k_single_scene_tasks(WaveTask *__restrict__ tasks, uint32_t nwav
         tasks[w] = WaveTask{0u, 64u * w};
 }
 
-double from_ordered(int32_t o) { return (double)__builtin_bit_cast(float, o >= 0 ? o : (int32_t)(o ^ 0x7FFFFFFF)); }
-
 // Device address of this device's scratch array, looked up on first use.
 int scratch_of_current_device(unsigned char **out)
 {
@@ -206,8 +204,6 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     // the bounding box borrows the first words of counts16, which is
     // cleared again before the output sort uses it
     int32_t *bbox = (int32_t *)at(L.counts16);
-    launch_fill_u32(st, (uint32_t *)bbox, 0x7FFFFFFFu, 3);
-    launch_fill_u32(st, (uint32_t *)bbox + 3, 0x80000000u, 3);
     launch_bbox(st, a.posA, n, bbox);
     int32_t bb[6];
     e = hipMemcpyAsync(bb, bbox, sizeof bb, hipMemcpyDeviceToHost, st);

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -42,6 +44,43 @@ struct DevBuf {
     ~DevBuf() { release(); }
 };
 
+// Pinned host memory that transfers to and from the caller's (pageable)
+// arrays pass through.  Small ones: an object's own, at most kPiece, kept with
+// it (256 kB straight from or to pageable memory takes 110 us in one copy,
+// 145 us in five; through pinned memory 18 us).  Large downloads: one for the
+// process, made for the first object that needs it, shared by all that do,
+// given back with the last of them.
+constexpr size_t kPiece = 2ull << 20;
+struct Staging;
+struct HostStage {
+    unsigned char *ptr = nullptr;
+    size_t bytes = 0;
+    std::shared_ptr<Staging> large;
+    HostStage() = default;
+    HostStage(const HostStage &) = delete;
+    HostStage &operator=(const HostStage &) = delete;
+    ~HostStage();
+    // at least `want` bytes (up to kPiece), or null: more, or none to be had
+    unsigned char *small(size_t want);
+};
+
+struct HostSpan {
+    void *dst;
+    const void *src;  // device
+    size_t bytes;
+};
+
+// Copies the spans to pageable host memory, after the work enqueued on st;
+// returns when they are there.  Large copies go through the shared memory in
+// pieces, several threads at a time: copying out of pinned memory (and
+// having the system provide the destination's pages) takes one thread several
+// times as long as the device needs to deliver (1M particles, 32 MB to fresh
+// pages: 13 ms directly, 3 this way).
+int copy_to_host(hipStream_t st, const HostSpan *spans, int count, HostStage &stage);
+
+// Inverse of the device's order-preserving map of floats to ints.
+inline double from_ordered(int32_t o) { return (double)__builtin_bit_cast(float, o >= 0 ? o : (int32_t)(o ^ 0x7FFFFFFF)); }
+
 // All device arrays of one particle set (see sph_kernels.h for the layout).
 struct Workspace {
     DevBuf posA, velA, posB, velB, cellcA, rankA, cellcB, perm, rhoB, posR, velR;
@@ -63,6 +102,7 @@ struct Workspace {
     uint32_t nwaves = 0;
     uint32_t nscenes = 0;
     bool staged = false;  // SceneSet::staged of the current scene set
+    std::vector<WaveTask> host_tasks;  // what `tasks` holds
     uint32_t part_cap = 0;  // part-task capacity of the current scene set
     int stencil_block = kStencilBlock;  // threads per block of the density and force passes
     int reserve_particles(uint32_t n);

@@ -15,6 +15,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../../include/sph_hip.h"
@@ -240,6 +241,174 @@ void DevBuf::release()
     bytes = 0;
 }
 
+// ------------------------------------------------------------ transfers
+
+namespace {
+constexpr int kCopiers = 8;
+}  // namespace
+
+struct Staging {
+    std::mutex mu;
+    unsigned char *base = nullptr;  // kCopiers pieces
+    ~Staging()
+    {
+        if (base)
+            (void)hipHostFree(base);
+    }
+};
+
+namespace {
+
+hipError_t pinned_alloc(void **p, size_t bytes)
+{
+    // another thread may be capturing a graph of its own meanwhile
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipHostMalloc(p, bytes, hipHostMallocPortable);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
+// null: no pinned memory to be had
+std::shared_ptr<Staging> staging()
+{
+    static std::mutex mu;
+    static std::weak_ptr<Staging> shared;
+    try {
+        std::lock_guard<std::mutex> lock(mu);
+        std::shared_ptr<Staging> s = shared.lock();
+        if (!s) {
+            s = std::make_shared<Staging>();
+            if (pinned_alloc((void **)&s->base, kPiece * kCopiers) != hipSuccess)
+                return nullptr;
+            shared = s;
+        }
+        return s;
+    } catch (const std::exception &) {
+        return nullptr;
+    }
+}
+
+// Copier t of a download: every kCopiers-th piece, through its own part of
+// the staging memory, while the copies of the others run.
+hipError_t copy_pieces(int device, hipStream_t st, const HostSpan *spans, int count, int t, unsigned char *buf)
+{
+    hipEvent_t done = nullptr;
+    hipError_t err = hipSetDevice(device);
+    if (err == hipSuccess)
+        err = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+    size_t piece = 0;
+    for (int k = 0; k < count; ++k)
+        for (size_t at = 0; at < spans[k].bytes && err == hipSuccess; at += kPiece, ++piece) {
+            if (piece % kCopiers != (size_t)t)
+                continue;
+            const size_t bytes = std::min(kPiece, spans[k].bytes - at);
+            err = hipMemcpyAsync(buf, (const char *)spans[k].src + at, bytes, hipMemcpyDeviceToHost, st);
+            if (err == hipSuccess)
+                err = hipEventRecord(done, st);
+            if (err == hipSuccess)
+                err = hipEventSynchronize(done);
+            if (err == hipSuccess)
+                std::memcpy((char *)spans[k].dst + at, buf, bytes);
+        }
+    if (done)
+        (void)hipEventDestroy(done);
+    return err;
+}
+
+}  // namespace
+
+HostStage::~HostStage()
+{
+    if (ptr)
+        (void)hipHostFree(ptr);
+}
+
+unsigned char *HostStage::small(size_t want)
+{
+    if (want > kPiece)
+        return nullptr;
+    if (want > bytes) {
+        size_t room = 64ull << 10;
+        while (room < want)
+            room *= 2;
+        if (ptr)
+            (void)hipHostFree(ptr);
+        ptr = nullptr;
+        bytes = pinned_alloc((void **)&ptr, room) == hipSuccess ? room : 0;
+    }
+    return ptr;
+}
+
+int copy_to_host(hipStream_t st, const HostSpan *spans, int count, HostStage &stage)
+{
+    size_t total = 0, pieces = 0;
+    for (int k = 0; k < count; ++k) {
+        total += spans[k].bytes;
+        pieces += (spans[k].bytes + kPiece - 1) / kPiece;
+    }
+    hipError_t e = hipSuccess;
+    if (unsigned char *buf = stage.small(total)) {
+        size_t at = 0;
+        for (int k = 0, next; k < count && e == hipSuccess; k = next) {  // neighbours on the device: one copy
+            size_t run = spans[k].bytes;
+            for (next = k + 1; next < count && spans[next].src == (const char *)spans[k].src + run; ++next)
+                run += spans[next].bytes;
+            e = hipMemcpyAsync(buf + at, spans[k].src, run, hipMemcpyDeviceToHost, st);
+            at += run;
+        }
+        const hipError_t w = hipStreamSynchronize(st);
+        e = e != hipSuccess ? e : w;
+        if (e != hipSuccess)
+            return hip_fail(e, "download");
+        for (int k = 0; k < count; buf += spans[k].bytes, ++k)
+            std::memcpy(spans[k].dst, buf, spans[k].bytes);
+        return SPH_OK;
+    }
+    if (!stage.large && total > kPiece)
+        stage.large = staging();
+    if (!stage.large || total <= kPiece) {
+        for (int k = 0; k < count && e == hipSuccess; ++k)
+            e = hipMemcpyAsync(spans[k].dst, spans[k].src, spans[k].bytes, hipMemcpyDeviceToHost, st);
+        const hipError_t w = hipStreamSynchronize(st);
+        e = e != hipSuccess ? e : w;
+        return e == hipSuccess ? SPH_OK : hip_fail(e, "download");
+    }
+    Staging &ring = *stage.large;
+    int device = 0;
+    e = hipStreamSynchronize(st);  // not with the staging memory held
+    if (e == hipSuccess)
+        e = hipGetDevice(&device);
+    if (e != hipSuccess)
+        return hip_fail(e, "download");
+    std::lock_guard<std::mutex> lock(ring.mu);
+    hipError_t failed[kCopiers] = {};
+    std::thread threads[kCopiers];
+    const int workers = (int)std::min<size_t>(kCopiers, pieces);
+    auto copier = [&](int t) { failed[t] = copy_pieces(device, st, spans, count, t, ring.base + kPiece * (size_t)t); };
+    for (int t = 1; t < workers; ++t) {
+        try {
+            threads[t] = std::thread(copier, t);
+        } catch (const std::exception &) {  // no thread to be had: this one does its share below
+        }
+    }
+    copier(0);
+    for (int t = 1; t < workers; ++t) {
+        if (threads[t].joinable())
+            threads[t].join();
+        else
+            copier(t);
+    }
+    e = hipStreamSynchronize(st);
+    for (hipError_t f : failed)
+        e = e != hipSuccess ? e : f;
+    return e == hipSuccess ? SPH_OK : hip_fail(e, "download");
+}
+
 int Workspace::reserve_particles(uint32_t n)
 {
     int rc;
@@ -287,9 +456,11 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
         for (uint32_t f = scenes[k].p_begin; f < scenes[k].p_end; f += 64u)
             t.push_back(WaveTask{k, f});
     int rc;
+    const void *had_tasks = tasks.ptr;
     if ((rc = params.reserve(sizeof(StepParams) * std::max<size_t>(scenes.size(), 1))) ||
         (rc = tasks.reserve(sizeof(WaveTask) * std::max<size_t>(t.size(), 1))))
         return rc;
+    const bool fresh_tasks = tasks.ptr != had_tasks;
     const size_t nw = std::max<size_t>(t.size(), 1);
     size_t nslots = 0;
     for (const StepParams &sp : scenes)
@@ -322,16 +493,21 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
     if (!scenes.empty())
         e = hipMemcpyAsync(params.ptr, scenes.data(), sizeof(StepParams) * scenes.size(),
                            hipMemcpyHostToDevice, st);
-    if (e == hipSuccess && !t.empty())
+    const bool same = !fresh_tasks && t.size() == host_tasks.size() &&
+                      std::memcmp(t.data(), host_tasks.data(), sizeof(WaveTask) * t.size()) == 0;
+    if (e == hipSuccess && !t.empty() && !same)
         e = hipMemcpyAsync(tasks.ptr, t.data(), sizeof(WaveTask) * t.size(), hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
         e = hipStreamSynchronize(st);  // the host vectors go out of scope
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        host_tasks.clear();
         return hip_fail(e, "scene table upload");
+    }
+    host_tasks = std::move(t);
     staged = false;
     for (const StepParams &sp : scenes)
         staged = staged || stageable(sp);
-    nwaves = (uint32_t)t.size();
+    nwaves = (uint32_t)host_tasks.size();
     nscenes = (uint32_t)scenes.size();
     part_cap = (uint32_t)cap;
     return SPH_OK;
@@ -417,6 +593,7 @@ void Workspace::release_all()
                       &ppartials, &pmeasure, &ptotal, &ptasks, &pqueue, &pbuf, &pdone, &pwalk, &pown,
                       &nlist, &ncount, &unordered})
         b->release();
+    host_tasks.clear();
     ncells_padded = 0;
     big_cap = 0;
     nwaves = 0;
@@ -462,6 +639,7 @@ struct Stateless {
     hipStream_t stream = nullptr;
     Workspace w;
     DevBuf aos_in, aos_out, xf, bbox, counts16, cstart16, partials16, perm16;
+    HostStage stage;
 };
 
 Stateless &stateless()
@@ -484,8 +662,6 @@ int stateless_init(Stateless &S)
     return SPH_OK;
 }
 
-double from_ordered(int32_t o) { return (double)__builtin_bit_cast(float, o >= 0 ? o : (int32_t)(o ^ 0x7FFFFFFF)); }
-
 // Uploads AoS particles, builds the grid from their bounding box, computes
 // keys and runs the scan/scatter/reorder/density passes.  Leaves the
 // workspace ready for the force pass.
@@ -499,17 +675,22 @@ int stateless_prepare(Stateless &S, const sph_particle_v1 *particles, uint32_t n
         (rc = S.bbox.reserve(64)))
         return rc;
     hipStream_t st = S.stream;
-    hipError_t e = hipMemcpyAsync(S.aos_in.ptr, particles, sizeof(sph_particle_v1) * (size_t)n,
-                                  hipMemcpyHostToDevice, st);
+    const size_t bytes = sizeof(sph_particle_v1) * (size_t)n;
+    const void *src = particles;
+    unsigned char *pinned = S.stage.small(bytes + 64);
+    if (pinned) {
+        std::memcpy(pinned + 64, particles, bytes);
+        src = pinned + 64;
+    }
+    hipError_t e = hipMemcpyAsync(S.aos_in.ptr, src, bytes, hipMemcpyHostToDevice, st);
     if (e != hipSuccess)
         return hip_fail(e, "upload particles");
     ParticleArrays a = w.particles();
     launch_unpack_aos(st, S.aos_in.ptr, n, a.posA, a.velA);
-    launch_fill_u32(st, (uint32_t *)S.bbox.ptr, 0x7FFFFFFFu, 3);      // min: INT32_MAX
-    launch_fill_u32(st, (uint32_t *)S.bbox.ptr + 3, 0x80000000u, 3);  // max: INT32_MIN
     launch_bbox(st, a.posA, n, (int32_t *)S.bbox.ptr);
-    int32_t bb[6];
-    e = hipMemcpyAsync(bb, S.bbox.ptr, sizeof bb, hipMemcpyDeviceToHost, st);
+    int32_t pageable[6];
+    int32_t *bb = pinned ? (int32_t *)pinned : pageable;
+    e = hipMemcpyAsync(bb, S.bbox.ptr, sizeof pageable, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess)
         e = hipStreamSynchronize(st);
     if (e != hipSuccess)
@@ -616,15 +797,9 @@ int update_particles(sph_particle_v1 *particles, float *transforms, size_t n_,
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
         return hip_fail(e, "kernel launch");
-    e = hipMemcpyAsync(particles, S.aos_out.ptr, sizeof(sph_particle_v1) * (size_t)n,
-                       hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess && transforms)
-        e = hipMemcpyAsync(transforms, S.xf.ptr, 64ull * n, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess)
-        e = hipStreamSynchronize(st);
-    if (e != hipSuccess)
-        return hip_fail(e, "download particles");
-    return SPH_OK;
+    const HostSpan out[2] = {{particles, S.aos_out.ptr, sizeof(sph_particle_v1) * (size_t)n},
+                             {transforms, S.xf.ptr, 64ull * n}};
+    return copy_to_host(st, out, transforms ? 2 : 1, S.stage);
 }
 
 int neighbors(const sph_particle_v1 *particles, size_t n_, const sph_settings_v1 *settings,
