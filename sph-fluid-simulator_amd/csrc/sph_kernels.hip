@@ -684,7 +684,20 @@ __device__ inline float dist2_ref(float4 pi, float4 q, float &dx, float &dy, flo
     return dx * dx + dy * dy + dz * dz;
 }
 
-// r = sqrt(x) correctly rounded and y = 1 / sqrt(x) within an ulp, for
+// Correctly rounded sqrt for x >= 2^-96 (any d2 a neighbour pair can have
+// short of coincident points; x = 0 also comes out exact): v_sqrt_f32 is
+// within 1 ulp, and the neighbouring value whose residual x - s * s' changes
+// sign is the correctly rounded root.
+__device__ inline float sqrt_rn(float x)
+{
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float down = __uint_as_float(__float_as_uint(s) - 1u);
+    const float up = __uint_as_float(__float_as_uint(s) + 1u);
+    const float below = fmaf(-down, s, x) <= 0.0f ? down : s;
+    return fmaf(-up, s, x) > 0.0f ? up : below;
+}
+
+// The same root r and y = 1 / sqrt(x) within an ulp, for
 // x >= 2^-96 (any d2 a neighbour pair can have short of coincident points,
 // where both come out NaN / inf as the reference's division by r = 0 does):
 // one Newton step on v_rsq_f32, whose result equals the rounded root for
@@ -729,12 +742,11 @@ __device__ inline RefCell ref_cell(float4 p, const StepParams &P)
 // The (2R + 1)^2 rows of the (2R + 1)^3 grid-cell stencil around packed
 // cell cc (R = P.reach), clipped to the grid: for row (y, z) the x-run of
 // cells [gx - R, gx + R] is one contiguous range [b, e) of the cell-ordered
-// arrays.  Calls row(b, e) for each row, z-major then y, both ascending, and
-// layer() after the last row of each z.
+// arrays.  Calls row(b, e) for each row, z-major then y, both ascending.
 // The bounds of the next row are loaded while the current row runs.
-template <class Row, class Layer>
+template <class Row>
 __device__ inline void for_each_row(const uint32_t *__restrict__ cstart, uint32_t cc,
-                                    const StepParams &P, Row row, Layer layer)
+                                    const StepParams &P, Row row)
 {
     const int gx = cell_x(cc), gy = cell_y(cc), gz = cell_z(cc), R = P.reach;
     const int x0 = max(gx - R, 0), x1 = min(gx + R, P.nx - 1);
@@ -748,8 +760,7 @@ __device__ inline void for_each_row(const uint32_t *__restrict__ cstart, uint32_
     uint32_t r0 = base(y, z);
     uint32_t b = cstart[r0 + (uint32_t)x0], e = cstart[r0 + (uint32_t)x1 + 1u];
     for (int k = 0; k < nrows; ++k) {
-        const bool last = ++y > y1;
-        if (last) {
+        if (++y > y1) {
             y = y0;
             ++z;
         }
@@ -760,8 +771,6 @@ __device__ inline void for_each_row(const uint32_t *__restrict__ cstart, uint32_
             en = cstart[r0 + (uint32_t)x1 + 1u];
         }
         row(b, e);
-        if (last)
-            layer();
         b = bn;
         e = en;
     }
@@ -811,11 +820,11 @@ __device__ inline float trim_gap(int d, float f)
 // gaps alone reach rho, else its x-run is cut to the cells within the
 // remaining chord.  Calls row(b, e) for every non-empty row, in
 // for_each_row's order, so the passing candidates come in the same order
-// as on the whole stencil, and layer() after each z.  The bounds of the next row are loaded while the
+// as on the whole stencil.  The bounds of the next row are loaded while the
 // current row runs.
-template <class Row, class Layer>
+template <class Row>
 __device__ inline void for_each_cut_row(const uint32_t *__restrict__ cstart, uint32_t cc, const LaneTrim &T,
-                                        const StepParams &P, Row row, Layer layer)
+                                        const StepParams &P, Row row)
 {
     const int gx = cell_x(cc), gy = cell_y(cc), gz = cell_z(cc), R = P.reach;
     const int y0 = max(gy - R, 0), y1 = min(gy + R, P.ny - 1);
@@ -840,8 +849,7 @@ __device__ inline void for_each_cut_row(const uint32_t *__restrict__ cstart, uin
     uint32_t b, e;
     bounds(y, z, b, e);
     for (int k = 0; k < nrows; ++k) {
-        const bool last = ++y > y1;
-        if (last) {
+        if (++y > y1) {
             y = y0;
             ++z;
         }
@@ -850,8 +858,6 @@ __device__ inline void for_each_cut_row(const uint32_t *__restrict__ cstart, uin
             bounds(y, z, bn, en);
         if (b < e)
             row(b, e);
-        if (last)
-            layer();
         b = bn;
         e = en;
     }
@@ -859,9 +865,9 @@ __device__ inline void for_each_cut_row(const uint32_t *__restrict__ cstart, uin
 
 // for_each_row restricted to the positions [lo, hi) of the lane's own
 // candidate sequence (its rows in order, slots ascending).
-template <class Row, class Layer>
+template <class Row>
 __device__ inline void for_each_row_span(const uint32_t *__restrict__ cstart, uint32_t cc, const StepParams &P,
-                                         uint32_t lo, uint32_t hi, Row row, Layer layer)
+                                         uint32_t lo, uint32_t hi, Row row)
 {
     uint32_t off = 0;
     for_each_row(cstart, cc, P, [&](uint32_t b, uint32_t e) {
@@ -870,7 +876,7 @@ __device__ inline void for_each_row_span(const uint32_t *__restrict__ cstart, ui
         if (s0 < s1)
             row(b + (s0 - off), b + (s1 - off));
         off += len;
-    }, layer);
+    });
 }
 
 __device__ inline int wave_min_i(int x)
@@ -1249,16 +1255,22 @@ constexpr uint32_t kStageCap = 1296;  // candidates, every row rounded up to a m
 constexpr uint32_t kStageSegs = 7;    // runs of lanes in one x-row of cells, 3 rows each per layer
 constexpr uint32_t kStageWords = 3;   // a lane's row: at most 32 candidates per mask word
                                       // (a lattice of spacing h / 2.1 can line up 66)
+// Room for the terms of one lane's neighbours in layers 1 and 2, the former
+// from the first row up, the latter from the last row down; each side's next
+// term is written wherever it will come to lie, so two rows more than terms.
+// A lattice of spacing h / 2 has 32 at most.  (Six blocks fit a CU with this;
+// with 52 rows, five: planning 64 scenes took 214 us instead of 195.)
+constexpr uint32_t kStageTerms = 34;
 struct StagedLayer {
     uint32_t shift[3 * kStageSegs];  // row -> LDS index less slot
     uint32_t x0[kStageSegs], x1[kStageSegs], yz[kStageSegs];
     uint32_t total, fits;
-    uint32_t own[64], listed[64];
-    float sum[64];
+    uint32_t own[64], listed[64], counted[64];
 };
 struct Stage {
     alignas(16) float x[kStageCap + 4], y[kStageCap + 4], z[kStageCap + 4];  // four are read ahead
     StagedLayer layer[3];
+    float term[kStageTerms][64];
 };
 
 // *src of each lane into dst + lane (dst wave-uniform), without registers
@@ -1285,13 +1297,18 @@ struct __attribute__((packed, aligned(4))) Bounds4 {
 // Walked from global memory the same pass is a chain of some fifty dependent
 // round trips, each also waiting for the list entries stored before it; here
 // it is three (cells, bounds, records), and a third as many candidates.
-// Sums are added per layer and lists written layer after layer, in the order
-// of every other walk, so both are the per-lane walk's bit for bit.
+// The waves only find the neighbours of their layers; their terms are then
+// added in the order of every other walk, and listed in it, so both are the
+// per-lane walk's bit for bit: the first wave adds its own, then those the
+// others left in LDS.
 // Measured, planning and density of a step together, walked from memory and
-// staged: 3,375 particles 56 and 18 us, 78 thousand 89 and 21 us, 64 scenes of
-// 1.06 million in all 263 and 153 us, a million 254 and 129 us.  What bounds
-// it at a million is the arithmetic (75 M vector instructions in 117 us);
-// below some thousand tasks, the latency of one wave.
+// staged: 8,000 particles 65 and 23 us, 64 scenes of 1.06 million in all 263
+// and 195 us.  What bounds those is the arithmetic (111 M vector
+// instructions in all; finding neighbours and adding their terms in order
+// are about equal shares); below some thousand tasks, the latency of one wave.
+// (Adding each layer's terms in its own wave takes 19 and 151 us, but then
+// the sums are not the per-lane walk's, and over a run of steps the particles
+// that meet a wall bounce a step apart.)
 //
 // All other tasks get a walk length (union count, or the largest own
 // stencil weighted), which splits them into parts, and are left to
@@ -1435,8 +1452,13 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
         if (__builtin_amdgcn_readfirstlane(layers[0].fits & layers[1].fits & layers[2].fits) != 0u &&
             longest <= kShortWalk) {
             const float h2 = in_vgpr(P.h2);
+            const float mp6 = P.mp6;
             float acc = 0.0f;
             uint32_t mask[3][kStageWords];
+            const int term0 = (lz == 2 ? (int)kStageTerms - 1 : 0) * 64 + (int)lane, next_term = lz == 2 ? -64 : 64;
+            const int term_lo = (lz == 2 ? 3 : 0) * 64 + (int)lane, term_hi = term_lo + ((int)kStageTerms - 4) * 64;
+            int at_term = term0;
+            float *const terms = &stage.term[0][0];
             auto test = [&](float x, float y, float z) {
                 float dx, dy, dz;
                 return h2 - dist2_ref(pi, make_float4(x, y, z, 0.0f), dx, dy, dz);
@@ -1444,21 +1466,21 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
             // Four candidates at a time, the next four read meanwhile.  What
             // lies before the row's first and behind its last candidate is
             // the rest of its x-row (beyond the cut or the stencil: it never
-            // passes) or a sentinel.  The passing ones are collected in a
-            // mask, the first on top.
-            auto walk = [&](auto unit_tag) {
+            // passes) or a sentinel.  The passing ones (h2 - d2 > 0: exactly
+            // when d2 < h2, the float difference of unequal values being
+            // nonzero) are collected in a mask, the first on top.
+            auto walk = [&](auto first_tag, auto unit_tag) {
+                constexpr bool first = decltype(first_tag)::value;  // layer 0
 #pragma unroll
                 for (int r = 0; r < 3; ++r) {
 #pragma unroll
                     for (uint32_t c = 0; c < kStageWords; ++c) {
                         const uint32_t k0 = 32u * c, m = n[r] > k0 ? min(32u, n[r] - k0) : 0u;
-                        // only row 1 of layer 1 holds the particle itself
-                        const uint32_t self = r == 1 && lz == 1 ? s + G.shift[3u * seg + 1u] - l0[1] - k0 : ~0u;
                         const uint32_t from = l0[r] + k0;
+                        // only row 1 of layer 1 holds the particle itself
+                        const uint32_t self = r == 1 && lz == 1 ? s + G.shift[3u * seg + 1u] - from : ~0u;
                         uint32_t bits = 0;
-                        auto quads = [&](auto own_row) {
-                            if (m == 0u)
-                                return;
+                        if (m != 0u) {
                             float4 x = *reinterpret_cast<const float4 *>(&stage.x[from]);
                             float4 y = *reinterpret_cast<const float4 *>(&stage.y[from]);
                             float4 z = *reinterpret_cast<const float4 *>(&stage.z[from]);
@@ -1471,37 +1493,51 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
 #pragma unroll
                                 for (int i = 0; i < 4; ++i) {
                                     float t = positive<decltype(unit_tag)::value>(u[i]);
-                                    if (decltype(own_row)::value)
-                                        t = (k + (uint32_t)i != self) ? t : 0.0f;
-                                    acc = fmaf(t * t, t, acc);
-                                    bits = __builtin_amdgcn_alignbit(bits, 0u - __float_as_uint(t), 31u);  // << 1 | (t > 0)
+                                    if (!first && r == 1)
+                                        t = k + (uint32_t)i != self ? t : 0.0f;
+                                    const uint32_t hit = (0u - __float_as_uint(t)) >> 31;
+                                    bits = bits << 1 | hit;
+                                    if (first) {
+                                        acc = acc + mp6 * ((t * t) * t);
+                                    } else {  // kept if it is one, else overwritten by the next
+                                        terms[at_term] = t;
+                                        at_term += __mul24((int)hit, next_term);
+                                    }
                                 }
+                                // inside the array after four more, whatever it overwrites
+                                if (!first)
+                                    at_term = min(max(at_term, term_lo), term_hi);
                             }
-                        };
-                        if (r == 1 && lz == 1)
-                            quads(std::true_type{});
-                        else
-                            quads(std::false_type{});
-                        mask[r][c] = m ? bits << (32u - ((m + 3u) & ~3u)) : 0u;
+                            bits <<= 32u - ((m + 3u) & ~3u);
+                        }
+                        mask[r][c] = bits;
                     }
                 }
             };
-            if (P.h2 <= 1.0f)
-                walk(std::true_type{});
-            else
-                walk(std::false_type{});
-            uint32_t nn = 0, cnt = 0;
+            if (P.h2 <= 1.0f) {
+                if (lz == 0)
+                    walk(std::true_type{}, std::true_type{});
+                else
+                    walk(std::false_type{}, std::true_type{});
+            } else {
+                if (lz == 0)
+                    walk(std::true_type{}, std::false_type{});
+                else
+                    walk(std::false_type{}, std::false_type{});
+            }
+            uint32_t nn = 0;
 #pragma unroll
             for (int r = 0; r < 3; ++r)
 #pragma unroll
                 for (uint32_t c = 0; c < kStageWords; ++c)
                     nn += (uint32_t)__builtin_popcount(mask[r][c]);
-            if (any_slow) {
-                // the terms again, neighbours only, each with its m_ij
-                RefCell ci{0, 0, 0};
-                if (slow)
-                    ci = ref_cell(pi, P);
-                acc = 0.0f;
+            G.listed[lane] = nn;
+            __syncthreads();
+            const uint32_t n0 = layers[0].listed[lane], n1 = layers[1].listed[lane], n2 = layers[2].listed[lane];
+            const uint32_t all = n0 + n1 + n2;
+            const bool listing = !__any(all > kListMax), 
+                       parallel = !__any(n1 + n2 + 2u > kStageTerms || max(n1, n2) > kStageTerms - 4u);
+            auto neighbours = [&](auto visit) {
 #pragma unroll
                 for (int r = 0; r < 3; ++r)
 #pragma unroll
@@ -1509,55 +1545,99 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
                         for (uint32_t bits = mask[r][c]; bits != 0u;) {
                             const uint32_t k = (uint32_t)__builtin_clz(bits);
                             bits &= ~(0x80000000u >> k);
-                            const uint32_t at_k = l0[r] + 32u * c + k;
-                            const float t = test(stage.x[at_k], stage.y[at_k], stage.z[at_k]);
-                            int mult = 1;
-                            if (slow) {
-                                const float hash = pos[at_k - G.shift[3u * seg + (uint32_t)r]].w;
-                                mult = bucket_multiplicity(ci.x, ci.y, ci.z, __float_as_uint(hash) & 0xFFFFu);
-                            }
-                            acc = fmaf((float)mult * (t * t), t, acc);
-                            cnt += (uint32_t)mult - 1u;
+                            visit(l0[r] + 32u * c + k, G.shift[3u * seg + (uint32_t)r]);
                         }
-            }
-            G.sum[lane] = acc;
-            G.listed[lane] = nn | (nn + cnt) << 16;  // entries, and with multiplicity
-            __syncthreads();
-            const uint32_t n0 = layers[0].listed[lane] & 0xFFFFu, n1 = layers[1].listed[lane] & 0xFFFFu;
-            const uint32_t all = n0 + n1 + (layers[2].listed[lane] & 0xFFFFu);
-            const bool listing = !__any(all > kListMax);
+            };
             if (listing) {
                 uint32_t *lp = nl.list + list_at(lz == 0 ? 0u : lz == 1 ? n0 : n0 + n1, s, nl.stride);
-#pragma unroll
-                for (int r = 0; r < 3; ++r) {
-                    const uint32_t slot0 = l0[r] - G.shift[3u * seg + (uint32_t)r];
-#pragma unroll
-                    for (uint32_t c = 0; c < kStageWords; ++c)
-                        for (uint32_t bits = mask[r][c]; bits != 0u;) {
-                            const uint32_t k = (uint32_t)__builtin_clz(bits);
-                            bits &= ~(0x80000000u >> k);
-                            *lp = slot0 + 32u * c + k;
-                            lp += nl.stride;
+                neighbours([&](uint32_t k, uint32_t shift) {
+                    *lp = k - shift;
+                    lp += nl.stride;
+                });
+            }
+            uint32_t cnt = nn;
+            if (parallel && !any_slow) {
+                if (COUNT)
+                    G.counted[lane] = cnt;
+                if (COUNT)
+                    __syncthreads();
+            } else {
+                // The terms again, neighbours only, each with its m_ij; one
+                // layer after the other where they don't all fit.
+                RefCell ci{0, 0, 0};
+                if (slow)
+                    ci = ref_cell(pi, P);
+                auto again = [&](auto add) {
+                    neighbours([&](uint32_t k, uint32_t shift) {
+                        const float t = test(stage.x[k], stage.y[k], stage.z[k]);
+                        float term = mp6 * ((t * t) * t);
+                        if (slow) {
+                            const uint32_t hash = __float_as_uint(pos[k - shift].w) & 0xFFFFu;
+                            const int mult = bucket_multiplicity(ci.x, ci.y, ci.z, hash);
+                            term = (float)mult * term;
+                            cnt += (uint32_t)mult - 1u;
                         }
+                        add(term);
+                    });
+                };
+                acc = 0.0f;
+                if (parallel) {
+                    at_term = term0;
+                    again([&](float term) {
+                        if (lz == 0) {
+                            acc += term;
+                        } else {
+                            terms[at_term] = term;
+                            at_term += next_term;
+                        }
+                    });
+                    G.counted[lane] = cnt;
+                    __syncthreads();
+                } else {
+                    for (int turn = 0; turn < 3; ++turn) {
+                        if (turn == lz) {
+                            acc = turn != 0 ? stage.term[0][lane] : 0.0f;
+                            again([&](float term) { acc += term; });
+                            stage.term[0][lane] = acc;
+                            G.counted[lane] = cnt;
+                        }
+                        __syncthreads();
+                    }
                 }
             }
             if (lz != 0)
                 return;
+            if (parallel) {
+                const uint32_t rest = n1 + n2, most = (uint32_t)wave_max_i((int)rest);
+                for (uint32_t k = 0; k < most; k += 4u) {
+                    float v[4];
+#pragma unroll
+                    for (uint32_t i = 0; i < 4u; ++i) {
+                        const uint32_t q = min(k + i, kStageTerms - 1u);
+                        v[i] = stage.term[q < n1 ? q : kStageTerms - 1u - (q - n1)][lane];
+                    }
+#pragma unroll
+                    for (uint32_t i = 0; i < 4u; ++i) {
+                        const float term = any_slow ? v[i] : mp6 * ((v[i] * v[i]) * v[i]);
+                        acc = k + i < rest ? acc + term : acc;
+                    }
+                }
+            } else {
+                acc = stage.term[0][lane];
+            }
             UnionRows U{0, 0, 0, 0, 0, 0, false};
             uint32_t ucount = 0, unused = kNoOwn, w = kWalkUnion | kWalkSummed;
             if (!listing && plan_union(cstart, cc, active, P, U, ucount, unused) && !any_slow)
                 w |= kWalkBox | (U.segments ? kWalkSegments : 0u);  // for the force pass
             if (active) {
                 const float4 vs = vel[s];
-                const float sum = (acc + layers[1].sum[lane]) + layers[2].sum[lane];
-                const float d = P.mp6 * sum + P.self_dens;
+                const float d = acc + P.self_dens;
                 rho[s] = d;
                 posR[s] = make_float4(pi.x, pi.y, pi.z, 0.5f / d);
                 velR[s] = make_float4(vs.x, vs.y, vs.z, P.gas * (d - P.rho0));
                 nl.count[s] = listing ? all : kNoList;
                 if (COUNT)
-                    count[s] = (layers[0].listed[lane] >> 16) + (layers[1].listed[lane] >> 16) +
-                               (layers[2].listed[lane] >> 16);
+                    count[s] = layers[0].counted[lane] + layers[1].counted[lane] + layers[2].counted[lane];
             }
             if (lane == 0u) {
                 pp.measure[task] = 0u;
@@ -1790,13 +1870,8 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
         if (slow)
             ci = ref_cell(pi, P);
         const float h2 = P.h2;
-        // Terms are added up per z-layer of the stencil, then the layers'
-        // sums in order, in every walk (k_plan_list sums layers in parallel).
-        float acc = 0.0f, sum = 0.0f;
-        auto layer = [&] {
-            sum = sum + acc;
-            acc = 0.0f;
-        };
+        const float mp6 = P.mp6;
+        float acc = 0.0f;
         uint32_t cnt = 0;
         uint32_t listed = kNoList;
         uint64_t w = (MODE == 2 && active) ? dump.off[s] : 0;
@@ -1812,7 +1887,8 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
                     m = bucket_multiplicity(cx, cy, cz, __float_as_uint(q.w) & 0xFFFFu);
                 }
                 float t = h2 - d2;
-                acc = fmaf((float)m * (t * t), t, acc);
+                const float term = mp6 * ((t * t) * t);
+                acc += (float)m * term;
                 if (kCount)
                     cnt += (uint32_t)m;
                 if (MODE == 2 && active) {
@@ -1844,14 +1920,16 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
             uint32_t *lp = nl.list + s;
             const uint32_t W = 2u * (uint32_t)P.reach + 1u;
             float4 me = pi;  // far away from the candidates of other lanes' segments
-            auto walk = [&](auto unit_tag) {
+            // Unsplit sums are the per-lane walk's bit for bit.  Split ones
+            // (added up part by part, so never quite those) leave the factor
+            // to the end of the part: two operations a term instead of four.
+            auto walk = [&](auto unit_tag, auto split_tag) {
+                constexpr bool unit = decltype(unit_tag)::value, split = decltype(split_tag)::value;
                 union_walk<1, false>(lo, hi, L.first, src, T, [&](const ChunkRecords<1> &c, const uint32_t *slots,
                                                                       uint32_t n, bool odd, uint32_t lz) {
-                    if (lz != at_layer) {
-                        layer();
+                    if (U.segments && lz != at_layer) {
                         at_layer = lz;
-                        if (U.segments)
-                            me.x = T.segment[threadIdx.x & 63u] == lz / W ? pi.x : kFarAway;
+                        me.x = T.segment[threadIdx.x & 63u] == lz / W ? pi.x : kFarAway;
                     }
                     // Branch-free: h2 - d2 > 0 exactly when d2 < h2 (the float
                     // difference of unequal values is nonzero), so clamping it
@@ -1859,14 +1937,19 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
                     // leaves acc unchanged bit for bit.
                     auto term = [&](float x, float y, float z) {
                         float dx, dy, dz;
-                        return positive<decltype(unit_tag)::value>(
-                            h2v - dist2_ref(me, make_float4(x, y, z, 0.0f), dx, dy, dz));
+                        return positive<unit>(h2v - dist2_ref(me, make_float4(x, y, z, 0.0f), dx, dy, dz));
                     };
-                    if (listing || odd) {
+                    auto add = [&](float t) {
+                        if (split)
+                            acc = fmaf(t * t, t, acc);
+                        else
+                            acc = acc + mp6 * ((t * t) * t);
+                    };
+                    if ((!split && listing) || odd) {
                         for (uint32_t k = 0; k < n; ++k) {
                             const uint32_t j = slots[k];
                             const float t = j != s ? term(c.x[k], c.y[k], c.z[k]) : 0.0f;
-                            acc = fmaf(t * t, t, acc);
+                            add(t);
                             if (t > 0.0f) {
                                 if (kCount)
                                     ++cnt;
@@ -1888,18 +1971,22 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
                                             term(x.w, y.w, z.w)};
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            acc = fmaf(t[i] * t[i], t[i], acc);
+                            add(t[i]);
                             if (kCount)
                                 cnt += t[i] > 0.0f ? 1u : 0u;
                         }
                     }
                 });
             };
-            if (P.h2 <= 1.0f)
-                walk(std::true_type{});
-            else
-                walk(std::false_type{});
-            layer();
+            if (nparts == 1u) {
+                walk(std::false_type{}, std::false_type{});
+            } else {
+                if (h2 <= 1.0f)
+                    walk(std::true_type{}, std::true_type{});
+                else
+                    walk(std::false_type{}, std::true_type{});
+                acc = mp6 * acc;
+            }
             if (listing)
                 listed = nn;
         } else if ((MODE == 0 || MODE == 3) && nl.list && nparts == 1u) {
@@ -1922,7 +2009,7 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
                 float dx, dy, dz;
                 const float d2 = dist2_ref(pi, q, dx, dy, dz);
                 const float t = fmaxf(h2 - d2, 0.0f);
-                acc = fmaf(t * t, t, acc);
+                acc = acc + mp6 * ((t * t) * t);
                 if (kCount)
                     cnt += t > 0.0f ? 1u : 0u;
                 return t > 0.0f;
@@ -2013,7 +2100,7 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
                     }
                     listing = !__any(nn > kListMax);
                 }
-            }, layer);
+            });
             if (!any_slow && direct)
                 listing = !__any(nn > kListMax);
             listed = listing ? nn : kNoList;
@@ -2036,9 +2123,8 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
                 for (; j < e; ++j)
                     if (j != s)
                         body(j, pos[j]);
-            }, layer);
+            });
         }
-        acc = sum;
         if (nparts > 1u) {
             if constexpr (kCount) {
                 float v[2] = {acc, (float)cnt};  // counts stay far below 2^24: exact
@@ -2055,7 +2141,7 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
         }
         if (!active)
             return;
-        const float r = P.mp6 * acc + P.self_dens;
+        const float r = acc + P.self_dens;
         const float p = P.gas * (r - P.rho0);
         rho[s] = r;
         posR[s] = make_float4(pi.x, pi.y, pi.z, 0.5f / r);
@@ -2183,17 +2269,29 @@ __device__ inline void integrate_and_walls(float4 &x, float4 &v, float fx, float
 // h - r cancels, and an error in r would be amplified).  A candidate that is
 // no neighbour has d2 >= fl(h h), so r >= h (the root of the rounded square
 // is h itself) and h - r clamps to 0: it adds zeros, without a test.
-template <bool UNIT>
+// SPLIT: the part of a split walk, whose sums depend on the parts' bounds
+// anyway: the same product in an order that takes fewer operations and root()
+// (28 against 49 issue cycles a wave before the six fmas).  Unsplit walks
+// keep one order of operations in all their forms.
+template <bool UNIT, bool SPLIT>
 __device__ inline void force_pair(float d2, float dx, float dy, float dz, float am, float4 w, float4 vi,
                                   float p_i, float h, float neg_m_spg, float mu2_m_lap, float &fx,
                                   float &fy, float &fz)
 {
-    float rinv;
-    const float r = root(d2, rinv);
-    const float hr = positive<UNIT>(h - r);
-    const float u = hr * am;
-    const float cp = ((p_i + w.w) * neg_m_spg) * u * (hr * rinv);
-    const float cv = u * mu2_m_lap;
+    float cp, cv;
+    if (SPLIT) {
+        float rinv;
+        const float r = root(d2, rinv);
+        const float hr = positive<UNIT>(h - r);
+        const float u = hr * am;
+        cp = ((p_i + w.w) * neg_m_spg) * u * (hr * rinv);
+        cv = u * mu2_m_lap;
+    } else {
+        const float r = sqrt_rn(d2);
+        const float hr = positive<UNIT>(h - r);
+        cp = neg_m_spg * (p_i + w.w) * am * (hr * hr) * __builtin_amdgcn_rcpf(r);
+        cv = mu2_m_lap * hr * am;
+    }
     fx = fmaf(cp, dx, fx);
     fy = fmaf(cp, dy, fy);
     fz = fmaf(cp, dz, fz);
@@ -2249,7 +2347,7 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                 asm volatile("" : "+v"(cx), "+v"(cy), "+v"(cz));
                 am = q.w * (float)bucket_multiplicity(cx, cy, cz, __float_as_uint(posB[j].w) & 0xFFFFu);
             }
-            force_pair<false>(d2, dx, dy, dz, am, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+            force_pair<false, false>(d2, dx, dy, dz, am, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
         };
         // Every lane holds its neighbour list (the density pass walked this
         // task per lane, unsplit): visit the listed slots four at a time,
@@ -2301,8 +2399,8 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
             const uint32_t W = 2u * (uint32_t)P.reach + 1u;
             uint32_t at_layer = kNoSlot;
             float4 me = pi;  // far away from the candidates of other lanes' segments
-            auto walk = [&](auto unit_tag) {
-                constexpr bool unit = decltype(unit_tag)::value;
+            auto walk = [&](auto unit_tag, auto split_tag) {
+                constexpr bool unit = decltype(unit_tag)::value, split = decltype(split_tag)::value;
                 union_walk<2, true>(lo, hi, L.first, src, T, [&](const ChunkRecords<2> &c, const uint32_t *slots,
                                                                      uint32_t n, bool odd, uint32_t lz) {
                     const float4(&rec)[2][64] = c.rec;
@@ -2316,23 +2414,25 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                             const float4 q = rec[0][k], w = rec[1][k];  // (x_j, 0.5 / rho_j), (v_j, p_j)
                             const float d2 = dist2_ref(me, q, dx, dy, dz);
                             if (d2 < h2 && slots[k] != s)
-                                force_pair<unit>(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                                force_pair<unit, split>(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
                         }
                         return;
                     }
                     for (uint32_t k = 0; k < n; k += 2u) {
                         const float4 q0 = rec[0][k], w0 = rec[1][k], q1 = rec[0][k + 1u], w1 = rec[1][k + 1u];
                         float d2 = dist2_ref(me, q0, dx, dy, dz);
-                        force_pair<unit>(d2, dx, dy, dz, q0.w, w0, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                        force_pair<unit, split>(d2, dx, dy, dz, q0.w, w0, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
                         d2 = dist2_ref(me, q1, dx, dy, dz);
-                        force_pair<unit>(d2, dx, dy, dz, q1.w, w1, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                        force_pair<unit, split>(d2, dx, dy, dz, q1.w, w1, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
                     }
                 });
             };
-            if (P.h <= 1.0f)
-                walk(std::true_type{});
+            if (nparts == 1u)
+                walk(std::false_type{}, std::false_type{});
+            else if (P.h <= 1.0f)
+                walk(std::true_type{}, std::true_type{});
             else
-                walk(std::false_type{});
+                walk(std::false_type{}, std::true_type{});
         } else {
             uint32_t lo = 0, hi = 0xFFFFFFFFu;
             if (nparts > 1u) {
@@ -2359,7 +2459,7 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                         pair(j, posR[j], velR[j]);  // (x_j, 0.5 / rho_j), (v_j, p_j)
                     }
                 }
-            }, [] {});
+            });
         }
         if (nparts > 1u) {
             float v[3] = {fx, fy, fz};
@@ -2463,7 +2563,7 @@ __global__ __launch_bounds__(kBlock) void k_grid_stat(const float4 *__restrict__
         const float4 pi = pos[s];
         const float h2 = P.h2;
         const uint32_t cc = cellc[s];
-        for_each_row(cstart, cc, P, [&](uint32_t b, uint32_t e) { cand += e - b; }, [] {});
+        for_each_row(cstart, cc, P, [&](uint32_t b, uint32_t e) { cand += e - b; });
         const uint32_t stride = max((cand + kGridStatTests - 1u) / kGridStatTests, 1u);
         uint32_t q = 0;  // offset of the next tested candidate in the current row
         for_each_row(cstart, cc, P, [&](uint32_t b, uint32_t e) {
@@ -2473,7 +2573,7 @@ __global__ __launch_bounds__(kBlock) void k_grid_stat(const float4 *__restrict__
                 nbr += (j != s && dist2_ref(pi, pos[j], dx, dy, dz) < h2) ? 1u : 0u;
             }
             q -= e - b;
-        }, [] {});
+        });
         nbr *= stride;
     }
     unsigned long long c = cand, nb = nbr;
