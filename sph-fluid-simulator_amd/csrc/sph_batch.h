@@ -72,7 +72,7 @@ struct Batch {
     uint64_t max_capacity = 0;  // particle capacity relayout may grow to (0: unbounded)
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    using GraphKey = std::array<uint64_t, 42>;
+    using GraphKey = std::array<uint64_t, 40>;
     GraphKey captured{};     // what the launches of `exec` were given
     bool complete = false;  // every scene has been uploaded since the scene list last changed
     DevBuf aos, xf;  // download_particles staging

@@ -568,10 +568,10 @@ Batch::GraphKey Batch::graph_key() const
     return GraphKey{at(a.posA),    at(a.velA),   at(a.posB),      at(a.velB),      at(a.cellcA),   at(a.rankA),
                     at(a.cellcB),  at(a.perm),   at(a.rhoB),      at(a.posR),      at(a.velR),     at(c.counts),
                     at(c.cstart),  at(c.partials), at(c.big),     at(c.unordered), at(S.params),   at(S.tasks),
-                    at(p.nparts),  at(p.off),    at(p.scan_partials), at(p.measure), at(p.total),  at(p.tasks),
+                    at(p.nparts),  at(p.off),    at(p.measure),  at(p.total),     at(p.tasks),
                     at(p.queue),   at(p.buf),    at(p.done),      at(p.walk),      at(p.own),      at(l.list),
                     at(l.count),   at(w.force.ptr), c.big_cap,    c.ncells_padded, S.nwaves,       S.staged,
-                    p.padded,      p.nscenes,    p.cap,           l.stride,        (uint64_t)w.stencil_block,
+                    p.nscenes,    p.cap,           l.stride,        (uint64_t)w.stencil_block,
                     keep_force};
 }
 
@@ -890,7 +890,7 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
     for (uint32_t k = 0; k < s; ++k)
         t0 += (scenes[k].desc.n + 63u) / 64u;
     const uint32_t nt = (n + 63u) / 64u;
-    std::vector<uint32_t> cnt(n), lc(n), off(nt + 1), ids(n);
+    std::vector<uint32_t> cnt(n), lc(n), parts(nt), ids(n);
     std::vector<float4> vb(n);
     std::vector<int4> wk(2ull * nt);
     std::vector<uint32_t> lst(list ? (size_t)kListMax * n : 0);
@@ -900,7 +900,7 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
     if (e == hipSuccess)
         e = hipMemcpyAsync(vb.data(), a.velB + p0, 16ull * n, hipMemcpyDeviceToHost, stream);
     if (e == hipSuccess)
-        e = hipMemcpyAsync(off.data(), pp.off + t0, 4ull * (nt + 1), hipMemcpyDeviceToHost, stream);
+        e = hipMemcpyAsync(parts.data(), pp.nparts + t0, 4ull * nt, hipMemcpyDeviceToHost, stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(wk.data(), pp.walk + 2ull * t0, sizeof(int4) * 2ull * nt, hipMemcpyDeviceToHost, stream);
     for (uint32_t k = 0; list && k < kListMax && e == hipSuccess; ++k)  // entry k of every slot
@@ -920,7 +920,7 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
             return fail(SPH_E_HIP, "walk_dump: slot %u holds id %u of %u", q, id, n);
         count[id] = cnt[q];
         if (walk)
-            walk[id] = (wk[2 * t + 1].w & (int)kWalkUnion ? 1u : 0u) | (off[t + 1] != off[t] ? 2u : 0u) | (lc[q] != kNoList ? 4u : 0u);
+            walk[id] = (wk[2 * t + 1].w & (int)kWalkUnion ? 1u : 0u) | (parts[t] ? 2u : 0u) | (lc[q] != kNoList ? 4u : 0u);
         if (list_count)
             list_count[id] = lc[q];
         if (list && lc[q] != kNoList)

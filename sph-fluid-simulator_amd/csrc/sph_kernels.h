@@ -117,17 +117,14 @@ SPH_HD inline uint64_t part_room(uint64_t waves)
 constexpr uint32_t kTotalSlots = 8;
 
 struct PartPlan {
-    uint32_t *nparts;    // per wave task: parts of a split task, 0 for an unsplit one; padded
-                         // to a kScanChunk multiple (zero outside use)
-    uint32_t *off;       // exclusive scan of nparts; off[nwaves] = number of queued part tasks
-    uint32_t *scan_partials;
-    uint32_t padded;     // padded length of nparts
+    uint32_t *nparts;    // per wave task: parts of a split task, 0 for an unsplit one
+    uint32_t *off;       // of a split task: place of its first part in tasks and buf
     uint32_t *measure;   // walk length per wave task
     unsigned long long *total;  // sums of the long walks' lengths, kTotalSlots per scene (zero between steps)
     uint32_t nscenes;
     uint32_t cap;        // part-task capacity: sum over scenes of waves + part_room(waves)
     uint32_t *tasks;     // (wave task << kPartBits) | part, cap entries
-    uint32_t *queue;     // pulled-task counters: [0] density, [1] force
+    uint32_t *queue;     // pulled-task counters: [0] density, [1] force; [2] parts queued
     float4 *buf;         // partial sums: four arrays of 64 lanes per part task (cap * 64 entries)
     uint32_t *done;      // parts finished per wave task (zero between passes)
     int4 *walk;          // per wave task, two entries: union box (x0, x1, y0, y1), (z0, z1, union

@@ -365,8 +365,11 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t x, uint32_t *total)
     return off + inc - x;
 }
 
-__global__ void k_scan_reduce(const uint32_t *__restrict__ counts, uint32_t *__restrict__ partials)
+__global__ void k_scan_reduce(const uint32_t *__restrict__ counts, uint32_t *__restrict__ partials,
+                              uint32_t *__restrict__ big)
 {
+    if (big && blockIdx.x == 0u && threadIdx.x == 0u)
+        big[0] = 0u;  // the big-cell count
     const uint4 *src = (const uint4 *)(counts + (size_t)blockIdx.x * kScanChunk);
     uint32_t s = 0;
 #pragma unroll
@@ -380,10 +383,8 @@ __global__ void k_scan_reduce(const uint32_t *__restrict__ counts, uint32_t *__r
         partials[blockIdx.x] = tot;
 }
 
-// One block: exclusive scan of nparts block totals in place; cstart_end
-// receives the grand total.  Also clears the big-cell count.
-__global__ void k_scan_partials(uint32_t *__restrict__ partials, uint32_t nparts,
-                                uint32_t *__restrict__ cstart_end, uint32_t *__restrict__ big)
+// One block: exclusive scan of nparts block totals in place.
+__global__ void k_scan_partials(uint32_t *__restrict__ partials, uint32_t nparts)
 {
     uint32_t carry = 0;
     for (uint32_t base = 0; base < nparts; base += kBlock) {
@@ -395,19 +396,21 @@ __global__ void k_scan_partials(uint32_t *__restrict__ partials, uint32_t nparts
             partials[i] = carry + ex;
         carry += tot;
     }
-    if (threadIdx.x == 0) {
-        *cstart_end = carry;
-        if (big)
-            big[0] = 0u;
-    }
 }
 
+// SUMS: partials holds the blocks' own totals, and each block adds up those
+// before it; otherwise k_scan_partials has.
+template <bool SUMS>
 __global__ void k_scan_final(uint32_t *__restrict__ counts, const uint32_t *__restrict__ partials,
                              uint32_t *__restrict__ cstart, uint32_t *__restrict__ big, uint32_t big_cap,
                              bool clear)
 {
     size_t base = (size_t)blockIdx.x * kScanChunk + (size_t)threadIdx.x * kScanItems;
     uint4 *src = (uint4 *)(counts + base);
+    uint32_t before = 0;
+    if (SUMS)
+        for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kBlock)
+            before += partials[b];
     uint32_t v[kScanItems];
 #pragma unroll
     for (int k = 0; k < kScanItems / 4; ++k) {
@@ -422,7 +425,13 @@ __global__ void k_scan_final(uint32_t *__restrict__ counts, const uint32_t *__re
     for (int k = 0; k < kScanItems; ++k)
         local += v[k];
     uint32_t tot;
-    uint32_t run = block_exclusive_scan(local, &tot) + partials[blockIdx.x];
+    uint32_t run = block_exclusive_scan(local, &tot);
+    if (SUMS) {
+        block_exclusive_scan(before, &tot);
+        run += tot;
+    } else {
+        run += partials[blockIdx.x];
+    }
     uint4 *dst = (uint4 *)(cstart + base);
 #pragma unroll
     for (int k = 0; k < kScanItems / 4; ++k) {
@@ -439,6 +448,8 @@ __global__ void k_scan_final(uint32_t *__restrict__ counts, const uint32_t *__re
         if (clear)
             src[k] = make_uint4(0u, 0u, 0u, 0u);
     }
+    if (blockIdx.x + 1u == gridDim.x && threadIdx.x + 1u == blockDim.x)
+        cstart[base + kScanItems] = run;  // the grand total, behind the last cell
     if (big) {
 #pragma unroll
         for (int k = 0; k < kScanItems; ++k) {
@@ -451,14 +462,24 @@ __global__ void k_scan_final(uint32_t *__restrict__ counts, const uint32_t *__re
     }
 }
 
+// Up to so many blocks each adds up the totals before it (a load or two a
+// thread): one launch fewer, which at a few cells is what a scan costs
+// (8,000 particles: 9.1 -> 8.2 us).  Beyond, those sums would read more than
+// the scan does.
+constexpr uint32_t kScanSumsMax = 1024;
+
 void launch_scan(hipStream_t st, const CellArrays &c, bool clear_counts)
 {
     uint32_t nparts = c.ncells_padded / kScanChunk;
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nparts), dim3(kBlock), 0, st, c.counts, c.partials);
-    hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kBlock), 0, st, c.partials, nparts,
-                       c.cstart + c.ncells_padded, c.big);
-    hipLaunchKernelGGL(k_scan_final, dim3(nparts), dim3(kBlock), 0, st, c.counts, c.partials,
-                       c.cstart, c.big, c.big_cap, clear_counts);
+    hipLaunchKernelGGL(k_scan_reduce, dim3(nparts), dim3(kBlock), 0, st, c.counts, c.partials, c.big);
+    if (nparts <= kScanSumsMax) {
+        hipLaunchKernelGGL((k_scan_final<true>), dim3(nparts), dim3(kBlock), 0, st, c.counts, c.partials, c.cstart,
+                           c.big, c.big_cap, clear_counts);
+        return;
+    }
+    hipLaunchKernelGGL(k_scan_partials, dim3(1), dim3(kBlock), 0, st, c.partials, nparts);
+    hipLaunchKernelGGL((k_scan_final<false>), dim3(nparts), dim3(kBlock), 0, st, c.counts, c.partials, c.cstart, c.big,
+                       c.big_cap, clear_counts);
 }
 
 // ---------------------------------------------------------- scatter/reorder
@@ -1327,6 +1348,8 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
     const uint32_t task = xcd_block();
     if (task >= S.nwaves)
         return;
+    if (task == 0u && threadIdx.x < 3u)
+        pp.queue[threadIdx.x] = 0u;  // parts taken by the density and force passes, parts queued
     Lane L;
     bool active;
     wave_task(S, task, L, active);
@@ -1682,43 +1705,44 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
     }
 }
 
-// Parts per wave task: the part size grows beyond kPartCandidates when the
-// scene's total walk over its part room would exceed it.
-__global__ void k_count_parts(const uint32_t *__restrict__ measure, SceneSet S,
-                              const unsigned long long *__restrict__ total, uint32_t *__restrict__ nparts)
+// Parts per wave task, queued: the part size grows beyond kPartCandidates
+// when the scene's total walk over its part room would exceed it.  A wave's
+// split tasks take their places in the queue with one atomic; their order
+// there varies, the sums of a task don't depend on it.  (8,000 particles: 4.8 us;
+// counting, a scan of
+// the counts and writing them out in five launches took 16.3.)
+__global__ __launch_bounds__(kBlock) void k_queue_parts(SceneSet S, PartPlan pp)
 {
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= S.nwaves)
-        return;
-    const uint32_t scene = S.tasks[g].scene;
-    const StepParams &P = S.params[scene];
-    const unsigned long long waves = (P.p_end - P.p_begin + 63u) / 64u;
-    const unsigned long long room = part_room(waves);
-    unsigned long long sum = 0;
-    for (uint32_t k = 0; k < kTotalSlots; ++k)
-        sum += total[kTotalSlots * scene + k];
-    const unsigned long long size = max((unsigned long long)kPartCandidates, (sum + room - 1u) / room);
-    const unsigned long long p = (measure[g] + size - 1u) / size;
-    const uint32_t np = (uint32_t)min(p, (unsigned long long)kMaxParts);
-    nparts[g] = np > 1u ? np : 0u;  // an unsplit task is not queued
-}
-
-__global__ void k_emit_parts(const uint32_t *__restrict__ off, uint32_t ntasks, uint32_t *__restrict__ tasks,
-                             uint32_t *__restrict__ queue, unsigned long long *__restrict__ total,
-                             uint32_t nscenes)
-{
-    const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g == 0) {
-        queue[0] = 0u;
-        queue[1] = 0u;
+    const uint32_t g = blockIdx.x * kBlock + threadIdx.x;
+    uint32_t np = 0;
+    if (g < S.nwaves) {
+        const uint32_t length = pp.measure[g];
+        if (length > kPartCandidates) {
+            const uint32_t scene = S.tasks[g].scene;
+            const StepParams &P = S.params[scene];
+            const unsigned long long waves = (P.p_end - P.p_begin + 63u) / 64u;
+            const unsigned long long room = part_room(waves);
+            unsigned long long sum = 0;
+            for (uint32_t k = 0; k < kTotalSlots; ++k)
+                sum += pp.total[kTotalSlots * scene + k];
+            const unsigned long long size = max((unsigned long long)kPartCandidates, (sum + room - 1u) / room);
+            const unsigned long long p = (length + size - 1u) / size;
+            np = (uint32_t)min(p, (unsigned long long)kMaxParts);
+            np = np > 1u ? np : 0u;  // an unsplit task is not queued
+        }
+        pp.nparts[g] = np;
     }
-    for (uint32_t k = g; k < kTotalSlots * nscenes; k += gridDim.x * blockDim.x)
-        total[k] = 0ull;  // for the next step's plan
-    if (g >= ntasks)
+    if (!__any(np != 0u))
         return;
-    const uint32_t b = off[g], e = off[g + 1];
-    for (uint32_t p = 0; b + p < e; ++p)
-        tasks[b + p] = (g << kPartBits) | p;
+    const uint32_t end = wave_inclusive_scan(np);
+    uint32_t base = 0;
+    if ((threadIdx.x & 63u) == 63u)
+        base = atomicAdd(&pp.queue[2], end);
+    base = (uint32_t)__builtin_amdgcn_readlane((int)base, 63) + end - np;
+    if (np != 0u)
+        pp.off[g] = base;
+    for (uint32_t p = 0; p < np; ++p)
+        pp.tasks[base + p] = (g << kPartBits) | p;
 }
 
 void launch_plan_parts(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
@@ -1735,18 +1759,7 @@ void launch_plan_parts(hipStream_t st, const ParticleArrays &a, const CellArrays
     else
         SPH_LAUNCH_PLAN(false, false);  // counts nothing itself
 #undef SPH_LAUNCH_PLAN
-    hipLaunchKernelGGL(k_count_parts, dim3(blocks_for(S.nwaves)), dim3(kBlock), 0, st, pp.measure, S, pp.total,
-                       pp.nparts);
-    CellArrays cs;
-    cs.counts = pp.nparts;
-    cs.cstart = pp.off;
-    cs.partials = pp.scan_partials;
-    cs.big = nullptr;
-    cs.big_cap = 0;
-    cs.ncells_padded = pp.padded;
-    launch_scan(st, cs, /*clear_counts=*/true);  // nparts must be zero for the next step
-    hipLaunchKernelGGL(k_emit_parts, dim3(blocks_for(S.nwaves)), dim3(kBlock), 0, st, pp.off, S.nwaves, pp.tasks,
-                       pp.queue, pp.total, pp.nscenes);
+    hipLaunchKernelGGL(k_queue_parts, dim3(blocks_for(std::max(1u, S.nwaves))), dim3(kBlock), 0, st, S, pp);
 }
 
 // Runs task(w, part, nparts) for the work the calling wave takes.  Without
@@ -1767,10 +1780,10 @@ __device__ inline void for_each_part(const SceneSet &S, const PartPlan &pp, uint
             task(first, 0u, 1u);
         return;
     }
-    const uint32_t total = __builtin_amdgcn_readfirstlane(pp.off[S.nwaves]);  // parts of split tasks
+    const uint32_t total = __builtin_amdgcn_readfirstlane(pp.queue[2]);  // parts of split tasks
     const uint32_t G = gridDim.x * (BLOCK / 64);
     for (uint32_t w = first; w < S.nwaves; w += G)
-        if (total == 0u || __builtin_amdgcn_readfirstlane(pp.off[w + 1] - pp.off[w]) == 0u)
+        if (total == 0u || __builtin_amdgcn_readfirstlane(pp.nparts[w]) == 0u)
             if (!skip_summed || !(__builtin_amdgcn_readfirstlane(pp.walk[2u * w + 1u].w) & (int)kWalkSummed))
                 task(w, 0u, 1u);
     if (total == 0u)
@@ -1784,7 +1797,7 @@ __device__ inline void for_each_part(const SceneSet &S, const PartPlan &pp, uint
             return;
         const uint32_t packed = __builtin_amdgcn_readfirstlane(pp.tasks[t]);
         const uint32_t w = packed >> kPartBits, part = packed & (kMaxParts - 1u);
-        const uint32_t nparts = __builtin_amdgcn_readfirstlane(pp.off[w + 1] - pp.off[w]);
+        const uint32_t nparts = __builtin_amdgcn_readfirstlane(pp.nparts[w]);
         task(w, part, nparts);
     }
 }
@@ -1855,6 +1868,9 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
 {
     constexpr bool kCount = MODE >= 1;
     __shared__ UnionStage<1> stage[MODE == 0 || MODE == 3 ? BLOCK / 64 : 1];
+    if (pp.queue && blockIdx.x == 0u)
+        for (uint32_t k = threadIdx.x; k < kTotalSlots * pp.nscenes; k += BLOCK)
+            pp.total[k] = 0ull;  // for the next step's plan
     for_each_part<BLOCK, true>(S, pp, pp.queue, [&](uint32_t wt, uint32_t part, uint32_t nparts) {
         Lane L;
         bool active;

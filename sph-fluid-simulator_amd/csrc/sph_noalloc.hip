@@ -51,10 +51,10 @@ struct Layout {
     size_t counts, cstart, partials, big;
     size_t force, perm16, counts16, cstart16, partials16;
     size_t params, tasks;
-    size_t nparts, off, ppartials, measure, total, ptasks, queue, buf, done, walk, own;
+    size_t nparts, off, measure, total, ptasks, queue, buf, done, walk, own;
     size_t nlist, ncount;
     size_t bytes;  // end of the last buffer
-    uint32_t ncells_padded, big_cap, nwaves, waves_padded, cap;
+    uint32_t ncells_padded, big_cap, nwaves, cap;
 };
 
 struct Carver {
@@ -105,11 +105,9 @@ Layout make_layout(uint32_t n, uint64_t ncells)
     L.params = c.take(sizeof(StepParams));
     L.nwaves = (n + 63u) / 64u;
     L.tasks = c.take(sizeof(WaveTask) * (size_t)L.nwaves);
-    L.waves_padded = (L.nwaves + kScanChunk - 1) / kScanChunk * kScanChunk;
     L.cap = (uint32_t)(L.nwaves + part_room(L.nwaves));
-    L.nparts = c.take(4ull * L.waves_padded);
-    L.off = c.take(4ull * (L.waves_padded + 1));
-    L.ppartials = c.take(4ull * (L.waves_padded / kScanChunk));
+    L.nparts = c.take(4ull * L.nwaves);
+    L.off = c.take(4ull * L.nwaves);
     L.measure = c.take(4ull * L.nwaves);
     L.total = c.take(8 * kTotalSlots);
     L.ptasks = c.take(4ull * L.cap);
@@ -255,8 +253,6 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     PartPlan pp;
     pp.nparts = (uint32_t *)at(L.nparts);
     pp.off = (uint32_t *)at(L.off);
-    pp.scan_partials = (uint32_t *)at(L.ppartials);
-    pp.padded = L.waves_padded;
     pp.measure = (uint32_t *)at(L.measure);
     pp.total = (unsigned long long *)at(L.total);
     pp.nscenes = 1;
@@ -268,10 +264,9 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     pp.walk = (int4 *)at(L.walk);
     pp.own = (uint32_t *)at(L.own);
     // the previous call's contents are still there: clear what the passes
-    // expect at zero (cell counts, part counts, finished-part counters, the
-    // per-scene total; the queue counters are cleared by the plan itself)
+    // expect at zero (cell counts, finished-part counters, the per-scene
+    // total; the queue counters are cleared by the plan itself)
     launch_fill_u32(st, c.counts, 0u, c.ncells_padded);
-    launch_fill_u32(st, pp.nparts, 0u, L.waves_padded);
     launch_fill_u32(st, pp.done, 0u, L.nwaves);
     launch_fill_u32(st, (uint32_t *)pp.total, 0u, 2 * kTotalSlots);
 

@@ -87,16 +87,15 @@ struct Workspace {
     DevBuf counts, cstart, partials, big;
     DevBuf force;
     DevBuf params, tasks;  // scene table of the batch living in this workspace
-    // split wave tasks: parts per task (padded), their scan, scan partials,
-    // walk lengths and their total, part tasks, queue counters, partial sums,
+    // split wave tasks: parts per task, place of the first in the queue, walk
+    // lengths and their total, part tasks, queue counters, partial sums,
     // finished-part counters
-    DevBuf pnparts, poff, ppartials, pmeasure, ptotal, ptasks, pqueue, pbuf, pdone, pwalk, pown;
+    DevBuf pnparts, poff, pmeasure, ptotal, ptasks, pqueue, pbuf, pdone, pwalk, pown;
     // neighbour lists the density pass writes and the force pass reads
     DevBuf nlist, ncount;
     // cells left in arrival order (above the in-cell sort's limit), summed
     // over steps
     DevBuf unordered;
-    uint32_t parts_padded = 0;
     uint32_t ncells_padded = 0;
     uint32_t big_cap = 0;
     uint32_t nwaves = 0;

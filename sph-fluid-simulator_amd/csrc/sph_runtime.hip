@@ -465,7 +465,6 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
     size_t nslots = 0;
     for (const StepParams &sp : scenes)
         nslots = std::max<size_t>(nslots, sp.p_end);
-    const uint32_t padded = (uint32_t)((nw + kScanChunk - 1) / kScanChunk * kScanChunk);
     size_t cap = 0;  // every scene's wave tasks plus its part room
     for (const StepParams &sp : scenes) {
         const uint64_t waves = ((uint64_t)sp.p_end - sp.p_begin + 63u) / 64u;
@@ -474,20 +473,17 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
     cap = std::max<size_t>(cap, nw);
     if (cap > 0xFFFFFFFFull)
         return fail(SPH_E_LIMIT, "part plan: %zu part tasks", cap);
-    const bool fresh_counters = padded > parts_padded || pdone.bytes < 4 * nw ||
+    const bool fresh_counters = pdone.bytes < 4 * nw ||
                                 ptotal.bytes < 8 * kTotalSlots * std::max<size_t>(scenes.size(), 1);
-    if ((rc = pnparts.reserve(4ull * padded)) || (rc = poff.reserve(4ull * (padded + 1))) ||
-        (rc = ppartials.reserve(4ull * (padded / kScanChunk))) || (rc = pmeasure.reserve(4ull * nw)) ||
+    if ((rc = pnparts.reserve(4ull * nw)) || (rc = poff.reserve(4ull * nw)) || (rc = pmeasure.reserve(4ull * nw)) ||
         (rc = ptotal.reserve(8ull * kTotalSlots * std::max<size_t>(scenes.size(), 1))) || (rc = ptasks.reserve(4ull * cap)) ||
         (rc = pqueue.reserve(16)) ||
         (rc = pbuf.reserve(sizeof(float4) * 64ull * cap)) || (rc = pdone.reserve(4ull * nw)) ||
         (rc = pwalk.reserve(2ull * sizeof(int4) * nw)) || (rc = pown.reserve(4ull * std::max<size_t>(nslots, 1))))
         return rc;
     if (fresh_counters) {  // zero outside use from here on: the step keeps them so
-        launch_fill_u32(st, (uint32_t *)pnparts.ptr, 0u, pnparts.bytes / 4);
         launch_fill_u32(st, (uint32_t *)pdone.ptr, 0u, pdone.bytes / 4);
         launch_fill_u32(st, (uint32_t *)ptotal.ptr, 0u, ptotal.bytes / 4);
-        parts_padded = (uint32_t)(pnparts.bytes / 4 / kScanChunk * kScanChunk);
     }
     hipError_t e = hipSuccess;
     if (!scenes.empty())
@@ -558,8 +554,6 @@ PartPlan Workspace::part_plan() const
     PartPlan p;
     p.nparts = (uint32_t *)pnparts.ptr;
     p.off = (uint32_t *)poff.ptr;
-    p.scan_partials = (uint32_t *)ppartials.ptr;
-    p.padded = (nwaves + kScanChunk - 1) / kScanChunk * kScanChunk;
     p.measure = (uint32_t *)pmeasure.ptr;
     p.total = (unsigned long long *)ptotal.ptr;
     p.nscenes = nscenes;
@@ -590,7 +584,7 @@ void Workspace::release_all()
 {
     for (DevBuf *b : {&posA, &velA, &posB, &velB, &cellcA, &rankA, &cellcB, &perm, &rhoB, &posR, &velR,
                       &counts, &cstart, &partials, &big, &force, &params, &tasks, &pnparts, &poff,
-                      &ppartials, &pmeasure, &ptotal, &ptasks, &pqueue, &pbuf, &pdone, &pwalk, &pown,
+                      &pmeasure, &ptotal, &ptasks, &pqueue, &pbuf, &pdone, &pwalk, &pown,
                       &nlist, &ncount, &unordered})
         b->release();
     host_tasks.clear();
@@ -598,7 +592,6 @@ void Workspace::release_all()
     big_cap = 0;
     nwaves = 0;
     nscenes = 0;
-    parts_padded = 0;
 }
 
 void enqueue_step(hipStream_t st, Workspace &w, float4 *force_out, bool next_keys, StepTimer *timer)
