@@ -245,6 +245,7 @@ void DevBuf::release()
 
 namespace {
 constexpr int kCopiers = 8;
+constexpr size_t kPerCopier = 4ull << 20;
 }  // namespace
 
 struct Staging {
@@ -293,9 +294,10 @@ std::shared_ptr<Staging> staging()
     }
 }
 
-// Copier t of a download: every kCopiers-th piece, through its own part of
-// the staging memory, while the copies of the others run.
-hipError_t copy_pieces(int device, hipStream_t st, const HostSpan *spans, int count, int t, unsigned char *buf)
+// Copier t of a download by `workers`: every workers-th piece, through its
+// own part of the staging memory, while the copies of the others run.
+hipError_t copy_pieces(int device, hipStream_t st, const HostSpan *spans, int count, int t, int workers,
+                       unsigned char *buf)
 {
     hipEvent_t done = nullptr;
     hipError_t err = hipSetDevice(device);
@@ -304,7 +306,7 @@ hipError_t copy_pieces(int device, hipStream_t st, const HostSpan *spans, int co
     size_t piece = 0;
     for (int k = 0; k < count; ++k)
         for (size_t at = 0; at < spans[k].bytes && err == hipSuccess; at += kPiece, ++piece) {
-            if (piece % kCopiers != (size_t)t)
+            if (piece % (size_t)workers != (size_t)t)
                 continue;
             const size_t bytes = std::min(kPiece, spans[k].bytes - at);
             err = hipMemcpyAsync(buf, (const char *)spans[k].src + at, bytes, hipMemcpyDeviceToHost, st);
@@ -346,11 +348,9 @@ unsigned char *HostStage::small(size_t want)
 
 int copy_to_host(hipStream_t st, const HostSpan *spans, int count, HostStage &stage)
 {
-    size_t total = 0, pieces = 0;
-    for (int k = 0; k < count; ++k) {
+    size_t total = 0;
+    for (int k = 0; k < count; ++k)
         total += spans[k].bytes;
-        pieces += (spans[k].bytes + kPiece - 1) / kPiece;
-    }
     hipError_t e = hipSuccess;
     if (unsigned char *buf = stage.small(total)) {
         size_t at = 0;
@@ -388,8 +388,11 @@ int copy_to_host(hipStream_t st, const HostSpan *spans, int count, HostStage &st
     std::lock_guard<std::mutex> lock(ring.mu);
     hipError_t failed[kCopiers] = {};
     std::thread threads[kCopiers];
-    const int workers = (int)std::min<size_t>(kCopiers, pieces);
-    auto copier = [&](int t) { failed[t] = copy_pieces(device, st, spans, count, t, ring.base + kPiece * (size_t)t); };
+    // (a thread's first calls into the runtime take a millisecond now and then)
+    const int workers = (int)std::min<size_t>(kCopiers, 1 + total / kPerCopier);
+    auto copier = [&](int t) {
+        failed[t] = copy_pieces(device, st, spans, count, t, workers, ring.base + kPiece * (size_t)t);
+    };
     for (int t = 1; t < workers; ++t) {
         try {
             threads[t] = std::thread(copier, t);
