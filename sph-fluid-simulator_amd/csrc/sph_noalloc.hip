@@ -285,9 +285,10 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     c16.counts = (uint32_t *)at(L.counts16);
     c16.cstart = (uint32_t *)at(L.cstart16);
     c16.partials = (uint32_t *)at(L.partials16);
-    c16.big = nullptr;
-    c16.big_cap = 0;
+    c16.big = c.big;  // free once the step's cells are in order
+    c16.big_cap = c.big_cap;
     c16.ncells_padded = 65536;
+    c16.unordered = nullptr;
     uint32_t *perm16 = (uint32_t *)at(L.perm16);
     launch_fill_u32(st, c16.counts, 0u, 65536);
     launch_h16_rank(st, a, c16, n);

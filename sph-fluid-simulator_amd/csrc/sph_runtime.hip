@@ -735,9 +735,10 @@ CellArrays cells16(Stateless &S)
     c.counts = (uint32_t *)S.counts16.ptr;
     c.cstart = (uint32_t *)S.cstart16.ptr;
     c.partials = (uint32_t *)S.partials16.ptr;
-    c.big = nullptr;
-    c.big_cap = 0;
+    c.big = (uint32_t *)S.w.big.ptr;  // free once the step's cells are in order
+    c.big_cap = S.w.big_cap;
     c.ncells_padded = 65536;
+    c.unordered = nullptr;
     return c;
 }
 
