@@ -570,7 +570,7 @@ Batch::GraphKey Batch::graph_key() const
                     at(c.cstart),  at(c.partials), at(c.big),     at(c.unordered), at(S.params),   at(S.tasks),
                     at(p.nparts),  at(p.off),    at(p.measure),  at(p.total),     at(p.tasks),
                     at(p.queue),   at(p.buf),    at(p.done),      at(p.walk),      at(p.own),      at(l.list),
-                    at(l.count),   at(w.force.ptr), c.big_cap,    c.ncells_padded, S.nwaves,       S.staged,
+                    at(l.count),   at(w.force.ptr), c.big_cap,    c.ncells_padded, S.nwaves,       (uint64_t)S.staged | (uint64_t)S.fine << 1,
                     p.nscenes,    p.cap,           l.stride,        (uint64_t)w.stencil_block,
                     keep_force};
 }

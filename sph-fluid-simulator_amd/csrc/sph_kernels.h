@@ -83,11 +83,17 @@ struct SceneSet {
     const WaveTask *tasks;     // one per 64-slot wave
     uint32_t nwaves;
     bool staged;               // some scene's walks may be staged (stageable)
+    bool fine;                 // none is, but some scene's on a finer grid (fine_stageable)
 };
 
 // Whether short walks of a scene are staged in LDS (k_plan_list): cells of
 // h or larger, and the per-lane walk not forced.
 SPH_HD inline bool stageable(const StepParams &P) { return P.reach == 1 && P.lane_walk == 0u; }
+// Or, in a launch without such a scene, those on cells of h / 2 to h (k_plan_fine).
+SPH_HD inline bool fine_stageable(const StepParams &P)
+{
+    return P.reach == 2 && P.lane_walk == 0u && P.h2 <= 1.0f;
+}
 
 // Spare part tasks of a scene of `waves` wave tasks (beyond one per task):
 // the scene's part size is its total walk over this room, so a scene

@@ -1288,17 +1288,96 @@ struct Stage {
     float term[kStageTerms][64];
 };
 
-// *src of each lane into dst + lane (dst wave-uniform), without registers
-// in between; the caller waits for vmcnt.
-__device__ inline void load_to_lds(const float *src, float *dst)
+// Coordinates of the records [first, first + n), first and n wave-uniform,
+// into LDS, without registers in between; the caller waits for vmcnt.
+// The lanes' offsets stay 32 bits beside a scalar address: one instruction
+// a load (64-bit vector addresses were a quarter of k_plan_fine).
+__device__ inline void load_to_lds(const float4 *__restrict__ pos, uint32_t first, uint32_t n, float *x, float *y,
+                                   float *z)
 {
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)src,
-                                     (__attribute__((address_space(3))) void *)dst, 4, 0, 0);
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t k = 0; k < n; k += 64u) {
+        const char *base = reinterpret_cast<const char *>(pos + (first + k));
+        if (lane < n - k) {
+            auto load = [&](uint32_t at, float *dst) {
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(base + (lane * 16u + at)),
+                                                 (__attribute__((address_space(3))) void *)(dst + k), 4, 0, 0);
+            };
+            load(0u, x);
+            load(4u, y);
+            load(8u, z);
+        }
+    }
 }
 
 struct __attribute__((packed, aligned(4))) Bounds4 {
     uint32_t v[4];
 };
+
+// The end of a staged task: its lanes' densities, and how the force pass
+// walks it where the lists (`listed` entries, or kNoList for any) don't do.
+__device__ inline void finish_staged(const uint32_t *__restrict__ cstart, uint32_t cc, bool active, bool any_slow,
+                                     const StepParams &P, const PartPlan &pp, const NeighborLists &nl, uint32_t task,
+                                     uint32_t s, float4 pi, const float4 *__restrict__ vel, float acc, uint32_t listed,
+                                     float *__restrict__ rho, float4 *__restrict__ posR, float4 *__restrict__ velR)
+{
+    UnionRows U{0, 0, 0, 0, 0, 0, false};
+    uint32_t ucount = 0, unused = kNoOwn, w = kWalkUnion | kWalkSummed;
+    if (__any(listed == kNoList) && plan_union(cstart, cc, active, P, U, ucount, unused) && !any_slow)
+        w |= kWalkBox | (U.segments ? kWalkSegments : 0u);
+    if (active) {
+        const float4 vs = vel[s];
+        const float d = acc + P.self_dens;
+        rho[s] = d;
+        posR[s] = make_float4(pi.x, pi.y, pi.z, 0.5f / d);
+        velR[s] = make_float4(vs.x, vs.y, vs.z, P.gas * (d - P.rho0));
+        nl.count[s] = listed;
+    }
+    if ((threadIdx.x & 63u) == 0u) {
+        pp.measure[task] = 0u;
+        pp.walk[2u * task] = make_int4(U.x0, U.x1, U.y0, U.y1);
+        pp.walk[2u * task + 1u] = make_int4(U.z0, U.z1, (int)ucount, (int)w);
+    }
+}
+
+// The walk, and its length, of a task left to k_density.  own: the lanes'
+// own candidate counts, or kNoOwn.
+__device__ inline void plan_walk(const uint32_t *__restrict__ cstart, uint32_t cc, bool active, bool any_slow,
+                                 const StepParams &P, const SceneSet &S, const PartPlan &pp, uint32_t task, uint32_t s,
+                                 uint32_t own)
+{
+    UnionRows U;
+    uint32_t ucount = 0, len, fresh = kNoOwn;
+    const bool use_union = plan_union(cstart, cc, active, P, U, ucount, fresh) && !any_slow;
+    if (__builtin_amdgcn_readfirstlane(own) == kNoOwn)  // wave-uniform
+        own = fresh;
+    if (!use_union && __builtin_amdgcn_readfirstlane(own) == kNoOwn)
+        own = stencil_length(cstart, cc, P);
+    const uint32_t longest = (uint32_t)wave_max_i((int)own);  // kNoOwn (-1): all lanes in one cell
+    if (longest <= kShortWalk) {
+        len = 0;  // left whole: it records neighbour lists, which the force pass then visits
+    } else if (use_union) {
+        len = ucount;
+    } else {
+        // Per-lane walks cost several times as much per candidate as the
+        // union walk (divergent gathers, no shared loads), so they count
+        // several times toward the part size; with slow lanes (m_ij counted
+        // from the 27 buckets per neighbour, the wave waiting on them) more
+        // again.
+        len = longest * (any_slow ? kSlowWalkWeight : kLaneWalkWeight);
+    }
+    if (!use_union && active)
+        pp.own[s] = own;
+    if ((threadIdx.x & 63u) == 0u) {
+        pp.walk[2u * task] = make_int4(U.x0, U.x1, U.y0, U.y1);
+        pp.walk[2u * task + 1u] = make_int4(
+            U.z0, U.z1, (int)ucount, use_union ? (int)(kWalkUnion | kWalkBox | (U.segments ? kWalkSegments : 0u)) : 0);
+        pp.measure[task] = len;
+        // only walks that may be split count toward the scene's part size
+        if (len > kPartCandidates)
+            atomicAdd(&pp.total[kTotalSlots * S.tasks[task].scene + task % kTotalSlots], (unsigned long long)len);
+    }
+}
 
 // Plans the walk of every wave task and, where all of its lanes' stencils
 // are short, runs its density pass at once: one block of three waves per
@@ -1411,13 +1490,7 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
                 const uint32_t bs = (uint32_t)__builtin_amdgcn_readlane((int)b, (int)e);
                 const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)len, (int)e);
                 const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, (int)e);
-                for (uint32_t k = 0; k < n; k += 64u)
-                    if (k + lane < n) {
-                        const float4 *q = pos + bs + k + lane;
-                        load_to_lds(&q->x, &stage.x[o + k]);
-                        load_to_lds(&q->y, &stage.y[o + k]);
-                        load_to_lds(&q->z, &stage.z[o + k]);
-                    }
+                load_to_lds(pos, bs, n, &stage.x[o], &stage.y[o], &stage.z[o]);
             }
             for (uint32_t k = 0; k < gap; ++k)  // behind a row: candidates that never pass
                 stage.x[off + len + k] = __builtin_inff();
@@ -1642,61 +1715,271 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
             } else {
                 acc = stage.term[0][lane];
             }
-            UnionRows U{0, 0, 0, 0, 0, 0, false};
-            uint32_t ucount = 0, unused = kNoOwn, w = kWalkUnion | kWalkSummed;
-            if (!listing && plan_union(cstart, cc, active, P, U, ucount, unused) && !any_slow)
-                w |= kWalkBox | (U.segments ? kWalkSegments : 0u);  // for the force pass
-            if (active) {
-                const float4 vs = vel[s];
-                const float d = acc + P.self_dens;
-                rho[s] = d;
-                posR[s] = make_float4(pi.x, pi.y, pi.z, 0.5f / d);
-                velR[s] = make_float4(vs.x, vs.y, vs.z, P.gas * (d - P.rho0));
-                nl.count[s] = listing ? all : kNoList;
-                if (COUNT)
-                    count[s] = layers[0].counted[lane] + layers[1].counted[lane] + layers[2].counted[lane];
-            }
-            if (lane == 0u) {
-                pp.measure[task] = 0u;
-                pp.walk[2u * task] = make_int4(U.x0, U.x1, U.y0, U.y1);
-                pp.walk[2u * task + 1u] = make_int4(U.z0, U.z1, (int)ucount, (int)w);
-            }
+            if (COUNT && active)
+                count[s] = layers[0].counted[lane] + layers[1].counted[lane] + layers[2].counted[lane];
+            finish_staged(cstart, cc, active, any_slow, P, pp, nl, task, s, pi, vel, acc, listing ? all : kNoList, rho,
+                          posR, velR);
             return;
         }
     }
     if (lz != 0)
         return;
-    UnionRows U;
-    uint32_t ucount = 0, len, fresh = kNoOwn;
-    const bool use_union = plan_union(cstart, cc, active, P, U, ucount, fresh) && !any_slow;
-    if (__builtin_amdgcn_readfirstlane(own) == kNoOwn)  // wave-uniform
-        own = fresh;
-    if (!use_union && __builtin_amdgcn_readfirstlane(own) == kNoOwn)
-        own = stencil_length(cstart, cc, P);
-    const uint32_t longest = (uint32_t)wave_max_i((int)own);  // kNoOwn (-1): all lanes in one cell
-    if (longest <= kShortWalk) {
-        len = 0;  // left whole: it records neighbour lists, which the force pass then visits
-    } else if (use_union) {
-        len = ucount;
-    } else {
-        // Per-lane walks cost several times as much per candidate as the
-        // union walk (divergent gathers, no shared loads), so they count
-        // several times toward the part size; with slow lanes (m_ij counted
-        // from the 27 buckets per neighbour, the wave waiting on them) more
-        // again.
-        len = longest * (any_slow ? kSlowWalkWeight : kLaneWalkWeight);
+    plan_walk(cstart, cc, active, any_slow, P, S, pp, task, s, own);
+}
+
+// The same for cells of h / 2 to h (reach 2), where a stencil is 25 rows of a
+// few cells: one wave per task, which copies layer after layer of its lanes'
+// rows to LDS, the next one while it walks one.  The bounds of the lanes' 25
+// cut rows are read at once beforehand, and a layer's neighbours are listed
+// after the next layer has arrived, so that no load waits for the list's
+// stores.  Planned and walked here, and the few tasks left over in k_density,
+// against planned and walked from memory there: 262 thousand particles 63 + 14
+// us and 26 + 86, a million 158 + 16 and 30 + 150.  What bounds it is the
+// arithmetic (57 M vector instructions, two thirds of the issue slots at the
+// twelve waves a CU that registers and LDS allow).
+// Tasks with a row of more than kFineRow candidates in a lane's stencil, or
+// with more than fit a layer's room, are left to k_density.
+constexpr uint32_t kFineCap = 448;  // candidates of a layer (64 slots and 4 cells in each of 5 rows: about 350)
+constexpr uint32_t kFineGap = 2;    // behind a row: three candidates are tested at a time
+constexpr uint32_t kFineRow = 30, kFineRowBits = 5, kFineAtBits = 9;
+constexpr uint32_t kFineSegs = 12;  // runs of lanes in one x-row of cells, 5 rows each per layer
+struct FineStage {
+    float x[2][kFineCap + 3], y[2][kFineCap + 3], z[2][kFineCap + 3];  // three are read ahead
+    uint32_t slot[5][64], at[5][64];  // of a row's first candidate
+    uint32_t x0[kFineSegs], x1[kFineSegs], yz[kFineSegs];
+};
+static_assert(kFineCap <= 1u << kFineAtBits && kFineRow < 1u << kFineRowBits && kFineRowBits + kFineAtBits <= 16, "");
+
+template <bool COUNT>
+__global__ __launch_bounds__(64) void k_plan_fine(
+    const float4 *__restrict__ pos, const float4 *__restrict__ vel, const uint32_t *__restrict__ cellcB,
+    const uint32_t *__restrict__ cstart, float *__restrict__ rho, float4 *__restrict__ posR,
+    float4 *__restrict__ velR, SceneSet S, PartPlan pp, NeighborLists nl, uint32_t *__restrict__ count)
+{
+    __shared__ FineStage stage;
+    const uint32_t lane = threadIdx.x;
+    const uint32_t task = xcd_block();
+    if (task >= S.nwaves)
+        return;
+    if (task == 0u && lane < 3u)
+        pp.queue[lane] = 0u;  // as in k_plan_list
+    Lane L;
+    bool active;
+    wave_task(S, task, L, active);
+    const StepParams P = *L.P;
+    const uint32_t s = L.slot;
+    const uint32_t cc = cellcB[s];
+    const bool slow = (cc & kSlowBit) != 0u;
+    const bool any_slow = __any(slow);
+    const uint64_t heads = segment_heads(cc, active);
+    const uint32_t nseg = (uint32_t)__builtin_popcountll(heads);
+    if (fine_stageable(P) && nl.list && nseg <= kFineSegs) {  // wave-uniform
+        const float4 pi = pos[s];
+        const int gx = cell_x(cc), gy = cell_y(cc), gz = cell_z(cc);
+        const uint32_t nact = (uint32_t)__builtin_popcountll(__ballot(active));
+        const uint32_t seg = active ? (uint32_t)__builtin_popcountll(heads & ((2ull << lane) - 1ull)) - 1u : 0u;
+        if ((heads >> lane & 1ull) != 0ull) {
+            stage.x0[seg] = (uint32_t)gx;
+            stage.yz[seg] = cc & ~kSlowBit & ~2047u;
+        }
+        if (active && (lane + 1u == nact || ((heads >> 1) >> lane & 1ull)))
+            stage.x1[seg] = (uint32_t)gx;
+        wave_lds_sync();
+        // All the bounds, 60 loads, without a branch between them (a branch
+        // each, and the compiler waits in each): rows that are out read cell 0.
+        const uint32_t nx = (uint32_t)P.nx, plane = nx * (uint32_t)P.ny;
+        // lane: row lane % 5 of segment lane / 5, in each layer
+        const bool owner = lane < 5u * nseg;
+        uint32_t b[5], len[5];
+        {
+            const uint32_t k = owner ? lane / 5u : 0u, c = stage.yz[k];
+            const int y = cell_y(c) + (int)(lane % 5u) - 2, z0 = cell_z(c) - 2;
+            const uint32_t row = P.cell_base + nx * (uint32_t)y + plane * (uint32_t)z0;
+            const uint32_t xa = (uint32_t)max((int)stage.x0[k] - 2, 0);
+            const uint32_t xb = (uint32_t)min((int)stage.x1[k] + 2, P.nx - 1) + 1u;
+            const bool in = owner && y >= 0 && y < P.ny;
+#pragma unroll
+            for (int l = 0; l < 5; ++l) {
+                const bool at = in && z0 + l >= 0 && z0 + l < P.nz;
+                const uint32_t r0 = row + plane * (uint32_t)l;
+                b[l] = cstart[at ? r0 + xa : 0u];
+                len[l] = cstart[at ? r0 + xb : 0u];
+            }
+        }
+        // The lane's cut rows: first candidate and count.  A cell whose
+        // squared gaps add up to the reach or more is out (see LaneTrim).
+        const LaneTrim T = lane_trim(pi, cc, P);
+        auto square = [](float g) { return g * g; };
+        const float left1 = square(trim_gap(-1, T.fx)), left2 = square(trim_gap(-2, T.fx));
+        const float right1 = square(trim_gap(1, T.fx)), right2 = square(trim_gap(2, T.fx));
+        uint32_t from[5][5], n[5][5];
+        {
+            const uint32_t row = P.cell_base + nx * (uint32_t)(gy - 2) + plane * (uint32_t)(gz - 2);
+            const int last = P.nx - 1;
+#pragma unroll
+            for (int l = 0; l < 5; ++l)
+#pragma unroll
+                for (int r = 0; r < 5; ++r) {
+                    const int y = gy + r - 2, z = gz + l - 2;
+                    const float rem = T.r2 - (square(trim_gap(r - 2, T.fy)) + square(trim_gap(l - 2, T.fz)));
+                    const bool in = rem > 0.0f && y >= 0 && y < P.ny && z >= 0 && z < P.nz;
+                    const int xa = max(gx - (left1 < rem ? 1 : 0) - (left2 < rem ? 1 : 0), 0);
+                    const int xb = min(gx + (right1 < rem ? 1 : 0) + (right2 < rem ? 1 : 0), last);
+                    const uint32_t r0 = row + nx * (uint32_t)r + plane * (uint32_t)l;
+                    from[l][r] = cstart[in ? r0 + (uint32_t)xa : 0u];
+                    n[l][r] = cstart[in ? r0 + (uint32_t)xb + 1u : 0u];
+                }
+        }
+#pragma unroll
+        for (int l = 0; l < 5; ++l) {
+            len[l] -= b[l];  // 0 for a row that is out
+#pragma unroll
+            for (int r = 0; r < 5; ++r)
+                n[l][r] -= from[l][r];
+        }
+        bool ok = true;
+#pragma unroll
+        for (int l = 0; l < 5; ++l) {
+            const uint32_t room = owner ? len[l] + kFineGap : 0u;
+            const uint32_t end = wave_inclusive_scan(room);
+            ok = ok && (uint32_t)__builtin_amdgcn_readlane((int)end, 63) <= kFineCap;
+            stage.slot[l][lane] = b[l];
+            stage.at[l][lane] = end - room;
+        }
+        wave_lds_sync();
+        // each row in 16 bits: count, offset of its first candidate
+        uint32_t rows[13] = {}, own = 0;
+#pragma unroll
+        for (int l = 0; l < 5; ++l)
+#pragma unroll
+            for (int r = 0; r < 5; ++r) {
+                const uint32_t off = n[l][r] ? from[l][r] - stage.slot[l][5u * seg + (uint32_t)r] : 0u;
+                ok = ok && n[l][r] <= kFineRow;
+                own += n[l][r];
+                rows[(5 * l + r) / 2] |= (n[l][r] | off << kFineRowBits) << (((5 * l + r) & 1) * 16);
+            }
+        if (__all(ok) && (uint32_t)wave_max_i((int)own) <= kShortWalk) {
+            auto stage_layer = [&](int l) {
+                const int buf = l & 1;
+                const uint32_t at0 = stage.at[l][lane];
+                for (uint32_t e = 0; e < 5u * nseg; ++e) {
+                    const uint32_t first = (uint32_t)__builtin_amdgcn_readlane((int)b[l], (int)e);
+                    const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)len[l], (int)e);
+                    const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)at0, (int)e);
+                    load_to_lds(pos, first, m, &stage.x[buf][o], &stage.y[buf][o], &stage.z[buf][o]);
+                }
+                if (owner)
+#pragma unroll
+                    for (uint32_t k = 0; k < kFineGap; ++k)  // candidates that never pass
+                        stage.x[buf][at0 + len[l] + k] = __builtin_inff();
+            };
+            auto arrived = [] {
+                __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt 0
+                wave_lds_sync();
+            };
+            const float h2 = in_vgpr(P.h2), mp6 = in_vgpr(P.mp6);
+            auto test = [&](float x, float y, float z) {  // h <= 1: clamping to 1 changes nothing
+                float dx, dy, dz;
+                return positive<true>(h2 - dist2_ref(pi, make_float4(x, y, z, 0.0f), dx, dy, dz));
+            };
+            RefCell ci{0, 0, 0};
+            if (slow)
+                ci = ref_cell(pi, P);
+            float acc = 0.0f, slow_acc = 0.0f;
+            uint32_t nn = 0, cnt = 0;
+            uint32_t *lp = nl.list + s;
+            stage_layer(0);
+            arrived();
+#pragma unroll
+            for (int l = 0; l < 5; ++l) {
+                const int buf = l & 1;
+                if (l < 4)
+                    stage_layer(l + 1);
+                uint32_t bits[5];
+#pragma unroll
+                for (int r = 0; r < 5; ++r) {
+                    const uint32_t row = rows[(5 * l + r) / 2] >> (((5 * l + r) & 1) * 16);
+                    const uint32_t m = row & ((1u << kFineRowBits) - 1u);
+                    const uint32_t off = row >> kFineRowBits & ((1u << kFineAtBits) - 1u);
+                    bits[r] = 0u;
+                    if (m == 0u)
+                        continue;
+                    const uint32_t at = stage.at[l][5u * seg + (uint32_t)r] + off;
+                    const float *px = &stage.x[buf][at], *py = &stage.y[buf][at], *pz = &stage.z[buf][at];
+                    // only the middle row holds the particle itself
+                    const uint32_t self = l == 2 && r == 2 ? s - stage.slot[l][5u * seg + (uint32_t)r] - off : 0u;
+                    float x[3], y[3], z[3];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        x[i] = px[i];
+                        y[i] = py[i];
+                        z[i] = pz[i];
+                    }
+                    uint32_t k = 0;
+                    do {
+                        float t[3];
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) {
+                            t[i] = test(x[i], y[i], z[i]);
+                            if (l == 2 && r == 2)
+                                t[i] = k + (uint32_t)i != self ? t[i] : 0.0f;
+                        }
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) {  // the next three, meanwhile
+                            x[i] = px[k + 3u + (uint32_t)i];
+                            y[i] = py[k + 3u + (uint32_t)i];
+                            z[i] = pz[k + 3u + (uint32_t)i];
+                        }
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) {
+                            acc = acc + mp6 * ((t[i] * t[i]) * t[i]);
+                            bits[r] = __builtin_amdgcn_alignbit(bits[r], 0u - __float_as_uint(t[i]), 31u);  // << 1 | (t > 0)
+                        }
+                        k += 3u;
+                    } while (k < m);
+                    bits[r] <<= 32u - k;  // the first on top (k <= 30)
+                }
+                if (l < 4)
+                    arrived();
+#pragma unroll
+                for (int r = 0; r < 5; ++r) {
+                    if (bits[r] == 0u)
+                        continue;
+                    const uint32_t row = rows[(5 * l + r) / 2] >> (((5 * l + r) & 1) * 16);
+                    const uint32_t off = row >> kFineRowBits & ((1u << kFineAtBits) - 1u);
+                    const uint32_t j0 = stage.slot[l][5u * seg + (uint32_t)r] + off;
+                    do {
+                        const uint32_t k = (uint32_t)__builtin_clz(bits[r]);
+                        bits[r] &= ~(0x80000000u >> k);
+                        if (nn < kListMax) {
+                            *lp = j0 + k;
+                            lp += nl.stride;
+                        }
+                        ++nn;
+                        if (any_slow) {
+                            // summed again, each with its m_ij
+                            const uint32_t at = stage.at[l][5u * seg + (uint32_t)r] + off + k;
+                            const float t = test(stage.x[buf][at], stage.y[buf][at], stage.z[buf][at]);
+                            int mult = 1;
+                            if (slow)
+                                mult = bucket_multiplicity(ci.x, ci.y, ci.z, __float_as_uint(pos[j0 + k].w) & 0xFFFFu);
+                            slow_acc += (float)mult * (mp6 * ((t * t) * t));
+                            cnt += (uint32_t)mult - 1u;
+                        }
+                    } while (bits[r] != 0u);
+                }
+            }
+            if (any_slow)
+                acc = slow_acc;
+            if (COUNT && active)
+                count[s] = nn + cnt;
+            const bool listing = !__any(nn > kListMax);
+            finish_staged(cstart, cc, active, any_slow, P, pp, nl, task, s, pi, vel, acc, listing ? nn : kNoList, rho,
+                          posR, velR);
+            return;
+        }
     }
-    if (!use_union && active)
-        pp.own[s] = own;
-    if (lane == 0u) {
-        pp.walk[2u * task] = make_int4(U.x0, U.x1, U.y0, U.y1);
-        pp.walk[2u * task + 1u] = make_int4(
-            U.z0, U.z1, (int)ucount, use_union ? (int)(kWalkUnion | kWalkBox | (U.segments ? kWalkSegments : 0u)) : 0);
-        pp.measure[task] = len;
-        // only walks that may be split count toward the scene's part size
-        if (len > kPartCandidates)
-            atomicAdd(&pp.total[kTotalSlots * S.tasks[task].scene + task % kTotalSlots], (unsigned long long)len);
-    }
+    plan_walk(cstart, cc, active, any_slow, P, S, pp, task, s, kNoOwn);
 }
 
 // Parts per wave task, queued: the part size grows beyond kPartCandidates
@@ -1750,9 +2033,15 @@ void launch_plan_parts(hipStream_t st, const ParticleArrays &a, const CellArrays
         SPH_LAUNCH_PLAN(true, true);
     else if (S.staged)
         SPH_LAUNCH_PLAN(true, false);
-    else
+    else if (!S.fine)
         SPH_LAUNCH_PLAN(false, false);  // counts nothing itself
 #undef SPH_LAUNCH_PLAN
+    else if (count)
+        hipLaunchKernelGGL((k_plan_fine<true>), grid, dim3(64), 0, st, a.posB, a.velB, a.cellcB, c.cstart, a.rhoB,
+                           a.posR, a.velR, S, pp, nl, count);
+    else
+        hipLaunchKernelGGL((k_plan_fine<false>), grid, dim3(64), 0, st, a.posB, a.velB, a.cellcB, c.cstart, a.rhoB,
+                           a.posR, a.velR, S, pp, nl, count);
     hipLaunchKernelGGL(k_queue_parts, dim3(blocks_for(std::max(1u, S.nwaves))), dim3(kBlock), 0, st, S, pp);
 }
 

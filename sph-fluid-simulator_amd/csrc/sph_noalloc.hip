@@ -249,6 +249,7 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     set.tasks = dtasks;
     set.nwaves = L.nwaves;
     set.staged = stageable(P);
+    set.fine = fine_stageable(P);
 
     PartPlan pp;
     pp.nparts = (uint32_t *)at(L.nparts);

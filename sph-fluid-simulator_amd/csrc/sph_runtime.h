@@ -100,7 +100,7 @@ struct Workspace {
     uint32_t big_cap = 0;
     uint32_t nwaves = 0;
     uint32_t nscenes = 0;
-    bool staged = false;  // SceneSet::staged of the current scene set
+    bool staged = false, fine = false;  // SceneSet's of the current scene set
     std::vector<WaveTask> host_tasks;  // what `tasks` holds
     uint32_t part_cap = 0;  // part-task capacity of the current scene set
     int stencil_block = kStencilBlock;  // threads per block of the density and force passes

@@ -503,9 +503,12 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
         return hip_fail(e, "scene table upload");
     }
     host_tasks = std::move(t);
-    staged = false;
-    for (const StepParams &sp : scenes)
+    staged = fine = false;
+    for (const StepParams &sp : scenes) {
         staged = staged || stageable(sp);
+        fine = fine || fine_stageable(sp);
+    }
+    fine = fine && !staged;
     nwaves = (uint32_t)host_tasks.size();
     nscenes = (uint32_t)scenes.size();
     part_cap = (uint32_t)cap;
@@ -549,6 +552,7 @@ SceneSet Workspace::scene_set() const
     S.tasks = (const WaveTask *)tasks.ptr;
     S.nwaves = nwaves;
     S.staged = staged;
+    S.fine = fine;
     return S;
 }
 
