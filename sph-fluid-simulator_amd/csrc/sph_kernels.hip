@@ -1340,11 +1340,43 @@ __device__ inline void finish_staged(const uint32_t *__restrict__ cstart, uint32
     }
 }
 
+// The lane's cut rows in layer l (0 .. 4) of a grid of reach 2: first
+// candidates, and behind the last ones (the same for a row that is out).  A
+// cell whose squared gaps add up to the reach or more is out (see LaneTrim).
+// Ten loads without a branch between them (a branch each, and the compiler
+// waits in each): rows that are out read cell 0.
+__device__ inline void cut_rows(const uint32_t *__restrict__ cstart, uint32_t cc, const LaneTrim &T,
+                                const StepParams &P, int l, uint32_t (&from)[5], uint32_t (&to)[5])
+{
+    const int gx = cell_x(cc), gy = cell_y(cc), z = cell_z(cc) + l - 2;
+    auto square = [](float g) { return g * g; };
+    const float left1 = square(trim_gap(-1, T.fx)), left2 = square(trim_gap(-2, T.fx));
+    const float right1 = square(trim_gap(1, T.fx)), right2 = square(trim_gap(2, T.fx));
+    const uint32_t nx = (uint32_t)P.nx;
+    const uint32_t row = P.cell_base + nx * ((uint32_t)(gy - 2) + (uint32_t)P.ny * (uint32_t)z);
+    const bool layer = z >= 0 && z < P.nz;
+#pragma unroll
+    for (int r = 0; r < 5; ++r) {
+        const int y = gy + r - 2;
+        const float rem = T.r2 - (square(trim_gap(r - 2, T.fy)) + square(trim_gap(l - 2, T.fz)));
+        const bool in = rem > 0.0f && layer && y >= 0 && y < P.ny;
+        const int xa = max(gx - (left1 < rem ? 1 : 0) - (left2 < rem ? 1 : 0), 0);
+        const int xb = min(gx + (right1 < rem ? 1 : 0) + (right2 < rem ? 1 : 0), P.nx - 1);
+        const uint32_t r0 = row + nx * (uint32_t)r;
+        from[r] = cstart[in ? r0 + (uint32_t)xa : 0u];
+        to[r] = cstart[in ? r0 + (uint32_t)xb + 1u : 0u];
+    }
+}
+
 // The walk, and its length, of a task left to k_density.  own: the lanes'
-// own candidate counts, or kNoOwn.
+// own candidate counts, or kNoOwn.  longest: on a grid of reach 2, the
+// largest count of a lane's cut rows, or kNoOwn.
+// A task is left whole by the same count in every launch (k_plan_fine's tasks
+// are planned here where scenes on other grids share the launch), so that a
+// scene's sums don't depend on its company.
 __device__ inline void plan_walk(const uint32_t *__restrict__ cstart, uint32_t cc, bool active, bool any_slow,
                                  const StepParams &P, const SceneSet &S, const PartPlan &pp, uint32_t task, uint32_t s,
-                                 uint32_t own)
+                                 uint32_t own, const float4 *__restrict__ pos, uint32_t longest_cut)
 {
     UnionRows U;
     uint32_t ucount = 0, len, fresh = kNoOwn;
@@ -1354,7 +1386,24 @@ __device__ inline void plan_walk(const uint32_t *__restrict__ cstart, uint32_t c
     if (!use_union && __builtin_amdgcn_readfirstlane(own) == kNoOwn)
         own = stencil_length(cstart, cc, P);
     const uint32_t longest = (uint32_t)wave_max_i((int)own);  // kNoOwn (-1): all lanes in one cell
-    if (longest <= kShortWalk) {
+    uint32_t shortness = longest;
+    if (fine_stageable(P)) {
+        shortness = longest_cut;
+        if (longest_cut == kNoOwn) {
+            const LaneTrim T = lane_trim(pos[s], cc, P);
+            uint32_t cut = 0;
+#pragma unroll 1
+            for (int l = 0; l < 5; ++l) {
+                uint32_t from[5], to[5];
+                cut_rows(cstart, cc, T, P, l, from, to);
+#pragma unroll
+                for (int r = 0; r < 5; ++r)
+                    cut += to[r] - from[r];
+            }
+            shortness = (uint32_t)wave_max_i((int)cut);
+        }
+    }
+    if (shortness <= kShortWalk) {
         len = 0;  // left whole: it records neighbour lists, which the force pass then visits
     } else if (use_union) {
         len = ucount;
@@ -1724,7 +1773,7 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
     }
     if (lz != 0)
         return;
-    plan_walk(cstart, cc, active, any_slow, P, S, pp, task, s, own);
+    plan_walk(cstart, cc, active, any_slow, P, S, pp, task, s, own, pos, kNoOwn);
 }
 
 // The same for cells of h / 2 to h (reach 2), where a stencil is 25 rows of a
@@ -1773,9 +1822,10 @@ __global__ __launch_bounds__(64) void k_plan_fine(
     const bool any_slow = __any(slow);
     const uint64_t heads = segment_heads(cc, active);
     const uint32_t nseg = (uint32_t)__builtin_popcountll(heads);
+    uint32_t longest = kNoOwn;
     if (fine_stageable(P) && nl.list && nseg <= kFineSegs) {  // wave-uniform
         const float4 pi = pos[s];
-        const int gx = cell_x(cc), gy = cell_y(cc), gz = cell_z(cc);
+        const int gx = cell_x(cc);
         const uint32_t nact = (uint32_t)__builtin_popcountll(__ballot(active));
         const uint32_t seg = active ? (uint32_t)__builtin_popcountll(heads & ((2ull << lane) - 1ull)) - 1u : 0u;
         if ((heads >> lane & 1ull) != 0ull) {
@@ -1785,8 +1835,7 @@ __global__ __launch_bounds__(64) void k_plan_fine(
         if (active && (lane + 1u == nact || ((heads >> 1) >> lane & 1ull)))
             stage.x1[seg] = (uint32_t)gx;
         wave_lds_sync();
-        // All the bounds, 60 loads, without a branch between them (a branch
-        // each, and the compiler waits in each): rows that are out read cell 0.
+        // All the bounds, 60 loads in flight together
         const uint32_t nx = (uint32_t)P.nx, plane = nx * (uint32_t)P.ny;
         // lane: row lane % 5 of segment lane / 5, in each layer
         const bool owner = lane < 5u * nseg;
@@ -1806,37 +1855,22 @@ __global__ __launch_bounds__(64) void k_plan_fine(
                 len[l] = cstart[at ? r0 + xb : 0u];
             }
         }
-        // The lane's cut rows: first candidate and count.  A cell whose
-        // squared gaps add up to the reach or more is out (see LaneTrim).
-        const LaneTrim T = lane_trim(pi, cc, P);
-        auto square = [](float g) { return g * g; };
-        const float left1 = square(trim_gap(-1, T.fx)), left2 = square(trim_gap(-2, T.fx));
-        const float right1 = square(trim_gap(1, T.fx)), right2 = square(trim_gap(2, T.fx));
         uint32_t from[5][5], n[5][5];
-        {
-            const uint32_t row = P.cell_base + nx * (uint32_t)(gy - 2) + plane * (uint32_t)(gz - 2);
-            const int last = P.nx - 1;
+        const LaneTrim T = lane_trim(pi, cc, P);
 #pragma unroll
-            for (int l = 0; l < 5; ++l)
-#pragma unroll
-                for (int r = 0; r < 5; ++r) {
-                    const int y = gy + r - 2, z = gz + l - 2;
-                    const float rem = T.r2 - (square(trim_gap(r - 2, T.fy)) + square(trim_gap(l - 2, T.fz)));
-                    const bool in = rem > 0.0f && y >= 0 && y < P.ny && z >= 0 && z < P.nz;
-                    const int xa = max(gx - (left1 < rem ? 1 : 0) - (left2 < rem ? 1 : 0), 0);
-                    const int xb = min(gx + (right1 < rem ? 1 : 0) + (right2 < rem ? 1 : 0), last);
-                    const uint32_t r0 = row + nx * (uint32_t)r + plane * (uint32_t)l;
-                    from[l][r] = cstart[in ? r0 + (uint32_t)xa : 0u];
-                    n[l][r] = cstart[in ? r0 + (uint32_t)xb + 1u : 0u];
-                }
-        }
+        for (int l = 0; l < 5; ++l)
+            cut_rows(cstart, cc, T, P, l, from[l], n[l]);
+        uint32_t own = 0;
 #pragma unroll
         for (int l = 0; l < 5; ++l) {
             len[l] -= b[l];  // 0 for a row that is out
 #pragma unroll
-            for (int r = 0; r < 5; ++r)
+            for (int r = 0; r < 5; ++r) {
                 n[l][r] -= from[l][r];
+                own += n[l][r];
+            }
         }
+        longest = (uint32_t)wave_max_i((int)own);
         bool ok = true;
 #pragma unroll
         for (int l = 0; l < 5; ++l) {
@@ -1848,17 +1882,16 @@ __global__ __launch_bounds__(64) void k_plan_fine(
         }
         wave_lds_sync();
         // each row in 16 bits: count, offset of its first candidate
-        uint32_t rows[13] = {}, own = 0;
+        uint32_t rows[13] = {};
 #pragma unroll
         for (int l = 0; l < 5; ++l)
 #pragma unroll
             for (int r = 0; r < 5; ++r) {
                 const uint32_t off = n[l][r] ? from[l][r] - stage.slot[l][5u * seg + (uint32_t)r] : 0u;
                 ok = ok && n[l][r] <= kFineRow;
-                own += n[l][r];
                 rows[(5 * l + r) / 2] |= (n[l][r] | off << kFineRowBits) << (((5 * l + r) & 1) * 16);
             }
-        if (__all(ok) && (uint32_t)wave_max_i((int)own) <= kShortWalk) {
+        if (__all(ok) && longest <= kShortWalk) {
             auto stage_layer = [&](int l) {
                 const int buf = l & 1;
                 const uint32_t at0 = stage.at[l][lane];
@@ -1979,7 +2012,7 @@ __global__ __launch_bounds__(64) void k_plan_fine(
             return;
         }
     }
-    plan_walk(cstart, cc, active, any_slow, P, S, pp, task, s, kNoOwn);
+    plan_walk(cstart, cc, active, any_slow, P, S, pp, task, s, kNoOwn, pos, longest);
 }
 
 // Parts per wave task, queued: the part size grows beyond kPartCandidates
