@@ -166,8 +166,7 @@ struct NeighborDump {
 };
 
 // Neighbour lists.  The density pass records, for every particle of an
-// unsplit wave task that walks its candidates per lane, the slots of its
-// neighbours (each once, in walk order: rows z-major, then y, slots
+// unsplit wave task, the slots of its neighbours (each once, in walk order: rows z-major, then y, slots
 // ascending) when there are at most kListMax of them; the force pass then
 // visits exactly those slots instead of filtering the stencil again.  The
 // order is the per-lane walk's, so the force sums are the same bit for bit.

@@ -1674,7 +1674,7 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
             __syncthreads();
             const uint32_t n0 = layers[0].listed[lane], n1 = layers[1].listed[lane], n2 = layers[2].listed[lane];
             const uint32_t all = n0 + n1 + n2;
-            const bool listing = !__any(all > kListMax), 
+            const bool listing = !__any(all > kListMax),
                        parallel = !__any(n1 + n2 + 2u > kStageTerms || max(n1, n2) > kStageTerms - 4u);
             auto neighbours = [&](auto visit) {
 #pragma unroll
@@ -1781,13 +1781,15 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
 // rows to LDS, the next one while it walks one.  The bounds of the lanes' 25
 // cut rows are read at once beforehand, and a layer's neighbours are listed
 // after the next layer has arrived, so that no load waits for the list's
-// stores.  Planned and walked here, and the few tasks left over in k_density,
-// against planned and walked from memory there: 262 thousand particles 63 + 14
-// us and 26 + 86, a million 158 + 16 and 30 + 150.  What bounds it is the
-// arithmetic (57 M vector instructions, two thirds of the issue slots at the
-// twelve waves a CU that registers and LDS allow).
-// Tasks with a row of more than kFineRow candidates in a lane's stencil, or
-// with more than fit a layer's room, are left to k_density.
+// stores.  Planned and walked here, against planned and walked from memory in
+// k_density: 262 thousand particles 62 us and 26 + 86, a million 157 and
+// 30 + 150.  What bounds it is the arithmetic (57 M vector instructions, two
+// thirds of the issue slots at the twelve waves a CU that registers and LDS
+// allow).
+// Tasks in many rows (a surface), whose layers don't fit the room, walk from
+// memory here (in k_density, behind the others, the latency of a few hundred
+// such waves was 40 us); those with a row of more than kFineRow candidates in a lane's
+// stencil, or a longer walk, are left to k_density.
 constexpr uint32_t kFineCap = 448;  // candidates of a layer (64 slots and 4 cells in each of 5 rows: about 350)
 constexpr uint32_t kFineGap = 2;    // behind a row: three candidates are tested at a time
 constexpr uint32_t kFineRow = 30, kFineRowBits = 5, kFineAtBits = 9;
@@ -1797,6 +1799,10 @@ struct FineStage {
     uint32_t slot[5][64], at[5][64];  // of a row's first candidate
     uint32_t x0[kFineSegs], x1[kFineSegs], yz[kFineSegs];
 };
+union FineShared {
+    FineStage staged;
+    uint32_t row[2][25][64];  // or each lane's rows: first slot, and count, then which are neighbours
+};
 static_assert(kFineCap <= 1u << kFineAtBits && kFineRow < 1u << kFineRowBits && kFineRowBits + kFineAtBits <= 16, "");
 
 template <bool COUNT>
@@ -1805,7 +1811,8 @@ __global__ __launch_bounds__(64) void k_plan_fine(
     const uint32_t *__restrict__ cstart, float *__restrict__ rho, float4 *__restrict__ posR,
     float4 *__restrict__ velR, SceneSet S, PartPlan pp, NeighborLists nl, uint32_t *__restrict__ count)
 {
-    __shared__ FineStage stage;
+    __shared__ FineShared shared;
+    FineStage &stage = shared.staged;
     const uint32_t lane = threadIdx.x;
     const uint32_t task = xcd_block();
     if (task >= S.nwaves)
@@ -1823,29 +1830,32 @@ __global__ __launch_bounds__(64) void k_plan_fine(
     const uint64_t heads = segment_heads(cc, active);
     const uint32_t nseg = (uint32_t)__builtin_popcountll(heads);
     uint32_t longest = kNoOwn;
-    if (fine_stageable(P) && nl.list && nseg <= kFineSegs) {  // wave-uniform
+    if (fine_stageable(P) && nl.list) {  // wave-uniform
         const float4 pi = pos[s];
         const int gx = cell_x(cc);
+        const bool few = nseg <= kFineSegs;
         const uint32_t nact = (uint32_t)__builtin_popcountll(__ballot(active));
-        const uint32_t seg = active ? (uint32_t)__builtin_popcountll(heads & ((2ull << lane) - 1ull)) - 1u : 0u;
-        if ((heads >> lane & 1ull) != 0ull) {
-            stage.x0[seg] = (uint32_t)gx;
-            stage.yz[seg] = cc & ~kSlowBit & ~2047u;
+        const uint32_t seg = active && few ? (uint32_t)__builtin_popcountll(heads & ((2ull << lane) - 1ull)) - 1u : 0u;
+        if (few) {
+            if ((heads >> lane & 1ull) != 0ull) {
+                stage.x0[seg] = (uint32_t)gx;
+                stage.yz[seg] = cc & ~kSlowBit & ~2047u;
+            }
+            if (active && (lane + 1u == nact || ((heads >> 1) >> lane & 1ull)))
+                stage.x1[seg] = (uint32_t)gx;
         }
-        if (active && (lane + 1u == nact || ((heads >> 1) >> lane & 1ull)))
-            stage.x1[seg] = (uint32_t)gx;
         wave_lds_sync();
         // All the bounds, 60 loads in flight together
         const uint32_t nx = (uint32_t)P.nx, plane = nx * (uint32_t)P.ny;
         // lane: row lane % 5 of segment lane / 5, in each layer
-        const bool owner = lane < 5u * nseg;
+        const bool owner = few && lane < 5u * nseg;
         uint32_t b[5], len[5];
         {
-            const uint32_t k = owner ? lane / 5u : 0u, c = stage.yz[k];
+            const uint32_t k = owner ? lane / 5u : 0u, c = owner ? stage.yz[k] : 0u;
             const int y = cell_y(c) + (int)(lane % 5u) - 2, z0 = cell_z(c) - 2;
             const uint32_t row = P.cell_base + nx * (uint32_t)y + plane * (uint32_t)z0;
-            const uint32_t xa = (uint32_t)max((int)stage.x0[k] - 2, 0);
-            const uint32_t xb = (uint32_t)min((int)stage.x1[k] + 2, P.nx - 1) + 1u;
+            const uint32_t xa = owner ? (uint32_t)max((int)stage.x0[k] - 2, 0) : 0u;
+            const uint32_t xb = owner ? (uint32_t)min((int)stage.x1[k] + 2, P.nx - 1) + 1u : 0u;
             const bool in = owner && y >= 0 && y < P.ny;
 #pragma unroll
             for (int l = 0; l < 5; ++l) {
@@ -1871,7 +1881,7 @@ __global__ __launch_bounds__(64) void k_plan_fine(
             }
         }
         longest = (uint32_t)wave_max_i((int)own);
-        bool ok = true;
+        bool ok = few, short_rows = true;
 #pragma unroll
         for (int l = 0; l < 5; ++l) {
             const uint32_t room = owner ? len[l] + kFineGap : 0u;
@@ -1888,10 +1898,10 @@ __global__ __launch_bounds__(64) void k_plan_fine(
 #pragma unroll
             for (int r = 0; r < 5; ++r) {
                 const uint32_t off = n[l][r] ? from[l][r] - stage.slot[l][5u * seg + (uint32_t)r] : 0u;
-                ok = ok && n[l][r] <= kFineRow;
+                short_rows = short_rows && n[l][r] <= kFineRow;
                 rows[(5 * l + r) / 2] |= (n[l][r] | off << kFineRowBits) << (((5 * l + r) & 1) * 16);
             }
-        if (__all(ok) && longest <= kShortWalk) {
+        if (__all(short_rows) && longest <= kShortWalk) {
             auto stage_layer = [&](int l) {
                 const int buf = l & 1;
                 const uint32_t at0 = stage.at[l][lane];
@@ -1921,85 +1931,150 @@ __global__ __launch_bounds__(64) void k_plan_fine(
             float acc = 0.0f, slow_acc = 0.0f;
             uint32_t nn = 0, cnt = 0;
             uint32_t *lp = nl.list + s;
-            stage_layer(0);
-            arrived();
-#pragma unroll
-            for (int l = 0; l < 5; ++l) {
-                const int buf = l & 1;
-                if (l < 4)
-                    stage_layer(l + 1);
-                uint32_t bits[5];
-#pragma unroll
-                for (int r = 0; r < 5; ++r) {
-                    const uint32_t row = rows[(5 * l + r) / 2] >> (((5 * l + r) & 1) * 16);
-                    const uint32_t m = row & ((1u << kFineRowBits) - 1u);
-                    const uint32_t off = row >> kFineRowBits & ((1u << kFineAtBits) - 1u);
-                    bits[r] = 0u;
-                    if (m == 0u)
-                        continue;
-                    const uint32_t at = stage.at[l][5u * seg + (uint32_t)r] + off;
-                    const float *px = &stage.x[buf][at], *py = &stage.y[buf][at], *pz = &stage.z[buf][at];
-                    // only the middle row holds the particle itself
-                    const uint32_t self = l == 2 && r == 2 ? s - stage.slot[l][5u * seg + (uint32_t)r] - off : 0u;
-                    float x[3], y[3], z[3];
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) {
-                        x[i] = px[i];
-                        y[i] = py[i];
-                        z[i] = pz[i];
-                    }
-                    uint32_t k = 0;
-                    do {
-                        float t[3];
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) {
-                            t[i] = test(x[i], y[i], z[i]);
-                            if (l == 2 && r == 2)
-                                t[i] = k + (uint32_t)i != self ? t[i] : 0.0f;
-                        }
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) {  // the next three, meanwhile
-                            x[i] = px[k + 3u + (uint32_t)i];
-                            y[i] = py[k + 3u + (uint32_t)i];
-                            z[i] = pz[k + 3u + (uint32_t)i];
-                        }
-#pragma unroll
-                        for (int i = 0; i < 3; ++i) {
-                            acc = acc + mp6 * ((t[i] * t[i]) * t[i]);
-                            bits[r] = __builtin_amdgcn_alignbit(bits[r], 0u - __float_as_uint(t[i]), 31u);  // << 1 | (t > 0)
-                        }
-                        k += 3u;
-                    } while (k < m);
-                    bits[r] <<= 32u - k;  // the first on top (k <= 30)
+            // a neighbour, in order: listed; summed again with its m_ij where
+            // the wave has slow lanes
+            auto neighbour = [&](uint32_t j, auto record) {
+                if (nn < kListMax) {
+                    *lp = j;
+                    lp += nl.stride;
                 }
-                if (l < 4)
-                    arrived();
+                ++nn;
+                if (any_slow) {
+                    const float4 q = record();
+                    const float t = test(q.x, q.y, q.z);
+                    int mult = 1;
+                    if (slow)
+                        mult = bucket_multiplicity(ci.x, ci.y, ci.z, __float_as_uint(pos[j].w) & 0xFFFFu);
+                    slow_acc += (float)mult * (mp6 * ((t * t) * t));
+                    cnt += (uint32_t)mult - 1u;
+                }
+            };
+            if (__all(ok)) {
+                stage_layer(0);
+                arrived();
 #pragma unroll
-                for (int r = 0; r < 5; ++r) {
-                    if (bits[r] == 0u)
-                        continue;
-                    const uint32_t row = rows[(5 * l + r) / 2] >> (((5 * l + r) & 1) * 16);
-                    const uint32_t off = row >> kFineRowBits & ((1u << kFineAtBits) - 1u);
-                    const uint32_t j0 = stage.slot[l][5u * seg + (uint32_t)r] + off;
-                    do {
-                        const uint32_t k = (uint32_t)__builtin_clz(bits[r]);
-                        bits[r] &= ~(0x80000000u >> k);
-                        if (nn < kListMax) {
-                            *lp = j0 + k;
-                            lp += nl.stride;
+                for (int l = 0; l < 5; ++l) {
+                    const int buf = l & 1;
+                    if (l < 4)
+                        stage_layer(l + 1);
+                    uint32_t bits[5];
+#pragma unroll
+                    for (int r = 0; r < 5; ++r) {
+                        const uint32_t row = rows[(5 * l + r) / 2] >> (((5 * l + r) & 1) * 16);
+                        const uint32_t m = row & ((1u << kFineRowBits) - 1u);
+                        const uint32_t off = row >> kFineRowBits & ((1u << kFineAtBits) - 1u);
+                        bits[r] = 0u;
+                        if (m == 0u)
+                            continue;
+                        const uint32_t at = stage.at[l][5u * seg + (uint32_t)r] + off;
+                        const float *px = &stage.x[buf][at], *py = &stage.y[buf][at], *pz = &stage.z[buf][at];
+                        // only the middle row holds the particle itself
+                        const uint32_t self = l == 2 && r == 2 ? s - stage.slot[l][5u * seg + (uint32_t)r] - off : 0u;
+                        float x[3], y[3], z[3];
+#pragma unroll
+                        for (int i = 0; i < 3; ++i) {
+                            x[i] = px[i];
+                            y[i] = py[i];
+                            z[i] = pz[i];
                         }
-                        ++nn;
-                        if (any_slow) {
-                            // summed again, each with its m_ij
-                            const uint32_t at = stage.at[l][5u * seg + (uint32_t)r] + off + k;
-                            const float t = test(stage.x[buf][at], stage.y[buf][at], stage.z[buf][at]);
-                            int mult = 1;
-                            if (slow)
-                                mult = bucket_multiplicity(ci.x, ci.y, ci.z, __float_as_uint(pos[j0 + k].w) & 0xFFFFu);
-                            slow_acc += (float)mult * (mp6 * ((t * t) * t));
-                            cnt += (uint32_t)mult - 1u;
+                        uint32_t k = 0;
+                        do {
+                            float t[3];
+#pragma unroll
+                            for (int i = 0; i < 3; ++i) {
+                                t[i] = test(x[i], y[i], z[i]);
+                                if (l == 2 && r == 2)
+                                    t[i] = k + (uint32_t)i != self ? t[i] : 0.0f;
+                            }
+#pragma unroll
+                            for (int i = 0; i < 3; ++i) {  // the next three, meanwhile
+                                x[i] = px[k + 3u + (uint32_t)i];
+                                y[i] = py[k + 3u + (uint32_t)i];
+                                z[i] = pz[k + 3u + (uint32_t)i];
+                            }
+#pragma unroll
+                            for (int i = 0; i < 3; ++i) {
+                                acc = acc + mp6 * ((t[i] * t[i]) * t[i]);
+                                bits[r] = __builtin_amdgcn_alignbit(bits[r], 0u - __float_as_uint(t[i]), 31u);  // << 1 | (t > 0)
+                            }
+                            k += 3u;
+                        } while (k < m);
+                        bits[r] <<= 32u - k;  // the first on top (k <= 30)
+                    }
+                    if (l < 4)
+                        arrived();
+#pragma unroll
+                    for (int r = 0; r < 5; ++r) {
+                        if (bits[r] == 0u)
+                            continue;
+                        const uint32_t row = rows[(5 * l + r) / 2] >> (((5 * l + r) & 1) * 16);
+                        const uint32_t off = row >> kFineRowBits & ((1u << kFineAtBits) - 1u);
+                        const uint32_t j0 = stage.slot[l][5u * seg + (uint32_t)r] + off;
+                        do {
+                            const uint32_t k = (uint32_t)__builtin_clz(bits[r]);
+                            bits[r] &= ~(0x80000000u >> k);
+                            neighbour(j0 + k, [&] {
+                                const uint32_t at = stage.at[l][5u * seg + (uint32_t)r] + off + k;
+                                return make_float4(stage.x[buf][at], stage.y[buf][at], stage.z[buf][at], 0.0f);
+                            });
+                        } while (bits[r] != 0u);
+                    }
+                }
+            } else {
+                // The thin surface of a flow: a wave's lanes lie in many rows,
+                // whose stencils don't fit.  Each lane walks its own rows from
+                // memory, the next row's first four candidates on the way
+                // meanwhile, and lists at the end.
+                wave_lds_sync();  // at[], slot[]
+#pragma unroll
+                for (int l = 0; l < 5; ++l)
+#pragma unroll
+                    for (int r = 0; r < 5; ++r) {
+                        shared.row[0][5 * l + r][lane] = from[l][r];
+                        shared.row[1][5 * l + r][lane] = n[l][r];
+                    }
+                wave_lds_sync();
+                auto four = [&](uint32_t first, uint32_t m, uint32_t k, float4 (&q)[4]) {
+#pragma unroll
+                    for (uint32_t i = 0; i < 4u; ++i)  // the last one again behind it
+                        q[i] = pos[m != 0u ? first + min(k + i, m - 1u) : s];
+                };
+                uint32_t first = shared.row[0][0][lane], m = shared.row[1][0][lane];
+                float4 q[4];
+                four(first, m, 0u, q);
+                for (uint32_t r = 0; r < 25u; ++r) {
+                    const uint32_t next = min(r + 1u, 24u);
+                    const uint32_t next_first = shared.row[0][next][lane], next_m = shared.row[1][next][lane];
+                    float4 next_q[4];
+                    four(next_first, next_m, 0u, next_q);
+                    uint32_t bits = 0, k = 0;
+                    for (;;) {
+#pragma unroll
+                        for (uint32_t i = 0; i < 4u; ++i) {
+                            float t = test(q[i].x, q[i].y, q[i].z);
+                            t = k + i < m && first + k + i != s ? t : 0.0f;
+                            acc = acc + mp6 * ((t * t) * t);
+                            bits = __builtin_amdgcn_alignbit(bits, 0u - __float_as_uint(t), 31u);
                         }
-                    } while (bits[r] != 0u);
+                        k += 4u;
+                        if (k >= m)
+                            break;
+                        four(first, m, k, q);
+                    }
+                    shared.row[1][r][lane] = bits << (32u - k);  // k <= 32
+                    first = next_first;
+                    m = next_m;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        q[i] = next_q[i];
+                }
+                for (uint32_t r = 0; r < 25u; ++r) {
+                    const uint32_t j0 = shared.row[0][r][lane];
+                    for (uint32_t bits = shared.row[1][r][lane]; bits != 0u;) {
+                        const uint32_t k = (uint32_t)__builtin_clz(bits);
+                        bits &= ~(0x80000000u >> k);
+                        neighbour(j0 + k, [&] { return pos[j0 + k]; });
+                    }
                 }
             }
             if (any_slow)
@@ -2174,7 +2249,8 @@ __device__ inline bool combine_parts(const PartPlan &pp, uint32_t w, uint32_t pa
 // particle.  MODE 2: also the neighbour ids (multiplicity-repeated).  MODE
 // 3: MODE 0 plus the neighbour count (with multiplicity) of the production
 // walks.  Writes rho, posR = (x, 0.5 / rho) and velR = (v, p) for the force
-// pass, and in MODE 0 / 3 the neighbour lists of unsplit per-lane tasks.
+// pass, and in MODE 0 / 3 the neighbour lists of unsplit tasks.  With a plan
+// it takes only the tasks the planning pass has not summed.
 template <int MODE, int BLOCK>
 __global__ __launch_bounds__(BLOCK, 6) void k_density(
     const float4 *__restrict__ pos, const float4 *__restrict__ vel,
@@ -2632,9 +2708,17 @@ __device__ inline void force_pair(float d2, float dx, float dy, float dz, float 
     fz = fmaf(cv, w.z - vi.z, fz);
 }
 
-// Two walks, chosen per wave by plan_union, with identical per-lane sums:
-//  * union: one wave-uniform candidate at a time (staged through LDS), the
-//    pair term predicated on the lane's own test;
+// Three walks.  Unsplit, they give the same sums bit for bit:
+//  * lists, where every lane of an unsplit task has one: the listed slots,
+//    four at a time.  Bound by the gathers: on cells of h / 2, where the k-th
+//    neighbours of neighbouring lanes are neighbours, a million particles take
+//    91 us, on cells of h 155;
+//  * union: one wave-uniform candidate at a time, staged through LDS and
+//    clamped to a term of zeros where it is none of the lane's.  Bound by
+//    arithmetic: in a late state of a million particles (3,260 neighbours
+//    each) 29 instructions, 79 cycles, a candidate and 90% of the issue slots;
+//    4.0 ms with operands in scalar registers, a test and two
+//    transcendentals a candidate, 3.55 now;
 //  * per lane: candidates filtered kForceChunk at a time into a per-lane
 //    bitmask, the terms then run only over the set bits, so a wave pays for
 //    the most neighbours any of its lanes has in the chunk.
