@@ -485,6 +485,16 @@ int Batch::grid_info(uint32_t s, float *cell_scale, double *cand_per_nbr)
 {
     if (s >= scenes.size())
         return fail(SPH_E_INVALID, "grid_info: bad scene");
+    bool settled = true, complete_now = true;  // replaced scenes choose their grids now, if not at a step
+    for (const BatchScene &o : scenes) {
+        settled = settled && !o.bounds_pending;
+        complete_now = complete_now && o.uploaded;
+    }
+    if (!settled && complete_now) {
+        int rc;
+        if ((!hold_grid && (rc = auto_grid())) || (rc = prepare()))
+            return rc;
+    }
     const BatchScene &b = scenes[s];
     if (cell_scale)
         *cell_scale = (float)(b.scale > 0.0 ? b.scale : (b.desc.cell_scale > 0.0f ? (double)b.desc.cell_scale : 1.0));

@@ -76,3 +76,51 @@ def test_frame_sizes(n):
     if n <= A.NOALLOC_MAX_PARTICLES:
         ref, rxf = A.update_particles_noalloc(p, S, 1e-3, BOX)
         assert out.tobytes() == ref.tobytes() and xf.tobytes() == rxf.tobytes()
+
+
+def test_threads_share_the_staging_memory():
+    """Downloads above 2 MiB from several threads at once, each its own scene."""
+    import threading
+
+    sizes, bad = (120000, 90001, 200003), []
+
+    def work(n):
+        try:
+            with A.Context(n, S, BOX, 1e-3) as c:
+                for k in range(4):
+                    pos, vel = _state(n, 10 * n + k)
+                    c.upload(pos, vel)
+                    got = c.download()
+                    if got["pos"].tobytes() != pos.tobytes() or got["vel"].tobytes() != vel.tobytes():
+                        bad.append((n, k))
+        except Exception as e:  # noqa: BLE001
+            bad.append((n, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(n,)) for n in sizes]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+def test_grid_info_after_a_scene_is_replaced():
+    """The automatic grid's choice for a replaced scene shows at once, as
+    after the first upload, and is the one it steps on."""
+    n = 140608  # 52^3, a uniform lattice: chooses cells of h / 2
+    g = np.stack(np.meshgrid(*[np.arange(52)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    pos = (g * 0.05 - 1.5 + np.random.default_rng(3).uniform(-0.005, 0.005, g.shape)).astype(F32)
+    small, _ = _state(500, 5, 0.3)
+    with A.Batch([A.scene_desc(n, S, BOX, 1e-3, auto_grid=True), A.scene_desc(500, S, BOX, 1e-3)]) as b:
+        b.upload(0, pos)
+        b.upload(1, small)
+        first = b.grid_info(0)
+        b.step(2)
+        b.upload(0, pos)
+        assert b.grid_info(0)[0] == first[0] == 0.5
+        b.step(2)
+        again = b.download(0)
+    with A.Context(n, S, BOX, 1e-3, auto_grid=True) as c:
+        c.upload(pos)
+        c.step(2)
+        assert _same(again, c.download())
