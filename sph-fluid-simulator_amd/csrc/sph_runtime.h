@@ -72,10 +72,10 @@ struct HostSpan {
 
 // Copies the spans to pageable host memory, after the work enqueued on st;
 // returns when they are there.  Large copies go through the shared memory in
-// pieces, several threads at a time: copying out of pinned memory (and
-// having the system provide the destination's pages) takes one thread several
-// times as long as the device needs to deliver (1M particles, 32 MB to fresh
-// pages: 13 ms directly, 3 this way).
+// pieces, several threads copying out of it: that (and having the system
+// provide the destination's pages) takes one thread several times as long as
+// the device needs to deliver (1M particles, 36 MB: 13 ms directly to fresh
+// pages, 2 this way).
 int copy_to_host(hipStream_t st, const HostSpan *spans, int count, HostStage &stage);
 
 // Inverse of the device's order-preserving map of floats to ints.

@@ -12,6 +12,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <condition_variable>
 #include <mutex>
 #include <new>
 #include <string>
@@ -244,13 +245,13 @@ void DevBuf::release()
 // ------------------------------------------------------------ transfers
 
 namespace {
-constexpr int kCopiers = 8;
-constexpr size_t kPerCopier = 4ull << 20;
+constexpr size_t kPieces = 8;              // of staging memory
+constexpr size_t kPerCopier = 4ull << 20;  // bytes of a download per copying thread, at least
 }  // namespace
 
 struct Staging {
     std::mutex mu;
-    unsigned char *base = nullptr;  // kCopiers pieces
+    unsigned char *base = nullptr;  // kPieces pieces
     ~Staging()
     {
         if (base)
@@ -284,7 +285,7 @@ std::shared_ptr<Staging> staging()
         std::shared_ptr<Staging> s = shared.lock();
         if (!s) {
             s = std::make_shared<Staging>();
-            if (pinned_alloc((void **)&s->base, kPiece * kCopiers) != hipSuccess)
+            if (pinned_alloc((void **)&s->base, kPiece * kPieces) != hipSuccess)
                 return nullptr;
             shared = s;
         }
@@ -294,33 +295,97 @@ std::shared_ptr<Staging> staging()
     }
 }
 
-// Copier t of a download by `workers`: every workers-th piece, through its
-// own part of the staging memory, while the copies of the others run.
-hipError_t copy_pieces(int device, hipStream_t st, const HostSpan *spans, int count, int t, int workers,
-                       unsigned char *buf)
-{
-    hipEvent_t done = nullptr;
-    hipError_t err = hipSetDevice(device);
-    if (err == hipSuccess)
-        err = hipEventCreateWithFlags(&done, hipEventDisableTiming);
-    size_t piece = 0;
-    for (int k = 0; k < count; ++k)
-        for (size_t at = 0; at < spans[k].bytes && err == hipSuccess; at += kPiece, ++piece) {
-            if (piece % (size_t)workers != (size_t)t)
-                continue;
-            const size_t bytes = std::min(kPiece, spans[k].bytes - at);
-            err = hipMemcpyAsync(buf, (const char *)spans[k].src + at, bytes, hipMemcpyDeviceToHost, st);
-            if (err == hipSuccess)
-                err = hipEventRecord(done, st);
-            if (err == hipSuccess)
-                err = hipEventSynchronize(done);
-            if (err == hipSuccess)
-                std::memcpy((char *)spans[k].dst + at, buf, bytes);
+// A download in pieces: this thread has the device bring them, copying
+// threads put them where they belong.  (The copying threads make no runtime
+// calls: a new thread's first ones take milliseconds at times.)
+struct Download {
+    const HostSpan *spans;
+    unsigned char *ring;
+    std::mutex mu;
+    std::condition_variable cv;
+    size_t pieces = 0, threads = 0;
+    size_t arrived = 0;             // pieces 0 .. arrived - 1 lie in the ring
+    size_t finished[kPieces] = {};  // pieces that have left each place
+    bool failed = false;
+
+    HostSpan piece(size_t p) const
+    {
+        for (const HostSpan *h = spans;; ++h) {
+            const size_t n = (h->bytes + kPiece - 1) / kPiece;
+            if (p < n)
+                return HostSpan{(char *)h->dst + p * kPiece, (const char *)h->src + p * kPiece,
+                                std::min(kPiece, h->bytes - p * kPiece)};
+            p -= n;
         }
-    if (done)
-        (void)hipEventDestroy(done);
-    return err;
-}
+    }
+    void put(size_t p)
+    {
+        const HostSpan h = piece(p);
+        std::memcpy(h.dst, ring + kPiece * (p % kPieces), h.bytes);
+    }
+    // copying thread t
+    void copy(size_t t)
+    {
+        std::unique_lock<std::mutex> lock(mu);
+        for (size_t p = t; p < pieces; p += threads) {
+            cv.wait(lock, [&] { return arrived > p || failed; });
+            if (failed)
+                return;
+            lock.unlock();
+            put(p);
+            lock.lock();
+            ++finished[p % kPieces];
+            cv.notify_all();
+        }
+    }
+    hipError_t run(hipStream_t st)
+    {
+        hipEvent_t there[kPieces] = {};
+        hipError_t e = hipSuccess;
+        for (size_t k = 0; k < std::min(kPieces, pieces) && e == hipSuccess; ++k)
+            e = hipEventCreateWithFlags(&there[k], hipEventDisableTiming);
+        size_t asked = 0;
+        for (size_t p = 0; p < pieces && e == hipSuccess; ++p) {
+            // as far ahead as the ring has room
+            while (asked < std::min(pieces, p + kPieces) && e == hipSuccess) {
+                const size_t at = asked % kPieces;
+                {
+                    std::unique_lock<std::mutex> lock(mu);
+                    if (finished[at] < asked / kPieces) {
+                        if (asked > p)
+                            break;
+                        cv.wait(lock, [&] { return finished[at] >= asked / kPieces; });
+                    }
+                }
+                const HostSpan h = piece(asked);
+                e = hipMemcpyAsync(ring + kPiece * at, h.src, h.bytes, hipMemcpyDeviceToHost, st);
+                if (e == hipSuccess)
+                    e = hipEventRecord(there[at], st);
+                ++asked;
+            }
+            if (e == hipSuccess)
+                e = hipEventSynchronize(there[p % kPieces]);
+            if (e == hipSuccess && threads == 0) {
+                put(p);
+                ++finished[p % kPieces];
+            } else if (e == hipSuccess) {
+                std::lock_guard<std::mutex> lock(mu);
+                arrived = p + 1;
+                cv.notify_all();
+            }
+        }
+        if (e != hipSuccess) {
+            std::lock_guard<std::mutex> lock(mu);
+            failed = true;
+            cv.notify_all();
+        }
+        const hipError_t w = hipStreamSynchronize(st);
+        for (hipEvent_t t : there)
+            if (t)
+                (void)hipEventDestroy(t);
+        return e != hipSuccess ? e : w;
+    }
+};
 
 }  // namespace
 
@@ -379,36 +444,32 @@ int copy_to_host(hipStream_t st, const HostSpan *spans, int count, HostStage &st
         return e == hipSuccess ? SPH_OK : hip_fail(e, "download");
     }
     Staging &ring = *stage.large;
-    int device = 0;
     e = hipStreamSynchronize(st);  // not with the staging memory held
-    if (e == hipSuccess)
-        e = hipGetDevice(&device);
     if (e != hipSuccess)
         return hip_fail(e, "download");
-    std::lock_guard<std::mutex> lock(ring.mu);
-    hipError_t failed[kCopiers] = {};
-    std::thread threads[kCopiers];
-    // (a thread's first calls into the runtime take a millisecond now and then)
-    const int workers = (int)std::min<size_t>(kCopiers, 1 + total / kPerCopier);
-    auto copier = [&](int t) {
-        failed[t] = copy_pieces(device, st, spans, count, t, workers, ring.base + kPiece * (size_t)t);
-    };
-    for (int t = 1; t < workers; ++t) {
-        try {
-            threads[t] = std::thread(copier, t);
-        } catch (const std::exception &) {  // no thread to be had: this one does its share below
+    std::lock_guard<std::mutex> held(ring.mu);
+    Download d;
+    d.spans = spans;
+    d.ring = ring.base;
+    for (int k = 0; k < count; ++k)
+        d.pieces += (spans[k].bytes + kPiece - 1) / kPiece;
+    const size_t want = total / kPerCopier;  // none below 4 MiB: this thread copies
+    std::thread threads[kPieces];
+    {
+        std::lock_guard<std::mutex> lock(d.mu);  // they start when all are known
+        for (size_t t = 0; t < std::min(kPieces, want); ++t) {
+            try {
+                threads[t] = std::thread([&d, t] { d.copy(t); });
+            } catch (const std::exception &) {
+                break;  // fewer then, or none
+            }
+            ++d.threads;
         }
     }
-    copier(0);
-    for (int t = 1; t < workers; ++t) {
-        if (threads[t].joinable())
-            threads[t].join();
-        else
-            copier(t);
-    }
-    e = hipStreamSynchronize(st);
-    for (hipError_t f : failed)
-        e = e != hipSuccess ? e : f;
+    e = d.run(st);
+    for (std::thread &t : threads)
+        if (t.joinable())
+            t.join();
     return e == hipSuccess ? SPH_OK : hip_fail(e, "download");
 }
 
