@@ -87,12 +87,16 @@ struct SceneSet {
 };
 
 // Whether short walks of a scene are staged in LDS (k_plan_list): cells of
-// h or larger, and the per-lane walk not forced.
-SPH_HD inline bool stageable(const StepParams &P) { return P.reach == 1 && P.lane_walk == 0u; }
+// h or larger, the per-lane walk not forced, and no neighbour beyond h (the
+// staged rows hold candidates beyond the lane's cut stencil, which must fail).
+SPH_HD inline bool stageable(const StepParams &P)
+{
+    return P.reach == 1 && P.lane_walk == 0u && P.h2 <= P.h * P.h;
+}
 // Or, in a launch without such a scene, those on cells of h / 2 to h (k_plan_fine).
 SPH_HD inline bool fine_stageable(const StepParams &P)
 {
-    return P.reach == 2 && P.lane_walk == 0u && P.h2 <= 1.0f;
+    return P.reach == 2 && P.lane_walk == 0u && P.h2 <= P.h * P.h && P.h2 <= 1.0f;
 }
 
 // Spare part tasks of a scene of `waves` wave tasks (beyond one per task):

@@ -2674,14 +2674,16 @@ __device__ inline void integrate_and_walls(float4 &x, float4 &v, float fx, float
 //   F += cp d + cv (v_j - v_i)
 // q = (x_j, 0.5 / rho_j), w = (v_j, p_j), d = x_j - x_i, am = m_ij (0.5 / rho_j).
 // r and h - r are the reference's values bit for bit (near the support edge
-// h - r cancels, and an error in r would be amplified).  A candidate that is
-// no neighbour has d2 >= fl(h h), so r >= h (the root of the rounded square
-// is h itself) and h - r clamps to 0: it adds zeros, without a test.
+// h - r cancels, and an error in r would be amplified).
+// CLAMP: also for candidates that are no neighbours, where h2 = fl(h h): they
+// have d2 >= h2, so r >= h (the root of the rounded square is h itself) and
+// h - r clamps to 0: they add zeros, without a test.  (With another h2 a
+// neighbour may be farther than h, and h - r below zero.)
 // SPLIT: the part of a split walk, whose sums depend on the parts' bounds
 // anyway: the same product in an order that takes fewer operations and root()
 // (28 against 49 issue cycles a wave before the six fmas).  Unsplit walks
 // keep one order of operations in all their forms.
-template <bool UNIT, bool SPLIT>
+template <bool CLAMP, bool UNIT, bool SPLIT>
 __device__ inline void force_pair(float d2, float dx, float dy, float dz, float am, float4 w, float4 vi,
                                   float p_i, float h, float neg_m_spg, float mu2_m_lap, float &fx,
                                   float &fy, float &fz)
@@ -2690,13 +2692,13 @@ __device__ inline void force_pair(float d2, float dx, float dy, float dz, float 
     if (SPLIT) {
         float rinv;
         const float r = root(d2, rinv);
-        const float hr = positive<UNIT>(h - r);
+        const float hr = CLAMP ? positive<UNIT>(h - r) : h - r;
         const float u = hr * am;
         cp = ((p_i + w.w) * neg_m_spg) * u * (hr * rinv);
         cv = u * mu2_m_lap;
     } else {
         const float r = sqrt_rn(d2);
-        const float hr = positive<UNIT>(h - r);
+        const float hr = CLAMP ? positive<UNIT>(h - r) : h - r;
         cp = neg_m_spg * (p_i + w.w) * am * (hr * hr) * __builtin_amdgcn_rcpf(r);
         cv = mu2_m_lap * hr * am;
     }
@@ -2763,7 +2765,7 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                 asm volatile("" : "+v"(cx), "+v"(cy), "+v"(cz));
                 am = q.w * (float)bucket_multiplicity(cx, cy, cz, __float_as_uint(posB[j].w) & 0xFFFFu);
             }
-            force_pair<false, false>(d2, dx, dy, dz, am, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+            force_pair<false, false, false>(d2, dx, dy, dz, am, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
         };
         // Every lane holds its neighbour list (the density pass walked this
         // task per lane, unsplit): visit the listed slots four at a time,
@@ -2809,8 +2811,9 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
             // Values that are not finite (or far beyond any scene's) would
             // reach a lane through a candidate that is no neighbour (0 x inf):
             // a chunk that holds some, and every chunk of a wave that does, is
-            // walked with a test per candidate, as are the wave's own slots.
-            const bool plain = __all(fabsf(pi.x) + fabsf(pi.y) + fabsf(pi.z) + fabsf(vi.x) + fabsf(vi.y) +
+            // walked with a test per candidate, as are the wave's own slots, and
+            // every chunk of a scene whose h2 is not its h squared (force_pair).
+            const bool plain = h2 == h * h && __all(fabsf(pi.x) + fabsf(pi.y) + fabsf(pi.z) + fabsf(vi.x) + fabsf(vi.y) +
                                          fabsf(vi.z) + fabsf(p_i) <= kFarAway);
             const uint32_t W = 2u * (uint32_t)P.reach + 1u;
             uint32_t at_layer = kNoSlot;
@@ -2830,16 +2833,16 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                             const float4 q = rec[0][k], w = rec[1][k];  // (x_j, 0.5 / rho_j), (v_j, p_j)
                             const float d2 = dist2_ref(me, q, dx, dy, dz);
                             if (d2 < h2 && slots[k] != s)
-                                force_pair<unit, split>(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                                force_pair<false, unit, split>(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
                         }
                         return;
                     }
                     for (uint32_t k = 0; k < n; k += 2u) {
                         const float4 q0 = rec[0][k], w0 = rec[1][k], q1 = rec[0][k + 1u], w1 = rec[1][k + 1u];
                         float d2 = dist2_ref(me, q0, dx, dy, dz);
-                        force_pair<unit, split>(d2, dx, dy, dz, q0.w, w0, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                        force_pair<true, unit, split>(d2, dx, dy, dz, q0.w, w0, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
                         d2 = dist2_ref(me, q1, dx, dy, dz);
-                        force_pair<unit, split>(d2, dx, dy, dz, q1.w, w1, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                        force_pair<true, unit, split>(d2, dx, dy, dz, q1.w, w1, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
                     }
                 });
             };
