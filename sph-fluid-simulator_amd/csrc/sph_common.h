@@ -78,6 +78,10 @@ struct StepParams {
     uint32_t p_begin, p_end;
     // 1: every wave walks its candidates per lane (never the union walk)
     uint32_t lane_walk;
+    // largest magnitude of a particle's values up to which the force of a
+    // candidate that is no neighbour comes out as zeros with h - r clamped at
+    // 0 (zero_term_limit); below 0: for none
+    float zero_limit;
 };
 
 SPH_HD inline uint32_t hash16(uint32_t cx, uint32_t cy, uint32_t cz)

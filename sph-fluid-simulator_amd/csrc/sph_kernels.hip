@@ -1113,9 +1113,11 @@ __device__ inline void wave_lds_sync()
 // candidate loop never waits on a global load, never pays per-row overhead,
 // and its operands are vector registers (fed from scalar registers the same
 // loop issues its three subtractions at half rate).  Places that hold no
-// candidate stage a record far away, with slot ~0, that fails every test, so
-// chunks run in groups of four unchecked.
-constexpr float kFarAway = 1.0e18f;  // its square is finite
+// candidate stage a record with slot ~0 that passes no test, so chunks run in
+// groups of four unchecked: at infinity, or, where products with its distance
+// must stay finite (FINITE), far away from every wave that has none of its
+// own near there (StepParams::zero_limit).
+constexpr float kFarAway = 0x1p60f;  // its square is finite
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 
 // One record array (positions, w unused) is kept as three coordinate arrays:
@@ -1198,11 +1200,12 @@ __device__ inline void part_slice(uint32_t total, uint32_t part, uint32_t nparts
 // multiple of four with the ones far away), all of z-layer `layer` (2R + 1 to
 // a segment).  odd: the
 // chunk holds some of the wave's own slots [first, first + 64) or, with
-// FINITE, a record that is not finite.
+// FINITE, a record with values beyond `limit` (or not finite).
 template <int NV, bool FINITE, class Chunk>
-__device__ inline void union_walk(uint32_t lo, uint32_t hi, uint32_t first, const float4 *const (&src)[NV],
-                                  UnionStage<NV> &T, Chunk chunk)
+__device__ inline void union_walk(uint32_t lo, uint32_t hi, uint32_t first, float limit,
+                                  const float4 *const (&src)[NV], UnionStage<NV> &T, Chunk chunk)
 {
+    constexpr float far = FINITE ? kFarAway : __builtin_inff();
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t ny = __builtin_amdgcn_readfirstlane(T.ny);
     uint32_t row = 0, next = T.start[1];
@@ -1219,7 +1222,7 @@ __device__ inline void union_walk(uint32_t lo, uint32_t hi, uint32_t first, cons
                 r[v] = src[v][slot];
         } else {
             slot = kNoSlot;
-            r[0] = make_float4(kFarAway, kFarAway, kFarAway, 0.0f);
+            r[0] = make_float4(far, far, far, 0.0f);
 #pragma unroll
             for (int v = 1; v < NV; ++v)
                 r[v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1237,7 +1240,7 @@ __device__ inline void union_walk(uint32_t lo, uint32_t hi, uint32_t first, cons
 #pragma unroll
             for (int v = 0; v < NV; ++v)
                 size += fabsf(nr[v].x) + fabsf(nr[v].y) + fabsf(nr[v].z) + fabsf(nr[v].w);
-            odd = odd || !(size <= 8.0f * kFarAway);
+            odd = odd || (ns != kNoSlot && !(size <= limit));
         }
         const bool any_odd = __any(odd);
         const uint32_t n = (uint32_t)__builtin_popcountll(__ballot(ns != kNoSlot));
@@ -2327,17 +2330,17 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
             uint32_t nn = 0, at_layer = kNoSlot;
             uint32_t *lp = nl.list + s;
             const uint32_t W = 2u * (uint32_t)P.reach + 1u;
-            float4 me = pi;  // far away from the candidates of other lanes' segments
+            float4 me = pi;  // at infinity for the candidates of other lanes' segments
             // Unsplit sums are the per-lane walk's bit for bit.  Split ones
             // (added up part by part, so never quite those) leave the factor
             // to the end of the part: two operations a term instead of four.
             auto walk = [&](auto unit_tag, auto split_tag) {
                 constexpr bool unit = decltype(unit_tag)::value, split = decltype(split_tag)::value;
-                union_walk<1, false>(lo, hi, L.first, src, T, [&](const ChunkRecords<1> &c, const uint32_t *slots,
+                union_walk<1, false>(lo, hi, L.first, 0.0f, src, T, [&](const ChunkRecords<1> &c, const uint32_t *slots,
                                                                       uint32_t n, bool odd, uint32_t lz) {
                     if (U.segments && lz != at_layer) {
                         at_layer = lz;
-                        me.x = T.segment[threadIdx.x & 63u] == lz / W ? pi.x : kFarAway;
+                        me.x = T.segment[threadIdx.x & 63u] == lz / W ? pi.x : __builtin_inff();
                     }
                     // Branch-free: h2 - d2 > 0 exactly when d2 < h2 (the float
                     // difference of unequal values is nonzero), so clamping it
@@ -2813,30 +2816,32 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
             // a chunk that holds some, and every chunk of a wave that does, is
             // walked with a test per candidate, as are the wave's own slots, and
             // every chunk of a scene whose h2 is not its h squared (force_pair).
-            const bool plain = h2 == h * h && __all(fabsf(pi.x) + fabsf(pi.y) + fabsf(pi.z) + fabsf(vi.x) + fabsf(vi.y) +
-                                         fabsf(vi.z) + fabsf(p_i) <= kFarAway);
+            const float limit = P.zero_limit;
+            const bool plain = __all(fabsf(pi.x) + fabsf(pi.y) + fabsf(pi.z) + fabsf(vi.x) + fabsf(vi.y) +
+                                         fabsf(vi.z) + fabsf(p_i) <= limit);
             const uint32_t W = 2u * (uint32_t)P.reach + 1u;
             uint32_t at_layer = kNoSlot;
-            float4 me = pi;  // far away from the candidates of other lanes' segments
+            bool mine = true;  // the chunk's candidates are those of the lane's segment
             auto walk = [&](auto unit_tag, auto split_tag) {
                 constexpr bool unit = decltype(unit_tag)::value, split = decltype(split_tag)::value;
-                union_walk<2, true>(lo, hi, L.first, src, T, [&](const ChunkRecords<2> &c, const uint32_t *slots,
+                union_walk<2, true>(lo, hi, L.first, limit, src, T, [&](const ChunkRecords<2> &c, const uint32_t *slots,
                                                                      uint32_t n, bool odd, uint32_t lz) {
                     const float4(&rec)[2][64] = c.rec;
                     float dx, dy, dz;
                     if (U.segments && lz != at_layer) {
                         at_layer = lz;
-                        me.x = T.segment[threadIdx.x & 63u] == lz / W ? pi.x : kFarAway;
+                        mine = T.segment[threadIdx.x & 63u] == lz / W;
                     }
                     if (odd || !plain) {
                         for (uint32_t k = 0; k < n; ++k) {
                             const float4 q = rec[0][k], w = rec[1][k];  // (x_j, 0.5 / rho_j), (v_j, p_j)
-                            const float d2 = dist2_ref(me, q, dx, dy, dz);
-                            if (d2 < h2 && slots[k] != s)
+                            const float d2 = dist2_ref(pi, q, dx, dy, dz);
+                            if (d2 < h2 && mine && slots[k] != s && slots[k] != kNoSlot)
                                 force_pair<false, unit, split>(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
                         }
                         return;
                     }
+                    const float4 me = make_float4(mine ? pi.x : kFarAway, pi.y, pi.z, 0.0f);
                     for (uint32_t k = 0; k < n; k += 2u) {
                         const float4 q0 = rec[0][k], w0 = rec[1][k], q1 = rec[0][k + 1u], w1 = rec[1][k + 1u];
                         float d2 = dist2_ref(me, q0, dx, dy, dz);

@@ -139,6 +139,26 @@ int grid_reach(double cell_scale)
     return R <= kMaxReach ? R : 0;
 }
 
+namespace {
+
+// StepParams::zero_limit.  Where h2 = fl(h h), a candidate that is no
+// neighbour has r >= h (see force_pair; the root is exact from 2^-96 on), and
+// its force is a product with max(h - r, 0) = 0: zero unless another factor
+// or their product overflows.  With values up to L (sums of two up to 2 L, of
+// their distance to the records far away up to 2^60), the products formed
+// before that zero are at most |m spikyGrad| 2 L L, and L = 2^56 keeps the
+// far records (kFarAway) farther than any h up to L.
+float zero_term_limit(const StepParams &P)
+{
+    const double g = std::fabs((double)P.neg_m_spg), largest = 0x1p56;
+    if (P.h2 != P.h * P.h || !(P.h2 >= 0x1p-96f) || !(P.h <= largest) || !std::isfinite(g) ||
+        !std::isfinite(2.0f * P.mu_m_lap))
+        return -1.0f;
+    return (float)std::min(largest, std::sqrt(1e38 / std::max(g, 1.0)));
+}
+
+}  // namespace
+
 StepParams make_params(const sph_settings_v1 &s, const sph_box_v1 &box, float dt)
 {
     StepParams P;
@@ -158,6 +178,7 @@ StepParams make_params(const sph_settings_v1 &s, const sph_box_v1 &box, float dt
     P.dt = dt;
     P.neg_m_spg = -(s.mass * s.spikyGrad);
     P.mu_m_lap = (s.viscosity * s.mass) * s.spikyLap;
+    P.zero_limit = zero_term_limit(P);
     for (int k = 0; k < 3; ++k) {
         P.wall_lo[k] = box.lo[k] + s.h;
         P.wall_hi[k] = box.hi[k] - s.h;
