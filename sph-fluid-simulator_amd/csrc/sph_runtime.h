@@ -101,7 +101,8 @@ struct Workspace {
     uint32_t nwaves = 0;
     uint32_t nscenes = 0;
     bool staged = false, fine = false;  // SceneSet's of the current scene set
-    std::vector<WaveTask> host_tasks;  // what `tasks` holds
+    std::vector<WaveTask> host_tasks;  // what `tasks` holds, or empty
+    bool counters_owed = true;  // pdone, ptotal have still to be cleared
     uint32_t part_cap = 0;  // part-task capacity of the current scene set
     int stencil_block = kStencilBlock;  // threads per block of the density and force passes
     int reserve_particles(uint32_t n);

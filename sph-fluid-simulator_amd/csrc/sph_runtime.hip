@@ -541,11 +541,14 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
         for (uint32_t f = scenes[k].p_begin; f < scenes[k].p_end; f += 64u)
             t.push_back(WaveTask{k, f});
     int rc;
-    const void *had_tasks = tasks.ptr;
+    // Known no longer from here on, should an allocation below fail.
+    const bool same = t.size() == host_tasks.size() && !t.empty() &&
+                      std::memcmp(t.data(), host_tasks.data(), sizeof(WaveTask) * t.size()) == 0;
+    if (!same)
+        host_tasks.clear();
     if ((rc = params.reserve(sizeof(StepParams) * std::max<size_t>(scenes.size(), 1))) ||
         (rc = tasks.reserve(sizeof(WaveTask) * std::max<size_t>(t.size(), 1))))
         return rc;
-    const bool fresh_tasks = tasks.ptr != had_tasks;
     const size_t nw = std::max<size_t>(t.size(), 1);
     size_t nslots = 0;
     for (const StepParams &sp : scenes)
@@ -558,24 +561,23 @@ int Workspace::set_scenes(const std::vector<StepParams> &scenes, hipStream_t st)
     cap = std::max<size_t>(cap, nw);
     if (cap > 0xFFFFFFFFull)
         return fail(SPH_E_LIMIT, "part plan: %zu part tasks", cap);
-    const bool fresh_counters = pdone.bytes < 4 * nw ||
-                                ptotal.bytes < 8 * kTotalSlots * std::max<size_t>(scenes.size(), 1);
+    counters_owed = counters_owed || pdone.bytes < 4 * nw ||
+                    ptotal.bytes < 8 * kTotalSlots * std::max<size_t>(scenes.size(), 1);
     if ((rc = pnparts.reserve(4ull * nw)) || (rc = poff.reserve(4ull * nw)) || (rc = pmeasure.reserve(4ull * nw)) ||
         (rc = ptotal.reserve(8ull * kTotalSlots * std::max<size_t>(scenes.size(), 1))) || (rc = ptasks.reserve(4ull * cap)) ||
         (rc = pqueue.reserve(16)) ||
         (rc = pbuf.reserve(sizeof(float4) * 64ull * cap)) || (rc = pdone.reserve(4ull * nw)) ||
         (rc = pwalk.reserve(2ull * sizeof(int4) * nw)) || (rc = pown.reserve(4ull * std::max<size_t>(nslots, 1))))
         return rc;
-    if (fresh_counters) {  // zero outside use from here on: the step keeps them so
+    if (counters_owed) {  // zero outside use from here on: the step keeps them so
         launch_fill_u32(st, (uint32_t *)pdone.ptr, 0u, pdone.bytes / 4);
         launch_fill_u32(st, (uint32_t *)ptotal.ptr, 0u, ptotal.bytes / 4);
+        counters_owed = false;
     }
     hipError_t e = hipSuccess;
     if (!scenes.empty())
         e = hipMemcpyAsync(params.ptr, scenes.data(), sizeof(StepParams) * scenes.size(),
                            hipMemcpyHostToDevice, st);
-    const bool same = !fresh_tasks && t.size() == host_tasks.size() &&
-                      std::memcmp(t.data(), host_tasks.data(), sizeof(WaveTask) * t.size()) == 0;
     if (e == hipSuccess && !t.empty() && !same)
         e = hipMemcpyAsync(tasks.ptr, t.data(), sizeof(WaveTask) * t.size(), hipMemcpyHostToDevice, st);
     if (e == hipSuccess)
@@ -677,6 +679,7 @@ void Workspace::release_all()
                       &nlist, &ncount, &unordered})
         b->release();
     host_tasks.clear();
+    counters_owed = true;
     ncells_padded = 0;
     big_cap = 0;
     nwaves = 0;
