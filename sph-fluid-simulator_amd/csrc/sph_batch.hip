@@ -781,7 +781,8 @@ int Batch::download(uint32_t s, float *pos, float *vel, float *rho, float *press
             return nullptr;
         float *at = raw;
         raw += per * n;
-        out[k++] = HostSpan{dst, at, 4 * per * n};
+        out[k] = HostSpan{dst, at, 4 * per * n, k > 0};
+        ++k;
         return at;
     };
     float *d_pos = span(pos, 3), *d_vel = span(vel, 3), *d_rho = span(rho, 1), *d_prs = span(pressure, 1);

@@ -68,6 +68,7 @@ struct HostSpan {
     void *dst;
     const void *src;  // device
     size_t bytes;
+    bool follows = false;  // lies behind the span before it, in the same allocation
 };
 
 // Copies the spans to pageable host memory, after the work enqueued on st;

@@ -440,9 +440,9 @@ int copy_to_host(hipStream_t st, const HostSpan *spans, int count, HostStage &st
     hipError_t e = hipSuccess;
     if (unsigned char *buf = stage.small(total)) {
         size_t at = 0;
-        for (int k = 0, next; k < count && e == hipSuccess; k = next) {  // neighbours on the device: one copy
+        for (int k = 0, next; k < count && e == hipSuccess; k = next) {  // one copy for spans of one piece
             size_t run = spans[k].bytes;
-            for (next = k + 1; next < count && spans[next].src == (const char *)spans[k].src + run; ++next)
+            for (next = k + 1; next < count && spans[next].follows; ++next)
                 run += spans[next].bytes;
             e = hipMemcpyAsync(buf + at, spans[k].src, run, hipMemcpyDeviceToHost, st);
             at += run;

@@ -1,6 +1,7 @@
 """The library's host code on a stand-in for the HIP runtime (fake_hip.c: no
-kernel runs): what it leaves behind when an allocation fails.  Each test is a
-process of its own, which loads the stand-in before the library."""
+kernel runs): what it leaves behind when an allocation fails, and that copies
+keep to their allocations.  Each test is a process of its own, which loads the
+stand-in before the library."""
 import os
 import subprocess
 import sys
@@ -76,4 +77,26 @@ def test_counters_after_a_failed_allocation(run):
         frame(n)
         assert fake.fake_launched(4 * ((n + 63) // 64)) == 1, k
     assert 20 < k < 199, k
+    """)
+
+
+def test_downloads_copy_within_their_allocations(run):
+    """Records and transforms of n particles, n a multiple of 1024, end on a
+    page, and the next allocation may begin there: each is copied by itself
+    (16,384: through small pinned memory, 40,960: in pieces)."""
+    run("""
+    for n in (1024, 2048, 15360, 16384, 40960):
+        frame(n)
+        pos = np.zeros((n, 3), np.float32)
+        with A.Context(n, S, BOX, 1e-3) as c:
+            c.upload(pos)
+            c.step(1)
+            c.download_particles()
+            c.download()
+        with A.Batch([A.scene_desc(n, S, BOX, 1e-3)] * 2) as b:
+            for k in range(2):
+                b.upload(k, pos)
+            b.step(1)
+            b.download_particles(1)
+            b.download(1)
     """)
