@@ -75,6 +75,7 @@ struct Batch {
     using GraphKey = std::array<uint64_t, 40>;
     GraphKey captured{};     // what the launches of `exec` were given
     bool complete = false;  // every scene has been uploaded since the scene list last changed
+    bool deferred = false;  // a replaced scene's set-up waits for the next call that needs it (settle)
     DevBuf aos, xf;  // download_particles staging
     DevBuf bounds;   // bounds of every scene's last upload
     HostStage stage;
@@ -115,6 +116,9 @@ struct Batch {
     GraphKey graph_key() const;
     // Gives freshly uploaded scenes their grids (waits for the device).
     int resolve_bounds();
+    // What an upload left for later: the automatic grid's choice, cells, scene
+    // table, keys, the step's graph.
+    int settle();
     // Sampled candidates per neighbour of every scene (ratio[s]): fresh =
     // from the cell order of the current state (sorted here), else from
     // the last step's (0 if there is none).

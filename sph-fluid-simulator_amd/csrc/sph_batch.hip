@@ -315,23 +315,33 @@ int Batch::upload(uint32_t s, const float *pos, const float *vel)
     // Once every scene holds particles, the first step's set-up (cells,
     // scene table, keys, the automatic grid's first choice, the step's graph)
     // runs here rather than inside the first step.  When a scene of several
-    // is replaced later, the others may follow: then the next step does it,
-    // once (64 scenes, each preparing all of them again: 13 ms).
+    // is replaced later, the others may follow: then the next call that needs
+    // it does it, once (64 scenes, each preparing all of them again: 13 ms).
     for (const BatchScene &o : scenes)
         if (!o.uploaded)
             return SPH_OK;
+    deferred = true;
     if (complete && scenes.size() > 1)
         return SPH_OK;
     complete = true;
-    if (!hold_grid && (rc = auto_grid()))
-        return rc;
-    if ((rc = prepare()))
-        return rc;
-    if (use_graph && (rc = capture()))
+    rc = settle();
+    deferred = false;
+    if (rc)
         return rc;
     e = hipStreamSynchronize(stream);
     if (e != hipSuccess)
         return hip_fail(e, "upload");
+    return SPH_OK;
+}
+
+int Batch::settle()
+{
+    if (!deferred)
+        return SPH_OK;
+    int rc;
+    if ((!hold_grid && (rc = auto_grid())) || (rc = prepare()) || (use_graph && (rc = capture())))
+        return rc;
+    deferred = false;
     return SPH_OK;
 }
 
@@ -413,6 +423,8 @@ int Batch::step(int nsteps)
         return fail(SPH_E_INVALID, "step: negative step count");
     if (scenes.empty() || nsteps == 0)
         return SPH_OK;
+    if ((rc = settle()))
+        return rc;
     bool any_auto = false;
     for (const BatchScene &b : scenes)
         any_auto = any_auto || (b.desc.flags & SPH_SCENE_AUTO_GRID) != 0u;
@@ -485,16 +497,8 @@ int Batch::grid_info(uint32_t s, float *cell_scale, double *cand_per_nbr)
 {
     if (s >= scenes.size())
         return fail(SPH_E_INVALID, "grid_info: bad scene");
-    bool settled = true, complete_now = true;  // replaced scenes choose their grids now, if not at a step
-    for (const BatchScene &o : scenes) {
-        settled = settled && !o.bounds_pending;
-        complete_now = complete_now && o.uploaded;
-    }
-    if (!settled && complete_now) {
-        int rc;
-        if ((!hold_grid && (rc = auto_grid())) || (rc = prepare()))
-            return rc;
-    }
+    if (const int rc = settle())
+        return rc;
     const BatchScene &b = scenes[s];
     if (cell_scale)
         *cell_scale = (float)(b.scale > 0.0 ? b.scale : (b.desc.cell_scale > 0.0f ? (double)b.desc.cell_scale : 1.0));
@@ -641,7 +645,7 @@ int Batch::step_timed(int nsteps, float *ms)
         return fail(SPH_E_INVALID, "step: negative step count");
     if (scenes.empty() || nsteps == 0)
         return SPH_OK;
-    if ((rc = prepare()))
+    if ((rc = settle()) || (rc = prepare()))
         return rc;
     while (events.size() < (size_t)nsteps + 1) {
         hipEvent_t e;
@@ -674,7 +678,7 @@ int Batch::autotune(int trial_steps, sph_tune_v1 *out, bool grid)
         return fail(SPH_E_INVALID, "autotune: bad arguments");
     if (scenes.empty())
         return fail(SPH_E_STATE, "autotune: no scenes");
-    if ((rc = prepare()))
+    if ((rc = settle()) || (rc = prepare()))
         return rc;
     std::memset(out, 0, sizeof *out);
     // The state every trial starts from (and is restored to at the end).
@@ -815,7 +819,7 @@ int Batch::profile(int nsteps, double *ms, int max_k, int *nk, char *names_buf, 
     int rc;
     if (nsteps <= 0 || !ms || !nk || max_k <= 0)
         return fail(SPH_E_INVALID, "profile: bad arguments");
-    if ((rc = prepare()))
+    if ((rc = settle()) || (rc = prepare()))
         return rc;
     std::vector<double> acc;
     std::vector<const char *> names;
@@ -863,7 +867,7 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
     int rc;
     if (s >= scenes.size() || !count)
         return fail(SPH_E_INVALID, "walk_dump: bad scene or NULL count");
-    if ((rc = prepare()))
+    if ((rc = settle()) || (rc = prepare()))
         return rc;
     const uint32_t N = total_n;
     // The B-side arrays hold the last step's order and densities, which the

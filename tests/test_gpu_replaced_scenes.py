@@ -1,0 +1,55 @@
+"""Replacing one scene of a batch leaves its grid, keys and automatic cell
+size to the next call that needs them: each such call sees what it would see
+after a first upload."""
+import numpy as np
+import pytest
+
+import sph_amd as A
+
+pytestmark = pytest.mark.gpu
+F32 = np.float32
+S = A.settings(mass=0.02, h=0.1)
+BOX = A.box((-2.0, -2.0, -2.0), (2.0, 2.0, 2.0))
+SIDE = 52  # a lattice of 52^3 particles chooses cells of h / 2
+N = SIDE ** 3
+
+
+def _lattice(seed=3):
+    g = np.stack(np.meshgrid(*[np.arange(SIDE)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    return (g * 0.05 - 1.5 + np.random.default_rng(seed).uniform(-0.005, 0.005, g.shape)).astype(F32)
+
+
+def _cloud(n, seed):
+    rng = np.random.default_rng(seed)
+    return rng.uniform(-0.5, 0.5, (n, 3)).astype(F32), rng.normal(0.0, 0.5, (n, 3)).astype(F32)
+
+
+def _batch():
+    return A.Batch([A.scene_desc(N, S, BOX, 1e-3, auto_grid=True), A.scene_desc(3000, S, BOX, 1e-3)])
+
+
+def _replaced():
+    """A batch that has run, its scene 0 replaced since by the lattice."""
+    b = _batch()
+    b.upload(0, _lattice(8))
+    b.upload(1, *_cloud(3000, 5))
+    b.step(2)
+    b.upload(0, _lattice())
+    return b
+
+
+def test_walk_dump_of_a_replaced_scene():
+    with _replaced() as b:
+        got = b.walk_dump(0, lists=True)
+    with _batch() as b:  # the same company: which kernel walks depends on it
+        b.upload(0, _lattice())
+        b.upload(1, *_cloud(3000, 5))
+        ref = b.walk_dump(0, lists=True)
+    for key, value in ref.items():  # the lists' order is that of the cells
+        assert np.array_equal(got[key], value), key
+
+
+def test_autotune_of_a_replaced_scene():
+    with _replaced() as b:
+        b.autotune(2)
+        assert b.grid_info(0)[0] == 0.5
