@@ -11,6 +11,7 @@
 namespace sph {
 
 constexpr uint32_t kMaxParticles = 1u << 30;
+constexpr uint64_t kMaxCells = 1ull << 31;  // of all scenes together
 
 // Automatic cell size (SPH_SCENE_AUTO_GRID): before a scene's first step
 // and every kRegridEvery steps after that (kRegridClumped below), the

@@ -78,12 +78,14 @@ void scene_grid(BatchScene &b, double pmin[3], double pmax[3])
     (void)scene_regrid(b, 0.0);  // desc.cell_scale was validated
 }
 
+// Cells a scene of n particles may have, at most, on any grid.
+static uint64_t max_cells(uint32_t n) { return std::max<uint64_t>(64ull * n, 1ull << 16); }
+
 int scene_regrid(BatchScene &b, double scale)
 {
     if (!(scale > 0.0))
         scale = b.desc.cell_scale > 0.0f ? (double)b.desc.cell_scale : 1.0;
-    const uint64_t max_cells = std::max<uint64_t>(64ull * b.desc.n, 1ull << 16);
-    return make_grid(b.P, b.lo, b.hi, scale, max_cells);
+    return make_grid(b.P, b.lo, b.hi, scale, max_cells(b.desc.n));
 }
 
 void Batch::drop_graph()
@@ -317,11 +319,16 @@ int Batch::upload(uint32_t s, const float *pos, const float *vel)
     // runs here rather than inside the first step.  When a scene of several
     // is replaced later, the others may follow: then the next call that needs
     // it does it, once (64 scenes, each preparing all of them again: 13 ms).
-    for (const BatchScene &o : scenes)
+    // Not where the scenes could have more cells than there may be: what is
+    // refused is refused here.
+    uint64_t most = 0;
+    for (const BatchScene &o : scenes) {
         if (!o.uploaded)
             return SPH_OK;
+        most += max_cells(o.desc.n);
+    }
     deferred = true;
-    if (complete && scenes.size() > 1)
+    if (complete && scenes.size() > 1 && most <= kMaxCells)
         return SPH_OK;
     complete = true;
     rc = settle();
@@ -389,7 +396,7 @@ int Batch::prepare()
         for (BatchScene &b : scenes) {
             b.P.cell_base = (uint32_t)base;
             base += (uint64_t)b.P.nx * b.P.ny * b.P.nz;
-            if (base > (1ull << 31))
+            if (base > kMaxCells)
                 return fail(SPH_E_LIMIT, "batch: %llu grid cells exceed the 2^31 limit", (unsigned long long)base);
             table.push_back(b.P);
         }

@@ -1,6 +1,6 @@
 """Replacing one scene of a batch leaves its grid, keys and automatic cell
 size to the next call that needs them: each such call sees what it would see
-after a first upload."""
+after a first upload, and what no grid can hold is refused by the upload."""
 import numpy as np
 import pytest
 
@@ -53,3 +53,28 @@ def test_autotune_of_a_replaced_scene():
     with _replaced() as b:
         b.autotune(2)
         assert b.grid_info(0)[0] == 0.5
+
+
+def test_upload_refuses_what_no_grid_holds():
+    """Two scenes of 17 million particles may have 64 cells a particle: both
+    spread out, 2^31.006 cells."""
+    n = 17_000_000
+    h = 0.01
+    s = A.settings(mass=1e-9, h=h)
+    edge = h * (1.0 + 2.0 ** -10)
+    # 1030 x 1023 x 1023 cells, one of them beside each wall: 63.4 a particle
+    size = np.array([1027.5, 1020.5, 1020.5]) * edge
+    box = A.box((0.0, 0.0, 0.0), (0.0, 0.0, 0.0))
+    pos = np.random.default_rng(1).random((n, 3), dtype=F32)
+    with A.Batch([A.scene_desc(n, s, box, 1e-3)] * 2) as b:
+        b.upload(0, pos)
+        b.upload(1, pos)
+        pos *= size.astype(F32)
+        pos[0], pos[1] = 0.0, size
+        b.upload(0, pos)
+        with pytest.raises(A.SphError) as err:
+            b.upload(1, pos)
+        assert err.value.code == A.SPH_E_LIMIT
+        with pytest.raises(A.SphError) as err:
+            b.step(1)
+        assert err.value.code == A.SPH_E_LIMIT
