@@ -81,6 +81,7 @@ struct Batch {
     DevBuf bounds;   // bounds of every scene's last upload
     HostStage stage;
     DevBuf gstat;    // grid statistic: candidates, neighbours per scene
+    bool hashes_kept = false;  // w.rankA holds the last step's hashes by A slot: the B order is a later sort's
     bool stat_ok = false;    // B order and cell ranges are those of the last step
     bool hold_grid = false;  // steps neither count nor re-grid (autotune trials)
     std::vector<hipEvent_t> events;

@@ -259,6 +259,7 @@ int Batch::relayout(std::vector<BatchScene> next, const std::vector<int> &from)
     scenes = std::move(next);
     total_n = (uint32_t)total;
     complete = false;
+    hashes_kept = false;
     layout_dirty = true;
     keys_dirty = true;
     stat_ok = false;
@@ -300,6 +301,8 @@ int Batch::upload(uint32_t s, const float *pos, const float *vel)
         return hip_fail(e, "upload");
     launch_load_state(stream, raw, vel ? raw_vel : nullptr, w.particles(),
                       keep_force ? (float4 *)w.force.ptr : nullptr, p0, n, (int32_t *)bounds.ptr + 6 * s);
+    if (hashes_kept)
+        launch_fill_u32(stream, (uint32_t *)w.rankA.ptr + p0, 0u, n);
     e = hipStreamSynchronize(stream);
     if (e == hipSuccess)
         e = hipGetLastError();
@@ -474,6 +477,11 @@ int Batch::grid_stat(std::vector<double> &ratio, bool fresh)
         const ParticleArrays a = w.particles();
         const CellArrays c = w.cells();
         const SceneSet S = w.scene_set();
+        // B slots are A's after a step, and hold the hashes it used: kept
+        // for downloads until the next one
+        if (!hashes_kept)
+            launch_keep_hashes(stream, a, total_n);
+        hashes_kept = true;
         launch_scan(stream, c, false);
         launch_scatter(stream, a, c, S);
         launch_sort_big_cells(stream, a, c);
@@ -642,6 +650,7 @@ int Batch::step_plain(int nsteps)
             return hip_fail(e, "step launch");
     }
     stat_ok = true;  // the B order and cell ranges are the last step's
+    hashes_kept = false;
     return SPH_OK;
 }
 
@@ -815,7 +824,7 @@ int Batch::download_particles(uint32_t s, sph_particle_v1 *out, float *transform
     const uint32_t n = scenes[s].desc.n, p0 = scenes[s].P.p_begin;
     if ((rc = aos.reserve(sizeof(sph_particle_v1) * (size_t)n)) || (transforms && (rc = xf.reserve(64ull * n))))
         return rc;
-    launch_pack_state(stream, w.particles(), keep_force ? (const float4 *)w.force.ptr : nullptr, p0, n,
+    launch_pack_state(stream, w.particles(), hashes_kept, keep_force ? (const float4 *)w.force.ptr : nullptr, p0, n,
                       scenes[s].P.xf_scale, aos.ptr, transforms ? (float *)xf.ptr : nullptr);
     const HostSpan spans[2] = {{out, aos.ptr, sizeof(sph_particle_v1) * (size_t)n}, {transforms, xf.ptr, 64ull * n}};
     return copy_to_host(stream, spans, transforms ? 2 : 1, stage);
@@ -837,6 +846,7 @@ int Batch::profile(int nsteps, double *ms, int max_k, int *nk, char *names_buf, 
         StepTimer t;
         enqueue(&t);
         stat_ok = true;
+        hashes_kept = false;
         if (!hold_grid)
             for (BatchScene &b : scenes)
                 ++b.steps;

@@ -6,7 +6,7 @@
 //     posA   float4  x, y, z, w = bits of the 16-bit bucket H16(getCell(x))
 //     velA   float4  vx, vy, vz, w = bits of the particle id
 //     cellcA u32     packed grid cell + slow-multiplicity flag
-//     rankA  u32     scratch (the drop-in output's 16-bit bucket ranks)
+//     rankA  u32     scratch (the drop-in output's 16-bit bucket ranks; a batch's kept hashes)
 //   "B" arrays: the same particles in grid-cell order (stable by A index)
 //     posB, velB, cellcB  as above
 //     rhoB   f32     density                          (density pass)
@@ -243,8 +243,11 @@ void launch_h16_scatter(hipStream_t st, const ParticleArrays &a, const CellArray
 void launch_pack_out(hipStream_t st, const ParticleArrays &a, const CellArrays &c16,
                      const uint32_t *perm16, const float4 *force, const void *aos_in, uint32_t n,
                      float xf_scale, void *aos_out, float *xf_out);
-// Resident download: AoS of slots [first, first + n) of the A state.
-void launch_pack_state(hipStream_t st, const ParticleArrays &a, const float4 *force, uint32_t first,
+// The hashes of B slots [0, n), to rankA.
+void launch_keep_hashes(hipStream_t st, const ParticleArrays &a, uint32_t n);
+// Resident download: AoS of slots [first, first + n) of the A state; the
+// hashes are those in B order, or kept ones.
+void launch_pack_state(hipStream_t st, const ParticleArrays &a, bool kept, const float4 *force, uint32_t first,
                        uint32_t n, float xf_scale, void *aos_out, float *xf_out);
 void launch_copy(hipStream_t st, const uint4 *src, uint4 *dst, size_t n16);
 

@@ -3153,9 +3153,10 @@ void launch_pack_out(hipStream_t st, const ParticleArrays &a, const CellArrays &
 // order).  Bucket, density and pressure belong to the last step (B slot s is
 // the same particle).
 __global__ void k_pack_state(const float4 *__restrict__ posA, const float4 *__restrict__ velA,
-                             const float4 *__restrict__ posB, const float *__restrict__ rhoB,
-                             const float4 *__restrict__ velR, const float4 *__restrict__ force,
-                             float *__restrict__ aos_out, float *__restrict__ xf_out, uint32_t first,
+                             const float4 *__restrict__ posB, const uint32_t *__restrict__ kept,
+                             const float *__restrict__ rhoB, const float4 *__restrict__ velR,
+                             const float4 *__restrict__ force, float *__restrict__ aos_out,
+                             float *__restrict__ xf_out, uint32_t first,
                              uint32_t n, float sc)
 {
     uint32_t o = blockIdx.x * blockDim.x + threadIdx.x;
@@ -3179,16 +3180,29 @@ __global__ void k_pack_state(const float4 *__restrict__ posA, const float4 *__re
     dst[11] = f.z;
     dst[12] = rhoB[s];
     dst[13] = velR[s].w;
-    dst[14] = __uint_as_float(__float_as_uint(posB[s].w) & 0xFFFFu);
+    dst[14] = __uint_as_float(kept ? kept[s] : __float_as_uint(posB[s].w) & 0xFFFFu);
     if (xf_out)
         write_transform(xf_out + (size_t)o * 16, x.x, x.y, x.z, sc);
 }
 
-void launch_pack_state(hipStream_t st, const ParticleArrays &a, const float4 *force, uint32_t first,
+__global__ void k_keep_hashes(const float4 *__restrict__ posB, uint32_t *__restrict__ kept, uint32_t n)
+{
+    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s < n)
+        kept[s] = __float_as_uint(posB[s].w) & 0xFFFFu;
+}
+
+void launch_keep_hashes(hipStream_t st, const ParticleArrays &a, uint32_t n)
+{
+    hipLaunchKernelGGL(k_keep_hashes, dim3(blocks_for(n)), dim3(kBlock), 0, st, a.posB, a.rankA, n);
+}
+
+void launch_pack_state(hipStream_t st, const ParticleArrays &a, bool kept, const float4 *force, uint32_t first,
                        uint32_t n, float xf_scale, void *aos_out, float *xf_out)
 {
     hipLaunchKernelGGL(k_pack_state, dim3(blocks_for(n)), dim3(kBlock), 0, st, a.posA, a.velA,
-                       a.posB, a.rhoB, a.velR, force, (float *)aos_out, xf_out, first, n, xf_scale);
+                       a.posB, kept ? a.rankA : nullptr, a.rhoB, a.velR, force, (float *)aos_out, xf_out, first, n,
+                       xf_scale);
 }
 
 // ------------------------------------------------------------------ copy

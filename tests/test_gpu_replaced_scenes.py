@@ -1,6 +1,7 @@
 """Replacing one scene of a batch leaves its grid, keys and automatic cell
 size to the next call that needs them: each such call sees what it would see
-after a first upload, and what no grid can hold is refused by the upload."""
+after a first upload, the other scenes' particles keep what the last step left
+them, and what no grid can hold is refused by the upload."""
 import numpy as np
 import pytest
 
@@ -53,6 +54,30 @@ def test_autotune_of_a_replaced_scene():
     with _replaced() as b:
         b.autotune(2)
         assert b.grid_info(0)[0] == 0.5
+
+
+def test_other_scenes_keep_their_hashes():
+    with _replaced() as b:
+        b.step(1)
+        before = b.download_particles(1)[0]
+        assert len(np.unique(before["hash"])) > 1
+        b.upload(0, _lattice())
+        for query in (lambda: b.grid_info(0), lambda: b.walk_dump(0), lambda: b.grid_info(1)):
+            query()
+            assert b.download_particles(1)[0].tobytes() == before.tobytes()
+            assert not b.download_particles(0)[0]["hash"].any()  # no step yet
+        b.upload(0, _lattice(9))
+        assert b.grid_info(0)[0] == 0.5
+        assert b.download_particles(1)[0].tobytes() == before.tobytes()
+        assert not b.download_particles(0)[0]["hash"].any()
+        b.upload(1, *_cloud(3000, 6))
+        assert not b.download_particles(1)[0]["hash"].any()
+        b.step(1)
+        fresh = b.download_particles(1)[0]
+    with A.Context(3000, S, BOX, 1e-3) as c:
+        c.upload(*_cloud(3000, 6))
+        c.step(1)
+        assert c.download_particles()[0].tobytes() == fresh.tobytes()
 
 
 def test_upload_refuses_what_no_grid_holds():
