@@ -205,8 +205,12 @@ int sph_hip_download_particles(sph_ctx *ctx, sph_particle_v1 *out,
  * particle id: count[i] = neighbours with multiplicity (the terms the
  * reference sums, src/sph.cpp:40-66); walk[i] (may be NULL) = bit 0: its
  * wave task walks the union of its lanes' stencils together (one candidate
- * at a time, or staged on chip), bit 1: the task is split into parts, bit 2: a neighbour list was recorded; list_count[i]
- * (may be NULL) = list entries or 0xFFFFFFFF; list (may be NULL): 64
+ * at a time, or staged on chip), bit 1: the task is split into parts, bit 2:
+ * a neighbour list was recorded, bit 3: staged on chip, its density summed by
+ * the planning pass, bit 4: what walks candidates after that pass (density
+ * without bit 3, force without bit 2) walks them one at a time for the whole
+ * wave, bit 5: those of each x-row of the wave's cells for its own lanes;
+ * list_count[i] (may be NULL) = list entries or 0xFFFFFFFF; list (may be NULL): 64
  * entries per id, the listed neighbours' ids (each once) in walk order. */
 int sph_hip_walk_dump(sph_ctx *ctx, uint32_t *count, uint32_t *walk,
                       uint32_t *list_count, uint32_t *list);

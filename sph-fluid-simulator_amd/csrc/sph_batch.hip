@@ -951,8 +951,11 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
         if (id >= n)
             return fail(SPH_E_HIP, "walk_dump: slot %u holds id %u of %u", q, id, n);
         count[id] = cnt[q];
-        if (walk)
-            walk[id] = (wk[2 * t + 1].w & (int)kWalkUnion ? 1u : 0u) | (parts[t] ? 2u : 0u) | (lc[q] != kNoList ? 4u : 0u);
+        if (walk) {
+            const uint32_t w = (uint32_t)wk[2 * t + 1].w;
+            walk[id] = (w & kWalkUnion ? 1u : 0u) | (parts[t] ? 2u : 0u) | (lc[q] != kNoList ? 4u : 0u) |
+                       (w & kWalkSummed ? 8u : 0u) | (w & kWalkBox ? 16u : 0u) | (w & kWalkSegments ? 32u : 0u);
+        }
         if (list_count)
             list_count[id] = lc[q];
         if (list && lc[q] != kNoList)

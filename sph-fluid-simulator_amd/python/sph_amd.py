@@ -407,6 +407,7 @@ def _walk_dump(fn, n: int, lists: bool):
     lst = np.zeros((n, LIST_MAX), np.uint32) if lists else None
     _check(fn(_ptr(count), _ptr(walk), _ptr(lcount), _ptr(lst)))
     return {"count": count, "union": (walk & 1) != 0, "split": (walk & 2) != 0, "listed": (walk & 4) != 0,
+            "staged": (walk & 8) != 0, "box": (walk & 16) != 0, "segments": (walk & 32) != 0,
             "list_count": lcount, "list": lst}
 
 
