@@ -913,8 +913,7 @@ int Batch::walk_dump(uint32_t s, uint32_t *count, uint32_t *walk, uint32_t *list
     launch_sort_big_cells(stream, a, c);
     launch_reorder(stream, a, c, S);
     launch_plan_parts(stream, a, c, S, pp, nl, (uint32_t *)tcount.ptr);
-    NeighborDump d{(uint32_t *)tcount.ptr, nullptr, nullptr, true};
-    launch_density(stream, a, c, S, &d, &pp, kStencilBlock, &nl);
+    launch_density(stream, a, c, S, pp, nl, kStencilBlock, (uint32_t *)tcount.ptr);
 
     const BatchScene &b = scenes[s];
     const uint32_t n = b.desc.n, p0 = b.P.p_begin;

@@ -157,22 +157,19 @@ struct NeighborLists;
 void launch_plan_parts(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
                        const PartPlan &pp, const NeighborLists &nl, uint32_t *count = nullptr);
 
-// Debug outputs of the density pass: per-particle neighbour count (with
+// Debug outputs of a density walk: per-particle neighbour count (with
 // multiplicity) and, when out != nullptr, the neighbour ids of row s at
-// out[off[s] ...].  With `production` set, only the count is written, by
-// the production walks of the step (part plan, union / per-lane / split
-// parts, neighbour lists) instead of a separate whole-stencil walk.
+// out[off[s] ...].
 struct NeighborDump {
     uint32_t *count;
     const uint64_t *off;
     uint32_t *out;
-    bool production = false;
 };
 
-// Neighbour lists.  The density pass records, for every particle of an
-// unsplit wave task, the slots of its neighbours (each once, in walk order: rows z-major, then y, slots
-// ascending) when there are at most kListMax of them; the force pass then
-// visits exactly those slots instead of filtering the stencil again.  The
+// Neighbour lists.  The planning and density passes record, for every particle
+// of an unsplit wave task, the slots of its neighbours (each once, in walk
+// order: rows z-major, then y, slots ascending) when there are at most kListMax
+// of them; the force pass then visits exactly those slots instead of filtering the stencil again.  The
 // order is the per-lane walk's, so the force sums are the same bit for bit.
 // Entry k of slot s lives at list[k stride + s]: the lanes of a wave
 // that append their k-th neighbour together write one contiguous run, so
@@ -212,19 +209,20 @@ void launch_scatter(hipStream_t st, const ParticleArrays &a, const CellArrays &c
 // Sorts the A indices of every listed big cell (deterministic in-cell order).
 void launch_sort_big_cells(hipStream_t st, const ParticleArrays &a, const CellArrays &c);
 void launch_reorder(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S);
-// `block`: threads per block of the stencil passes, 64, 128 or 256 (the
-// dump modes always use kStencilBlock); results do not depend on it.
-// `parts` (may be null: every wave task unsplit, one wave each) is the
-// plan launch_plan_parts made for this step.
-// `lists` (may be null: none) receives the neighbour lists of the step;
-// the force pass reads the same.
+// The passes over what the planning pass left: `parts` is the plan
+// launch_plan_parts made for this step, `lists` receives the neighbour lists
+// of the step's other tasks, and the force pass reads them.  `block`: threads
+// per block, 64, 128 or 256; results do not depend on it.  `count` (may be
+// null; kStencilBlock then) receives neighbour counts with multiplicity.
 void launch_density(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
-                    const NeighborDump *dump, const PartPlan *parts = nullptr, int block = kStencilBlock,
-                    const NeighborLists *lists = nullptr);
+                    const PartPlan &parts, const NeighborLists &lists, int block = kStencilBlock,
+                    uint32_t *count = nullptr);
 void launch_force_integrate(hipStream_t st, const ParticleArrays &a, const CellArrays &c,
                             const SceneSet &S, float4 *force_out, bool next_keys,
-                            const PartPlan *parts = nullptr, int block = kStencilBlock,
-                            const NeighborLists *lists = nullptr);
+                            const PartPlan &parts, const NeighborLists &lists, int block = kStencilBlock);
+// Densities, and the dump, from every lane's whole stencil, without a plan.
+void launch_neighbor_dump(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
+                          const NeighborDump &dump);
 // Sampled candidates per neighbour of every scene (one wave task in
 // kGridStatEvery of each scene), from the current B order and cell ranges:
 // stat[2 s] = candidates, stat[2 s + 1] = neighbours of scene s (cleared

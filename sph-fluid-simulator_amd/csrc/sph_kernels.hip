@@ -84,18 +84,6 @@ __device__ inline void wave_task(const SceneSet &S, uint32_t w, Lane &out, bool 
     out.slot = active ? slot : first;
 }
 
-// As lane_of, but with every lane of a live wave live (see wave_task).
-// Returns false only for waves past the task list (the whole wave).
-template <int BLOCK>
-__device__ inline bool wave_lanes(const SceneSet &S, Lane &out, bool &active)
-{
-    const uint32_t w = __builtin_amdgcn_readfirstlane(xcd_block() * (BLOCK / 64) + (threadIdx.x >> 6));
-    if (w >= S.nwaves)
-        return false;
-    wave_task(S, w, out, active);
-    return true;
-}
-
 inline uint32_t blocks_for_waves(uint32_t nwaves, int block) { return (nwaves + block / 64 - 1) / (block / 64); }
 
 // Waves the device holds at once: CUs x 4 SIMDs x 8 wave slots.
@@ -2575,44 +2563,34 @@ static uint32_t occupancy_waves(const void *kernel, int block)
     return std::min<uint32_t>(resident_waves(), (uint32_t)nb * (uint32_t)(block / 64) * (resident_waves() / 32u));
 }
 
-// Waves of a stencil pass: one per wave task without a plan; with one, a
-// persistent grid of the waves the device holds at once for this kernel
-// (a wave launched beyond them would start only as the first ones finish,
-// with a full share of a static assignment), and at most 4 per wave task
-// (more would only pull from an empty queue: a small scene splits into
-// about as many parts as it has wave tasks).
-inline uint32_t stencil_waves(const SceneSet &S, const PartPlan *pp, uint32_t resident)
+// Waves of a stencil pass with a plan: a persistent grid of the waves the
+// device holds at once for this kernel (a wave launched beyond them would
+// start only as the first ones finish, with a full share of a static
+// assignment), and at most 4 per wave task (more would only pull from an
+// empty queue: a small scene splits into about as many parts as it has wave
+// tasks).
+inline uint32_t stencil_waves(const SceneSet &S, const PartPlan &pp, uint32_t resident)
 {
-    if (!pp)
-        return S.nwaves;
-    return std::min<uint32_t>(std::min<uint32_t>(pp->cap, resident), 4u * std::max(S.nwaves, 1u));
+    return std::min<uint32_t>(std::min<uint32_t>(pp.cap, resident), 4u * std::max(S.nwaves, 1u));
 }
 
 template <int MODE, int BLOCK>
 static void launch_density_block(hipStream_t st, const ParticleArrays &a, const CellArrays &c,
-                                 const SceneSet &S, const NeighborDump &d, const PartPlan *pp,
-                                 const NeighborLists *lists)
+                                 const SceneSet &S, const NeighborDump &d, const PartPlan &pp,
+                                 const NeighborLists &nl)
 {
-    PartPlan p{};
-    if (pp)
-        p = *pp;
-    NeighborLists nl{nullptr, nullptr, 0u};
-    if (lists)
-        nl = *lists;
     static const uint32_t resident = occupancy_waves(reinterpret_cast<const void *>(&k_density<MODE, BLOCK>), BLOCK);
-    hipLaunchKernelGGL((k_density<MODE, BLOCK>), dim3(std::max(1u, blocks_for_waves(stencil_waves(S, pp, resident), BLOCK))),
-                       dim3(BLOCK), 0, st, a.posB, a.velB, a.cellcB, c.cstart, a.rhoB, a.posR, a.velR, S, d, p, nl);
+    const uint32_t waves = pp.queue ? stencil_waves(S, pp, resident) : S.nwaves;
+    hipLaunchKernelGGL((k_density<MODE, BLOCK>), dim3(std::max(1u, blocks_for_waves(waves, BLOCK))), dim3(BLOCK), 0, st,
+                       a.posB, a.velB, a.cellcB, c.cstart, a.rhoB, a.posR, a.velR, S, d, pp, nl);
 }
 
 void launch_density(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
-                    const NeighborDump *dump, const PartPlan *parts, int block, const NeighborLists *lists)
+                    const PartPlan &parts, const NeighborLists &lists, int block, uint32_t *count)
 {
-    NeighborDump d = dump ? *dump : NeighborDump{nullptr, nullptr, nullptr};
-    if (dump && dump->production)  // the step's own walks, plus the count
+    const NeighborDump d{count, nullptr, nullptr};
+    if (count)
         return launch_density_block<3, kStencilBlock>(st, a, c, S, d, parts, lists);
-    if (dump)  // the dump modes walk every lane's whole stencil in one task
-        return dump->out ? launch_density_block<2, kStencilBlock>(st, a, c, S, d, nullptr, nullptr)
-                         : launch_density_block<1, kStencilBlock>(st, a, c, S, d, nullptr, nullptr);
     switch (block) {
     case 64:
         return launch_density_block<0, 64>(st, a, c, S, d, parts, lists);
@@ -2621,6 +2599,16 @@ void launch_density(hipStream_t st, const ParticleArrays &a, const CellArrays &c
     default:
         return launch_density_block<0, kStencilBlock>(st, a, c, S, d, parts, lists);
     }
+}
+
+void launch_neighbor_dump(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
+                          const NeighborDump &dump)
+{
+    const NeighborLists none{nullptr, nullptr, 0u};
+    if (dump.out)
+        launch_density_block<2, kStencilBlock>(st, a, c, S, dump, PartPlan{}, none);
+    else
+        launch_density_block<1, kStencilBlock>(st, a, c, S, dump, PartPlan{}, none);
 }
 
 // ----------------------------------------------------- force + integrate
@@ -2718,10 +2706,10 @@ __device__ inline void force_pair(float d2, float dx, float dy, float dz, float 
 //    four at a time.  Bound by the gathers: on cells of h / 2, where the k-th
 //    neighbours of neighbouring lanes are neighbours, a million particles take
 //    91 us, on cells of h 155;
-//  * union: one wave-uniform candidate at a time, staged through LDS and
-//    clamped to a term of zeros where it is none of the lane's.  Bound by
+//  * union: candidates shared by the wave, 64 at a time through LDS and
+//    clamped to terms of zeros where they are none of the lane's.  Bound by
 //    arithmetic: in a late state of a million particles (3,260 neighbours
-//    each) 29 instructions, 79 cycles, a candidate and 90% of the issue slots;
+//    each) 29 instructions, 79 cycles, a candidate;
 //    4.0 ms with operands in scalar registers, a test and two
 //    transcendentals a candidate, 3.55 now;
 //  * per lane: candidates filtered kForceChunk at a time into a per-lane
@@ -2770,12 +2758,13 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
             }
             force_pair<false, false, false>(d2, dx, dy, dz, am, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
         };
-        // Every lane holds its neighbour list (the density pass walked this
-        // task per lane, unsplit): visit the listed slots four at a time,
-        // the next group of four slots loaded while the current one runs;
-        // entries past a lane's list stand for its own slot and add nothing.
-        const uint32_t listed = (nl.count && nparts == 1u) ? nl.count[s] : kNoList;
-        const bool use_list = nl.count && nparts == 1u && __all(listed != kNoList);
+        // Every lane holds its neighbour list (the task is unsplit; the
+        // planning pass or the density pass has recorded them): visit the
+        // listed slots four at a time, the next group of four slots loaded
+        // while the current one runs; entries past a lane's list stand for its
+        // own slot and add nothing.
+        const uint32_t listed = nparts == 1u ? nl.count[s] : kNoList;
+        const bool use_list = nparts == 1u && __all(listed != kNoList);
         UnionRows U;
         if (use_list) {
             const uint32_t groups = ((uint32_t)wave_max_i((int)listed) + 3u) >> 2;
@@ -2913,21 +2902,15 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
 
 template <int BLOCK>
 static void launch_force_block(hipStream_t st, const ParticleArrays &a, const CellArrays &c, const SceneSet &S,
-                               float4 *force_out, bool next_keys, const PartPlan *pp, const NeighborLists *lists)
+                               float4 *force_out, bool next_keys, const PartPlan &pp, const NeighborLists &nl)
 {
-    PartPlan p{};
-    if (pp)
-        p = *pp;
-    NeighborLists nl{nullptr, nullptr, 0u};
-    if (lists)
-        nl = *lists;
     static const uint32_t resident =
         occupancy_waves(reinterpret_cast<const void *>(&k_force_integrate<false, true, BLOCK>), BLOCK);
     dim3 g(std::max(1u, blocks_for_waves(stencil_waves(S, pp, resident), BLOCK))), b(BLOCK);
 #define SPH_LAUNCH_FI(WF, NK)                                                                          \
     hipLaunchKernelGGL((k_force_integrate<WF, NK, BLOCK>), g, b, 0, st, a.posB, a.velB, a.posR, a.velR, \
                        a.cellcB, c.cstart, a.rhoB, a.posA, a.velA, a.cellcA, c.counts,         \
-                       force_out, S, p, nl)
+                       force_out, S, pp, nl)
     if (force_out && next_keys)
         SPH_LAUNCH_FI(true, true);
     else if (force_out)
@@ -2940,8 +2923,8 @@ static void launch_force_block(hipStream_t st, const ParticleArrays &a, const Ce
 }
 
 void launch_force_integrate(hipStream_t st, const ParticleArrays &a, const CellArrays &c,
-                            const SceneSet &S, float4 *force_out, bool next_keys, const PartPlan *parts,
-                            int block, const NeighborLists *lists)
+                            const SceneSet &S, float4 *force_out, bool next_keys, const PartPlan &parts,
+                            const NeighborLists &lists, int block)
 {
     switch (block) {
     case 64:

@@ -279,8 +279,8 @@ int update_particles_noalloc(sph_particle_v1 *particles, float *transforms, size
     float4 *force = (float4 *)at(L.force);
     const NeighborLists nl{(uint32_t *)at(L.nlist), (uint32_t *)at(L.ncount), n};
     launch_plan_parts(st, a, c, set, pp, nl);
-    launch_density(st, a, c, set, nullptr, &pp, kStencilBlock, &nl);
-    launch_force_integrate(st, a, c, set, force, /*next_keys=*/false, &pp, kStencilBlock, &nl);
+    launch_density(st, a, c, set, pp, nl);
+    launch_force_integrate(st, a, c, set, force, /*next_keys=*/false, pp, nl);
 
     CellArrays c16;
     c16.counts = (uint32_t *)at(L.counts16);

@@ -706,10 +706,10 @@ void enqueue_step(hipStream_t st, Workspace &w, float4 *force_out, bool next_key
         timer->mark(st, "reorder");
     const NeighborLists nl = w.lists();
     launch_plan_parts(st, a, c, S, pp, nl);
-    launch_density(st, a, c, S, nullptr, &pp, w.stencil_block, &nl);
+    launch_density(st, a, c, S, pp, nl, w.stencil_block);
     if (timer)
         timer->mark(st, "density");
-    launch_force_integrate(st, a, c, S, force_out, next_keys, &pp, w.stencil_block, &nl);
+    launch_force_integrate(st, a, c, S, force_out, next_keys, pp, nl, w.stencil_block);
     if (timer)
         timer->mark(st, "force_integrate");
 }
@@ -871,8 +871,8 @@ int update_particles(sph_particle_v1 *particles, float *transforms, size_t n_,
     const PartPlan pp = w.part_plan();
     const NeighborLists nl = w.lists();
     launch_plan_parts(st, a, c, set, pp, nl);
-    launch_density(st, a, c, set, nullptr, &pp, kStencilBlock, &nl);
-    launch_force_integrate(st, a, c, set, (float4 *)w.force.ptr, /*next_keys=*/false, &pp, kStencilBlock, &nl);
+    launch_density(st, a, c, set, pp, nl);
+    launch_force_integrate(st, a, c, set, (float4 *)w.force.ptr, /*next_keys=*/false, pp, nl);
     CellArrays c16 = cells16(S);
     launch_fill_u32(st, c16.counts, 0u, 65536);
     launch_h16_rank(st, a, c16, n);
@@ -925,7 +925,7 @@ int neighbors(const sph_particle_v1 *particles, size_t n_, const sph_settings_v1
         return rc;
     SceneSet set = w.scene_set();
     NeighborDump d{(uint32_t *)dcount.ptr, nullptr, nullptr};
-    launch_density(st, a, c, set, &d);
+    launch_neighbor_dump(st, a, c, set, d);
     std::vector<uint32_t> cnt(n), ids(n);
     std::vector<float4> velB(n);
     hipError_t e = hipMemcpyAsync(cnt.data(), dcount.ptr, 4ull * n, hipMemcpyDeviceToHost, st);
@@ -967,7 +967,7 @@ int neighbors(const sph_particle_v1 *particles, size_t n_, const sph_settings_v1
     if (e != hipSuccess)
         return hip_fail(e, "neighbour offsets");
     NeighborDump d2{(uint32_t *)dcount.ptr, (const uint64_t *)doff.ptr, (uint32_t *)dout.ptr};
-    launch_density(st, a, c, set, &d2);
+    launch_neighbor_dump(st, a, c, set, d2);
     std::vector<uint32_t> rows(tot);
     e = hipMemcpyAsync(rows.data(), dout.ptr, 4ull * tot, hipMemcpyDeviceToHost, st);
     if (e == hipSuccess)
