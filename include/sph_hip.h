@@ -210,8 +210,9 @@ int sph_hip_download_particles(sph_ctx *ctx, sph_particle_v1 *out,
  * the planning pass, bit 4: what walks candidates after that pass (density
  * without bit 3, force without bit 2) walks them one at a time for the whole
  * wave, bit 5: those of each x-row of the wave's cells for its own lanes;
- * list_count[i] (may be NULL) = list entries or 0xFFFFFFFF; list (may be NULL): 64
- * entries per id, the listed neighbours' ids (each once) in walk order. */
+ * list_count[i] (may be NULL) = list entries or 0xFFFFFFFF; list (may be
+ * NULL): 64 entries per id, the listed neighbours' ids (each once) in walk
+ * order. */
 int sph_hip_walk_dump(sph_ctx *ctx, uint32_t *count, uint32_t *walk,
                       uint32_t *list_count, uint32_t *list);
 /* The scene's current cell scale (in units of h (1 + 2^-10)) and the
@@ -244,6 +245,10 @@ typedef struct sph_batch sph_batch;
 int sph_batch_create(const sph_scene_desc_v1 *descs, uint32_t nscenes,
                      sph_batch **out);
 int sph_batch_destroy(sph_batch *b);
+/* Replacing a scene of a batch that has run leaves its grid, and the
+ * automatic choice of it, to the next call that needs them (a step, grid_info,
+ * walk_dump, profile, autotune), so that replacing many costs that once; that
+ * call then reports what it cannot allocate. */
 int sph_batch_upload(sph_batch *b, uint32_t scene, const float *pos,
                      const float *vel);
 int sph_batch_step(sph_batch *b, int nsteps);

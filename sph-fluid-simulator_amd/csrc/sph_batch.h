@@ -36,8 +36,11 @@ constexpr double kToCoarseRatio = 4.0;  // at cell scale 1/2: below this, go to 
 constexpr double kClumpedRatio = 4.0;
 constexpr uint64_t kRegridClumped = 256;
 // Smaller scenes keep cells of h: on the batched workload (256 scenes of
-// 1k-64k particles) cells of h / 2 made the 500-step job 26% slower (eight
-// times the cells to scan, and no faster density pass at these sizes).
+// 1k-64k particles) cells of h / 2 made the 500-step job 26% slower.  That job
+// and the thresholds above were timed before short walks were staged on either
+// grid; since then, with all scenes of a batch on one size, cells of h / 2 take
+// 1.41 ms a step from the job's initial states and 2.26 from its last ones,
+// cells of h 1.51 and 1.38.
 constexpr uint32_t kAutoGridMinParticles = 1u << 17;
 
 struct BatchScene {

@@ -1437,9 +1437,11 @@ __device__ inline void plan_walk(const uint32_t *__restrict__ cstart, uint32_t c
 // others left in LDS.
 // Measured, planning and density of a step together, walked from memory and
 // staged: 8,000 particles 65 and 23 us, 64 scenes of 1.06 million in all 263
-// and 195 us.  What bounds those is the arithmetic (111 M vector
-// instructions in all; finding neighbours and adding their terms in order
-// are about equal shares); below some thousand tasks, the latency of one wave.
+// and 195 us.  What bounds those is arithmetic and waiting about equally (90 M
+// vector instructions for a lattice of a million, finding neighbours and adding
+// their terms in order about equal shares: 0.45 of the issue slots at two
+// cycles each; three waves a SIMD that wait 40% of their time); below some
+// thousand tasks, the latency of one wave.
 // (Adding each layer's terms in its own wave takes 19 and 151 us, but then
 // the sums are not the per-lane walk's, and over a run of steps the particles
 // that meet a wall bounce a step apart.)
@@ -1774,9 +1776,10 @@ __global__ __launch_bounds__(STAGED ? 192 : 64) void k_plan_list(
 // after the next layer has arrived, so that no load waits for the list's
 // stores.  Planned and walked here, against planned and walked from memory in
 // k_density: 262 thousand particles 62 us and 26 + 86, a million 157 and
-// 30 + 150.  What bounds it is the arithmetic (57 M vector instructions, two
-// thirds of the issue slots at the twelve waves a CU that registers and LDS
-// allow).
+// 30 + 150.  What bounds it is waiting at low occupancy: 163 registers let
+// three waves onto a SIMD, 2.2 are there on average, and they spend 44% of
+// their time waiting for LDS and memory, 27% in vector instructions (58 M for
+// a million particles: 0.29 of the issue slots at two cycles each).
 // Tasks in many rows (a surface), whose layers don't fit the room, walk from
 // memory here (in k_density, behind the others, the latency of a few hundred
 // such waves was 40 us); those with a row of more than kFineRow candidates in a lane's
@@ -2709,7 +2712,8 @@ __device__ inline void force_pair(float d2, float dx, float dy, float dz, float 
 //  * union: candidates shared by the wave, 64 at a time through LDS and
 //    clamped to terms of zeros where they are none of the lane's.  Bound by
 //    arithmetic: in a late state of a million particles (3,260 neighbours
-//    each) 29 instructions, 79 cycles, a candidate;
+//    each) 29 instructions, 79 cycles, a candidate: 0.70 of the issue slots at
+//    two cycles each, and this mix takes 2.7;
 //    4.0 ms with operands in scalar registers, a test and two
 //    transcendentals a candidate, 3.55 now;
 //  * per lane: candidates filtered kForceChunk at a time into a per-lane
