@@ -2672,7 +2672,7 @@ __device__ inline void integrate_and_walls(float4 &x, float4 &v, float fx, float
 // CLAMP: also for candidates that are no neighbours, where h2 = fl(h h): they
 // have d2 >= h2, so r >= h (the root of the rounded square is h itself) and
 // h - r clamps to 0: they add zeros, without a test.  (With another h2 a
-// neighbour may be farther than h, and h - r below zero.)
+// neighbour may be farther than h, and h - r below zero.)  For split walks.
 // SPLIT: the part of a split walk, whose sums depend on the parts' bounds
 // anyway: the same product in an order that takes fewer operations and root()
 // (28 against 49 issue cycles a wave before the six fmas).  Unsplit walks
@@ -2710,8 +2710,8 @@ __device__ inline void force_pair(float d2, float dx, float dy, float dz, float 
 //    neighbours of neighbouring lanes are neighbours, a million particles take
 //    91 us, on cells of h 155;
 //  * union: candidates shared by the wave, 64 at a time through LDS and
-//    clamped to terms of zeros where they are none of the lane's.  Bound by
-//    arithmetic: in a late state of a million particles (3,260 neighbours
+//    tested, or in split walks clamped to terms of zeros where they are none
+//    of the lane's.  Bound by arithmetic: in a late state of a million particles (3,260 neighbours
 //    each) 29 instructions, 79 cycles, a candidate: 0.70 of the issue slots at
 //    two cycles each, and this mix takes 2.7;
 //    4.0 ms with operands in scalar registers, a test and two
@@ -2812,6 +2812,13 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
             const float limit = P.zero_limit;
             const bool plain = __all(fabsf(pi.x) + fabsf(pi.y) + fabsf(pi.z) + fabsf(vi.x) + fabsf(vi.y) +
                                          fabsf(vi.z) + fabsf(p_i) <= limit);
+            // A test also lets the wave skip a candidate that is no lane's
+            // neighbour.  That pays in unsplit walks, whose pair terms are the
+            // dearer ones (a lattice of spacing 0.4 h, 97 thousand particles:
+            // 281 us without, 212 with), and on cells much larger than h, where
+            // two thirds of the candidates are such (spacing h / 2 on cells of
+            // 1.7 h, 262 thousand: 336 and 232).
+            const bool tested = !plain || (P.reach == 1 && P.grid_inv * (double)P.h < 0.8);
             const uint32_t W = 2u * (uint32_t)P.reach + 1u;
             uint32_t at_layer = kNoSlot;
             bool mine = true;  // the chunk's candidates are those of the lane's segment
@@ -2825,12 +2832,25 @@ __global__ __launch_bounds__(BLOCK, 5) void k_force_integrate(
                         at_layer = lz;
                         mine = T.segment[threadIdx.x & 63u] == lz / W;
                     }
-                    if (odd || !plain) {
-                        for (uint32_t k = 0; k < n; ++k) {
-                            const float4 q = rec[0][k], w = rec[1][k];  // (x_j, 0.5 / rho_j), (v_j, p_j)
-                            const float d2 = dist2_ref(pi, q, dx, dy, dz);
-                            if (d2 < h2 && mine && slots[k] != s && slots[k] != kNoSlot)
-                                force_pair<false, unit, split>(d2, dx, dy, dz, q.w, w, vi, p_i, h, neg_m_spg, mu2_m_lap, fx, fy, fz);
+                    if (!split || odd || tested) {
+                        for (uint32_t k = 0; k < n; k += 4u) {
+                            float4 q[4], w[4];  // (x_j, 0.5 / rho_j), (v_j, p_j)
+#pragma unroll
+                            for (uint32_t i = 0; i < 4u; ++i) {
+                                q[i] = rec[0][k + i];
+                                w[i] = rec[1][k + i];
+                            }
+                            const uint4 j = *reinterpret_cast<const uint4 *>(&slots[k]);
+                            auto visit = [&](uint32_t slot, const float4 &qi, const float4 &wi) {
+                                const float d2 = dist2_ref(pi, qi, dx, dy, dz);
+                                if (d2 < h2 && mine && slot != s && slot != kNoSlot)
+                                    force_pair<false, unit, split>(d2, dx, dy, dz, qi.w, wi, vi, p_i, h, neg_m_spg, mu2_m_lap,
+                                                                   fx, fy, fz);
+                            };
+                            visit(j.x, q[0], w[0]);
+                            visit(j.y, q[1], w[1]);
+                            visit(j.z, q[2], w[2]);
+                            visit(j.w, q[3], w[3]);
                         }
                         return;
                     }
