@@ -2347,37 +2347,70 @@ __global__ __launch_bounds__(BLOCK, 6) void k_density(
                         else
                             acc = acc + mp6 * ((t * t) * t);
                     };
-                    if ((!split && listing) || odd) {
-                        for (uint32_t k = 0; k < n; ++k) {
-                            const uint32_t j = slots[k];
-                            const float t = j != s ? term(c.x[k], c.y[k], c.z[k]) : 0.0f;
-                            add(t);
-                            if (t > 0.0f) {
-                                if (kCount)
-                                    ++cnt;
-                                if (listing && nn < kListMax) {
-                                    *lp = j;
-                                    lp += nl.stride;
-                                }
-                                ++nn;
-                            }
-                        }
-                        listing = listing && !__any(nn > kListMax);
-                        return;
-                    }
-                    for (uint32_t k = 0; k < n; k += 4u) {
+                    // candidates k .. k + 3, each given to visit in turn
+                    auto four = [&](uint32_t k, auto self_tag, auto visit) {
                         const float4 x = *reinterpret_cast<const float4 *>(&c.x[k]);
                         const float4 y = *reinterpret_cast<const float4 *>(&c.y[k]);
                         const float4 z = *reinterpret_cast<const float4 *>(&c.z[k]);
-                        const float t[4] = {term(x.x, y.x, z.x), term(x.y, y.y, z.y), term(x.z, y.z, z.z),
-                                            term(x.w, y.w, z.w)};
+                        float t[4] = {term(x.x, y.x, z.x), term(x.y, y.y, z.y), term(x.z, y.z, z.z),
+                                      term(x.w, y.w, z.w)};
+                        if (decltype(self_tag)::value) {
+                            const uint4 j = *reinterpret_cast<const uint4 *>(&slots[k]);
+                            t[0] = j.x != s ? t[0] : 0.0f;
+                            t[1] = j.y != s ? t[1] : 0.0f;
+                            t[2] = j.z != s ? t[2] : 0.0f;
+                            t[3] = j.w != s ? t[3] : 0.0f;
+                        }
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             add(t[i]);
-                            if (kCount)
-                                cnt += t[i] > 0.0f ? 1u : 0u;
+                            visit(t[i]);
                         }
+                    };
+                    if (!split && listing) {
+                        // Neighbours are marked as they pass (two operations a
+                        // candidate) and appended 32 candidates at a time.
+                        // (With a branch and a store for each: a lattice of
+                        // spacing 0.4 h, 97 thousand particles, 173 us instead
+                        // of 151, spacing h / 2 on cells of 1.7 h, 262
+                        // thousand, 267 instead of 217.)
+                        for (uint32_t k0 = 0; k0 < n; k0 += 32u) {
+                            const uint32_t m = min(32u, n - k0);
+                            uint32_t bits = 0;
+                            auto mark = [&](float t) {  // << 1 | (t > 0)
+                                bits = __builtin_amdgcn_alignbit(bits, 0u - __float_as_uint(t), 31u);
+                            };
+                            if (odd)
+                                for (uint32_t k = 0; k < m; k += 4u)
+                                    four(k0 + k, std::true_type{}, mark);
+                            else
+                                for (uint32_t k = 0; k < m; k += 4u)
+                                    four(k0 + k, std::false_type{}, mark);
+                            bits <<= 32u - m;  // the first on top
+                            if (kCount)
+                                cnt += (uint32_t)__builtin_popcount(bits);
+                            for (; bits != 0u; ++nn) {
+                                const uint32_t k = (uint32_t)__builtin_clz(bits);
+                                bits &= ~(0x80000000u >> k);
+                                if (nn < kListMax) {
+                                    *lp = slots[k0 + k];
+                                    lp += nl.stride;
+                                }
+                            }
+                        }
+                        listing = !__any(nn > kListMax);
+                        return;
                     }
+                    auto pass = [&](float t) {
+                        if (kCount)
+                            cnt += t > 0.0f ? 1u : 0u;
+                    };
+                    if (odd)
+                        for (uint32_t k = 0; k < n; k += 4u)
+                            four(k, std::true_type{}, pass);
+                    else
+                        for (uint32_t k = 0; k < n; k += 4u)
+                            four(k, std::false_type{}, pass);
                 });
             };
             if (nparts == 1u) {

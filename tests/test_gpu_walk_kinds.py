@@ -167,3 +167,46 @@ def test_values_in_segment_walks_stay_where_they_belong(sph, value):
         assert np.array_equal(got[0][key], got[1][key], equal_nan=True), key
     assert not np.isfinite(got[0]["force"]).all() or np.isfinite(value)
     assert np.isfinite(got[0]["force"]).any()
+
+
+@pytest.mark.parametrize("cell_scale", [1.7, 2.0, 2.6])
+@pytest.mark.parametrize("spacing", [0.5, 0.64, 0.9])
+def test_union_walks_that_record_lists(sph, orc32, spacing, cell_scale):
+    """Whole union walks of the density pass with lists of a few to some thirty
+    neighbours (cells larger than h, too many candidates to be staged): lists,
+    counts and densities are the oracle's, sums the per-lane walk's bit for bit
+    where that one is not split either."""
+    h = 0.1
+    g = np.stack(np.meshgrid(*[np.arange(12)] * 3, indexing="ij"), -1).reshape(-1, 3) * spacing * h
+    pos = g + np.random.default_rng(7).uniform(-0.1, 0.1, g.shape) * spacing * h + [0.83, 0.71, -1.94]
+    sc = test_gpu_staged_walk._scene(pos)
+    dump = _dump(sph, sc, cell_scale)
+    whole = dump["box"] & ~dump["staged"] & ~dump["split"] & dump["listed"]
+    if 409 < 27 * (cell_scale / spacing) ** 3 < 800:  # too long to be staged, short enough to be left whole
+        assert whole.any(), "premise: whole union walks with lists"
+    out = []
+    for lane_walk in (False, True):
+        with sph.Context(sc.n, sph.settings(*sc.settings_args()), sph.box(sc.box_lo, sc.box_hi), sc.dt,
+                         cell_scale=cell_scale, lane_walk=lane_walk) as ctx:
+            ctx.upload(sc.pos, sc.vel)
+            d = ctx.walk_dump(lists=True)
+            ids = np.arange(sc.n)
+            ost = test_gpu_union_walk.OracleState(orc32, sc, sc.pos, sc.vel)
+            try:
+                test_gpu_union_walk._check_dump(d, ost.rows(ids), ids, f"lane_walk={lane_walk}")
+                ost.forces(ids[:1])  # computes the densities
+                rho, prs = ost.rho_p_by_id()
+            finally:
+                ost.close()
+            ctx.step(1)
+            got = ctx.download()
+            by_id = {k: np.zeros_like(got[k]) for k in ("rho", "pressure")}
+            for k in by_id:
+                by_id[k][got["ids"]] = got[k]
+            test_gpu_union_walk.pu.assert_rho_p(by_id["rho"], by_id["pressure"], rho, prs, ost.s)
+            out.append((d, got))
+    assert np.array_equal(out[0][1]["ids"], out[1][1]["ids"])
+    ids = out[0][1]["ids"]
+    same = ~(out[0][0]["split"] | out[1][0]["split"])[ids]
+    for key in ("rho", "pressure"):
+        assert out[0][1][key][same].tobytes() == out[1][1][key][same].tobytes(), key
