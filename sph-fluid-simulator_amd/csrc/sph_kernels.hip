@@ -2149,12 +2149,10 @@ void launch_plan_parts(hipStream_t st, const ParticleArrays &a, const CellArrays
 
 // Runs task(w, part, nparts) for the work the calling wave takes.  Without
 // a plan each wave runs wave task w of its own index, unsplit.  With one,
-// each wave first runs its static, XCD-contiguous share of the unsplit
-// tasks -- wave v takes tasks v, v + G, ... that are not split, with no
-// queue traffic, neighbouring tasks sharing an L2 -- then pulls the parts
-// of split tasks from the queue counter until that list is exhausted
-// (every wave exits then), which also evens out the static share.  All 64
-// lanes must be live on entry.
+// each wave first runs its static share of the unsplit tasks, with no queue
+// traffic, neighbouring tasks on one XCD sharing its L2, then parts of split
+// tasks until there are none left (every wave exits then), which also evens
+// out the static share.  All 64 lanes must be live on entry.
 // skip_summed: leave out the tasks whose sums the planning pass made.
 template <int BLOCK, bool skip_summed, class Task>
 __device__ inline void for_each_part(const SceneSet &S, const PartPlan &pp, uint32_t *queue, Task task)
@@ -2166,24 +2164,65 @@ __device__ inline void for_each_part(const SceneSet &S, const PartPlan &pp, uint
         return;
     }
     const uint32_t total = __builtin_amdgcn_readfirstlane(pp.queue[2]);  // parts of split tasks
-    const uint32_t G = gridDim.x * (BLOCK / 64);
-    for (uint32_t w = first; w < S.nwaves; w += G)
+    constexpr uint32_t kWaves = BLOCK / 64;
+    const uint32_t G = gridDim.x * kWaves;
+    // G tasks at a time, each XCD a contiguous share of them in proportion to
+    // its waves (blocks go round the XCDs).  Fewer tasks than waves are spread
+    // over all XCDs so; dealt by wave index, contiguous on each XCD too, they
+    // fell to the first of them, beside parts that are taken everywhere (97
+    // thousand particles at spacing 0.4 h: density 152 and 80 us, force 212 and
+    // 135).
+    const uint32_t xcd = blockIdx.x & 7u, per = gridDim.x >> 3, rem = gridDim.x & 7u;
+    const uint32_t below = (xcd * per + min(xcd, rem)) * kWaves;  // waves on lower XCDs
+    const uint32_t here = (per + (xcd < rem ? 1u : 0u)) * kWaves;
+    const uint32_t mine = __builtin_amdgcn_readfirstlane((blockIdx.x >> 3) * kWaves + (threadIdx.x >> 6));
+    // Of n <= G tasks, this wave's, if `mine` of the XCD's share is below hi.
+    // (Products below 2^32: G is at most the waves resident at once.)
+    auto share = [&](uint32_t n, uint32_t &lo, uint32_t &hi) {
+        lo = n * below / G;
+        hi = n * (below + here) / G;
+    };
+    // Waves without a share take a part of their own first, as many on every
+    // XCD (`spare`, what the XCD with the fewest has at least), without asking:
+    // where these are all the parts, the counter is not touched (a few thousand
+    // waves that ask once each to learn it cost a pass some 50 us).
+    uint32_t t = kNoSlot, dealt = 0;
+    if (total != 0u && S.nwaves < G) {
+        uint32_t lo, hi;
+        share(S.nwaves, lo, hi);
+        const uint32_t spare = per * kWaves - (per * kWaves * S.nwaves + G - 1u) / G;
+        const uint32_t k = mine - (hi - lo);  // huge for a wave with a share
+        dealt = 8u * spare;
+        if (k < spare)
+            t = k * 8u + xcd;
+    }
+    for (uint32_t base = 0; base < S.nwaves; base += G) {
+        uint32_t lo, hi;
+        share(min(G, S.nwaves - base), lo, hi);
+        const uint32_t w = base + lo + mine;
+        if (lo + mine >= hi)
+            continue;
         if (total == 0u || __builtin_amdgcn_readfirstlane(pp.nparts[w]) == 0u)
             if (!skip_summed || !(__builtin_amdgcn_readfirstlane(pp.walk[2u * w + 1u].w) & (int)kWalkSummed))
                 task(w, 0u, 1u);
-    if (total == 0u)
+    }
+    if (t == kNoSlot && total <= dealt)
         return;
     for (;;) {
-        uint32_t t = 0;
-        if ((threadIdx.x & 63u) == 0u)
-            t = atomicAdd(queue, 1u);
-        t = __builtin_amdgcn_readfirstlane(t);
+        if (t == kNoSlot) {
+            uint32_t asked = 0;
+            if ((threadIdx.x & 63u) == 0u)
+                asked = atomicAdd(queue, 1u);
+            t = dealt + (uint32_t)__builtin_amdgcn_readfirstlane((int)asked);
+        }
         if (t >= total)
             return;
         const uint32_t packed = __builtin_amdgcn_readfirstlane(pp.tasks[t]);
         const uint32_t w = packed >> kPartBits, part = packed & (kMaxParts - 1u);
-        const uint32_t nparts = __builtin_amdgcn_readfirstlane(pp.nparts[w]);
-        task(w, part, nparts);
+        task(w, part, __builtin_amdgcn_readfirstlane(pp.nparts[w]));
+        if (total <= dealt)
+            return;
+        t = kNoSlot;
     }
 }
 

@@ -210,3 +210,31 @@ def test_union_walks_that_record_lists(sph, orc32, spacing, cell_scale):
     same = ~(out[0][0]["split"] | out[1][0]["split"])[ids]
     for key in ("rho", "pressure"):
         assert out[0][1][key][same].tobytes() == out[1][1][key][same].tobytes(), key
+
+
+@pytest.mark.parametrize("n", [1, 65, 130, 300, 511, 1300, 5000, 9001])
+@pytest.mark.parametrize("clumps", [0, 1, 5])
+def test_every_task_and_part_is_taken_once(sph, orc32, n, clumps):
+    """From one block to hundreds, unsplit tasks alone, with a few parts beside
+    them, and many: counts exactly and densities within the parity bar."""
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(-0.06, 0.06, (n, 3)) * n ** (1.0 / 3.0) + 1.1
+    m = n // 2 if clumps else 0  # half of the particles in clumps
+    pos[:m] = (rng.uniform(0.6, 1.6, (clumps or 1, 3))[np.arange(m) % (clumps or 1)] + rng.normal(0.0, 0.02, (m, 3)))
+    sc = test_gpu_staged_walk._scene(pos, box=4.0)
+    with sph.Context(sc.n, sph.settings(*sc.settings_args()), sph.box(sc.box_lo, sc.box_hi), sc.dt) as ctx:
+        ctx.upload(sc.pos, sc.vel)
+        count = ctx.walk_dump()["count"]
+        ctx.step(1)
+        got = ctx.download()
+    ost = test_gpu_union_walk.OracleState(orc32, sc, sc.pos, sc.vel)
+    try:
+        assert np.array_equal(count, [len(r) for r in ost.rows(np.arange(n))])
+        ost.forces(np.arange(1))  # computes the densities
+        rho, prs = ost.rho_p_by_id()
+    finally:
+        ost.close()
+    by_id = {k: np.zeros_like(got[k]) for k in ("rho", "pressure")}
+    for k in by_id:
+        by_id[k][got["ids"]] = got[k]
+    test_gpu_union_walk.pu.assert_rho_p(by_id["rho"], by_id["pressure"], rho, prs, ost.s)
